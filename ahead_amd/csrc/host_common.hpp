@@ -10,9 +10,11 @@
 #include "../../include/ahead_hip.h"
 #include "an_device.hpp"
 
-// A workspace holds two device allocations.  `base` is the WsHeader followed by the operators'
-// scratch regions (hash tables, partials, offsets), laid out per operator.  `status` holds only
-// look-back status words: a word whose epoch equals the current launch's must have been written
+// A workspace holds three device allocations.  `base` is the WsHeader followed by the operators'
+// scratch regions (hash tables, partials, offsets), laid out per operator.  `stream` belongs to the
+// single-pass engine (stream.hpp): a 256-byte header with its ticket and epoch word, then its
+// look-back status words; that epoch lives on the device, so the two kinds of status words never
+// share memory.  `status` holds only look-back status words: a word whose epoch equals the current launch's must have been written
 // by that launch, so no other data may ever be stored there (scratch data of an earlier operator
 // could carry any bit pattern, the current epoch included).
 struct ahead_hip_ws {
@@ -22,6 +24,9 @@ struct ahead_hip_ws {
     void *status = nullptr;  // look-back status words only
     size_t status_bytes = 0;
     uint32_t epoch = 0;      // last look-back epoch handed out
+    void *stream = nullptr;  // the single-pass engine's header and status words
+    size_t stream_bytes = 0;
+    uint32_t stream_calls = 0;  // its launches since the words were last cleared
 };
 
 namespace ahead_host {
@@ -47,6 +52,11 @@ int ws_ensure(ahead_hip_ws *ws, size_t bytes);
 // Ensures the status allocation holds `bytes`; grown the same way.  The epoch keeps counting
 // (a zero word carries epoch 0, which is never handed out).
 int ws_ensure_status(ahead_hip_ws *ws, size_t bytes);
+
+// The single-pass engine's ticket word and `bytes` of status words.  The allocation is cleared when
+// it grows, and by a fill kernel on the stream before its 30-bit epoch could repeat.
+int stream_state(ahead_hip_ws *ws, size_t bytes, hipStream_t s, unsigned long long **te, uint64_t **status);
+constexpr size_t kStreamHeader = 256;
 
 // Next look-back epoch (1 .. 2^30-1).  On wrap-around the status allocation is cleared.
 int ws_next_epoch(ahead_hip_ws *ws, uint32_t *epoch);

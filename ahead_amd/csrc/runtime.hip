@@ -22,67 +22,67 @@ int hip_fail(hipError_t e, const char *what) {
     return e == hipErrorOutOfMemory ? AHEAD_ERR_NOMEM : AHEAD_ERR_HIP;
 }
 
-int ws_ensure(ahead_hip_ws *ws, size_t bytes) {
-    if (ws == nullptr) return fail(AHEAD_ERR_INVALID, "workspace is NULL");
-    const size_t need = kHeaderBytes + align_up(bytes, 256);
-    if (ws->base != nullptr && ws->bytes >= need) return AHEAD_OK;
-    size_t grow = ws->bytes + ws->bytes / 2;
-    const size_t target = need > grow ? need : grow;
+// Grows a zero-filled device allocation of the workspace to at least `need` bytes (by half more than
+// it held); hipFree waits for the device before the old one goes.
+static int grow(ahead_hip_ws *ws, void **mem, size_t *held, size_t need, const char *what) {
+    if (*mem != nullptr && *held >= need) return AHEAD_OK;
+    const size_t more = *held + *held / 2;
+    const size_t target = need > more ? need : more;
     int cur = 0;
     AHEAD_HIP_TRY(hipGetDevice(&cur));
     if (cur != ws->device) AHEAD_HIP_TRY(hipSetDevice(ws->device));
-    if (ws->base != nullptr) {
-        AHEAD_HIP_TRY(hipFree(ws->base));
-        ws->base = nullptr;
-        ws->bytes = 0;
+    if (*mem != nullptr) {
+        AHEAD_HIP_TRY(hipFree(*mem));
+        *mem = nullptr;
+        *held = 0;
     }
     void *p = nullptr;
     hipError_t e = hipMalloc(&p, target);
     if (e != hipSuccess) {
         if (cur != ws->device) (void)hipSetDevice(cur);
-        return hip_fail(e, "hipMalloc(workspace)");
+        return hip_fail(e, what);
     }
     e = hipMemset(p, 0, target);
     if (e == hipSuccess) e = hipDeviceSynchronize();
     if (cur != ws->device) (void)hipSetDevice(cur);
     if (e != hipSuccess) {
         (void)hipFree(p);
-        return hip_fail(e, "hipMemset(workspace)");
+        return hip_fail(e, what);
     }
-    ws->base = p;
-    ws->bytes = target;
+    *mem = p;
+    *held = target;
     return AHEAD_OK;
+}
+
+int ws_ensure(ahead_hip_ws *ws, size_t bytes) {
+    if (ws == nullptr) return fail(AHEAD_ERR_INVALID, "workspace is NULL");
+    return grow(ws, &ws->base, &ws->bytes, kHeaderBytes + align_up(bytes, 256), "hipMalloc(workspace)");
 }
 
 int ws_ensure_status(ahead_hip_ws *ws, size_t bytes) {
     if (ws == nullptr) return fail(AHEAD_ERR_INVALID, "workspace is NULL");
-    const size_t need = align_up(bytes > 0 ? bytes : 1, 256);
-    if (ws->status != nullptr && ws->status_bytes >= need) return AHEAD_OK;
-    const size_t grow = ws->status_bytes + ws->status_bytes / 2;
-    const size_t target = need > grow ? need : grow;
-    int cur = 0;
-    AHEAD_HIP_TRY(hipGetDevice(&cur));
-    if (cur != ws->device) AHEAD_HIP_TRY(hipSetDevice(ws->device));
-    if (ws->status != nullptr) {
-        AHEAD_HIP_TRY(hipFree(ws->status));
-        ws->status = nullptr;
-        ws->status_bytes = 0;
+    return grow(ws, &ws->status, &ws->status_bytes, align_up(bytes > 0 ? bytes : 1, 256),
+                "hipMalloc(workspace status)");
+}
+
+static int ws_ensure_stream(ahead_hip_ws *ws, size_t bytes) {
+    if (ws == nullptr) return fail(AHEAD_ERR_INVALID, "workspace is NULL");
+    const size_t held = ws->stream_bytes;
+    const int st = grow(ws, &ws->stream, &ws->stream_bytes, kStreamHeader + align_up(bytes, 256),
+                        "hipMalloc(workspace stream)");
+    if (st == AHEAD_OK && ws->stream_bytes != held) ws->stream_calls = 0;
+    return st;
+}
+
+int stream_state(ahead_hip_ws *ws, size_t bytes, hipStream_t s, unsigned long long **te, uint64_t **status) {
+    int st = ws_ensure_stream(ws, bytes);
+    if (st != AHEAD_OK) return st;
+    if (++ws->stream_calls >= (1u << 29)) {
+        if ((st = fill_u64(static_cast<uint64_t *>(ws->stream), ws->stream_bytes / 8, 0, s)) != AHEAD_OK) return st;
+        ws->stream_calls = 0;
     }
-    void *p = nullptr;
-    hipError_t e = hipMalloc(&p, target);
-    if (e != hipSuccess) {
-        if (cur != ws->device) (void)hipSetDevice(cur);
-        return hip_fail(e, "hipMalloc(workspace status)");
-    }
-    e = hipMemset(p, 0, target);
-    if (e == hipSuccess) e = hipDeviceSynchronize();
-    if (cur != ws->device) (void)hipSetDevice(cur);
-    if (e != hipSuccess) {
-        (void)hipFree(p);
-        return hip_fail(e, "hipMemset(workspace status)");
-    }
-    ws->status = p;
-    ws->status_bytes = target;
+    *te = static_cast<unsigned long long *>(ws->stream);
+    *status = reinterpret_cast<uint64_t *>(static_cast<char *>(ws->stream) + kStreamHeader);
     return AHEAD_OK;
 }
 
@@ -185,6 +185,7 @@ int ahead_hip_ws_create(int device, ahead_hip_ws **ws) {
     w->device = device;
     int st = ws_ensure(w, 1 << 20);
     if (st == AHEAD_OK) st = ws_ensure_status(w, 1 << 16);
+    if (st == AHEAD_OK) st = ws_ensure_stream(w, 1 << 16);
     if (st != AHEAD_OK) {
         (void)ahead_hip_ws_destroy(w);
         return st;
@@ -196,9 +197,9 @@ int ahead_hip_ws_create(int device, ahead_hip_ws **ws) {
 int ahead_hip_ws_destroy(ahead_hip_ws *ws) {
     if (ws == nullptr) return AHEAD_OK;
     hipError_t e = hipSuccess;
-    if (ws->base != nullptr) e = hipFree(ws->base);
-    if (ws->status != nullptr) {
-        const hipError_t e2 = hipFree(ws->status);
+    for (void *p : {ws->base, ws->status, ws->stream}) {
+        if (p == nullptr) continue;
+        const hipError_t e2 = hipFree(p);
         if (e == hipSuccess) e = e2;
     }
     delete ws;
@@ -207,12 +208,14 @@ int ahead_hip_ws_destroy(ahead_hip_ws *ws) {
 }
 
 int ahead_hip_ws_reserve(ahead_hip_ws *ws, size_t bytes) {
-    const int st = ws_ensure(ws, bytes);
-    return st != AHEAD_OK ? st : ws_ensure_status(ws, bytes);
+    int st = ws_ensure(ws, bytes);
+    if (st == AHEAD_OK) st = ws_ensure_status(ws, bytes);
+    if (st == AHEAD_OK) st = ws_ensure_stream(ws, bytes);
+    return st;
 }
 
 size_t ahead_hip_ws_bytes(const ahead_hip_ws *ws) {
-    return ws == nullptr ? 0 : ws->bytes + ws->status_bytes;
+    return ws == nullptr ? 0 : ws->bytes + ws->status_bytes + ws->stream_bytes;
 }
 
 int ahead_hip_set_tiling(uint32_t max_subtiles, uint32_t min_tiles) {

@@ -1,0 +1,325 @@
+// stream.hpp -- the single-pass engine of the operators that emit at most one entry per row into an
+// ordered main output: check-and-decode, fetch, positional match, hash probe of unique keys.
+//
+// A persistent grid (one workgroup of 1024 threads per CU) takes tiles of 1024 x G rows in ticket
+// order.  Per tile, every lane evaluates its G rows, the tile publishes how many rows it keeps and
+// reports, takes its place among all tiles from its predecessors' counts, and writes every entry
+// once, at its final place.  Nothing is staged, moved or re-read: the traffic is the inputs once
+// and the outputs once, whether rows are dropped or not.
+//
+// Bound by HBM as long as three latencies stay off the path (60M 8-byte codes checked and decoded
+// to 4 bytes, 720 MB, on one MI355X; the same loads and stores without any order take 103 us):
+//  - the place of a tile: a look-back that walks 64 predecessors at a time advances 128 tiles per
+//    device-scope round trip, and a round trip takes several microseconds while HBM is saturated
+//    (206 us).  Here one round reads the counts of all kStreamWindow predecessors, one per thread,
+//    and the inclusive prefix just before them; with one workgroup per CU that prefix belongs to a
+//    tile of an earlier generation and is there (170 us).  Windows of 256, 512 and 1024 tiles
+//    measured alike; 512 covers two tickets per CU.
+//  - the next tile's loads go out before the look-back's polls (128 us).
+//  - tickets come from one address, about 15 ns each: 7325 tiles of 8192 rows take 190 us, 3663 of
+//    16384 rows 128 us.
+//
+// The tickets and the epoch of the status words are one 64-bit word in device memory (epoch in the
+// high half, ticket in the low): one atomic hands out both, and the workgroup that takes the
+// launch's last ticket (every workgroup takes one past the end) starts the next epoch.  A launch
+// needs nothing from the host and can be captured in a graph and replayed.  Every ticket's holder
+// is running, and a tile waits for lower tickets only, so the chain always drains.
+//
+// Op interface (beside eval / emit_err / finish of rowtile.hpp, which the rare error rows use):
+//   static constexpr int kErr, kG;      // error streams; rows per lane (at most 32)
+//   struct Raw; using State;            // a row's streamed inputs; what its entry needs
+//   uint64_t out_cap;                   // entries the outputs hold
+//   void load(uint64_t first, uint32_t k, Raw &) const;        // row first + k
+//   template <int G> void eval_tile(const char *lds, uint64_t first, uint32_t lane,
+//            const Raw (&)[G], uint32_t live, State (&)[G], uint32_t &keep, uint32_t (&err)[kErr]) const;
+//       // rows first + 64 g + lane; bit g of live: the row exists (raw is zero where it does not);
+//       // sets bit g of keep / err[e] for live rows that emit an entry / report into stream e
+//   void emit(const State &, uint64_t first, uint64_t pos, uint32_t row, uint32_t k) const;
+//       // entry pos + k, of row first + row (first and pos are wave-uniform: scalar bases)
+//   void report(uint64_t row, State &, uint32_t &errs) const;  // the error streams of one row
+//   void init(char *lds) const;         // all threads, before the first tile; a barrier follows
+//   bool skip() const;                  // the whole launch stands down (decided from device state)
+#pragma once
+
+#include "rowtile.hpp"
+
+namespace ahead_dev {
+
+constexpr int kStreamThreads = 1024;
+constexpr int kStreamWaves = kStreamThreads / 64;
+constexpr uint32_t kStreamWindow = 512;
+
+struct StreamArgs {
+    unsigned long long *te;  // epoch << 32 | ticket
+    WsHeader *hdr;           // fail flag
+    uint64_t *agg;           // [tiles] epoch << 34 | reports << 33 | kept
+    uint64_t *incl;          // [1 + kErr][tiles] epoch << 34 | inclusive count
+    uint64_t *erep;          // [kErr][tiles] epoch << 34 | rows reported (tiles with reports only)
+    uint32_t tiles;
+    uint32_t last;           // the launch's last ticket: tiles + workgroups - 1
+};
+
+// A ticket word's tile; the holder of the launch's last ticket starts the next epoch.
+__device__ __forceinline__ uint32_t stream_tile(const StreamArgs &m, unsigned long long v) {
+    const uint32_t t = static_cast<uint32_t>(v);
+    if (t == m.last)
+        __hip_atomic_store(m.te, ((v >> 32) + 1ull) << 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return t;
+}
+
+__device__ __forceinline__ uint64_t stream_word(uint32_t epoch, uint64_t v) {
+    return (static_cast<uint64_t>(epoch) << 34) | v;
+}
+// A status word of this launch (polled until its tile has published it; the spin is bounded).
+__device__ __forceinline__ uint64_t stream_poll(const StreamArgs &m, const uint64_t *w, uint32_t epoch) {
+    uint64_t v = lb_load(w);
+    uint32_t spins = 0;
+    while (static_cast<uint32_t>(v >> 34) != epoch) {
+        if (++spins >= kSpinLimit) {
+            atomicOr(&m.hdr->fail, 1u);
+            return 0;
+        }
+        __builtin_amdgcn_s_sleep(1);
+        v = lb_load(w);
+    }
+    return v;
+}
+
+__device__ __forceinline__ uint32_t wave_rank(uint64_t ballot) {
+    return __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(ballot >> 32),
+                                     __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(ballot), 0u));
+}
+
+// The streamed inputs of a lane's G rows first + 64 g + lane; left: rows of the wave that exist.
+template <class Op, int G>
+__device__ __forceinline__ void stream_load(const Op &op, uint64_t first, uint32_t lane, uint32_t left,
+                                            typename Op::Raw (&raw)[G]) {
+    if (left == 64u * G) {
+#pragma unroll
+        for (int g = 0; g < G; ++g) op.load(first, static_cast<uint32_t>(g * 64) + lane, raw[g]);
+    } else {
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            const uint32_t k = static_cast<uint32_t>(g * 64) + lane;
+            raw[g] = typename Op::Raw{};
+            if (k < left) op.load(first, k, raw[g]);
+        }
+    }
+}
+__device__ __forceinline__ uint32_t uniform(uint32_t x) { return __builtin_amdgcn_readfirstlane(x); }
+
+template <class Op>
+__global__ __launch_bounds__(kStreamThreads) void k_stream(Op op, StreamArgs m) {
+    constexpr int G = Op::kG, NS = 1 + Op::kErr, NW = kStreamWaves;
+    constexpr uint32_t kWaveRows = 64u * G, kAll = G == 32 ? 0xFFFFFFFFu : (1u << (G & 31)) - 1u;
+    static_assert(NS <= 64, "one wave polls the inclusive prefixes");
+    extern __shared__ char s_op[];
+    __shared__ uint32_t s_cnt[NS][NW], s_sum[NS][NW];
+    __shared__ uint32_t s_tile, s_epoch;
+    if (op.skip()) return;
+    if (threadIdx.x == 0) {
+        const unsigned long long v = atomicAdd(m.te, 1ull);
+        s_tile = stream_tile(m, v);
+        s_epoch = static_cast<uint32_t>(v >> 32) % ((1u << 30) - 1u) + 1u;
+    }
+    op.init(s_op);
+    __syncthreads();
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t epoch = __builtin_amdgcn_readfirstlane(s_epoch);
+    uint32_t tile = __builtin_amdgcn_readfirstlane(s_tile);
+    auto first_of = [&](uint32_t t) { return (static_cast<uint64_t>(t) * NW + wave) * kWaveRows; };
+    auto left_of = [&](uint64_t first) {
+        return first >= op.n ? 0u : op.n - first < kWaveRows ? static_cast<uint32_t>(op.n - first) : kWaveRows;
+    };
+    typename Op::Raw raw[G];
+    if (tile < m.tiles) stream_load<Op, G>(op, first_of(tile), lane, left_of(first_of(tile)), raw);
+    while (tile < m.tiles) {
+        unsigned long long ticket = 0;
+        if (threadIdx.x == 0) ticket = atomicAdd(m.te, 1ull);
+        const uint64_t first = first_of(tile);
+        const uint32_t left = left_of(first);
+        uint32_t live = kAll;
+        if (left != kWaveRows) {
+            live = 0;
+#pragma unroll
+            for (int g = 0; g < G; ++g) live |= (static_cast<uint32_t>(g * 64) + lane < left ? 1u : 0u) << g;
+        }
+        typename Op::State st[G];
+        uint32_t keep = 0, err[Op::kErr] = {};
+        op.template eval_tile<G>(s_op, first, lane, raw, live, st, keep, err);
+
+        // what the wave keeps and reports
+        const bool whole = __ballot(keep == kAll) == ~0ull;
+        const uint32_t kept = whole ? kWaveRows : __builtin_amdgcn_readfirstlane(wave_sum(
+                                                      static_cast<uint32_t>(__popc(keep))));
+        uint32_t any = 0;
+#pragma unroll
+        for (int e = 0; e < Op::kErr; ++e) any |= err[e];
+        const bool reports = __ballot(any != 0u) != 0ull;
+        uint32_t ecnt[Op::kErr] = {};
+        if (reports) {
+#pragma unroll
+            for (int e = 0; e < Op::kErr; ++e) ecnt[e] = wave_sum(static_cast<uint32_t>(__popc(err[e])));
+        }
+        if (lane == 0) {
+            s_cnt[0][wave] = kept;
+#pragma unroll
+            for (int e = 0; e < Op::kErr; ++e) s_cnt[1 + e][wave] = ecnt[e];
+        }
+        if (threadIdx.x == 0) s_tile = stream_tile(m, ticket);
+        __syncthreads();
+        uint32_t agg[NS], before[NS], rep = 0;
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            agg[s] = 0;
+            before[s] = 0;
+#pragma unroll
+            for (int w = 0; w < NW; ++w) {
+                const uint32_t c = s_cnt[s][w];
+                if (w < static_cast<int>(wave)) before[s] += c;
+                agg[s] += c;
+            }
+            agg[s] = uniform(agg[s]);
+            before[s] = uniform(before[s]);
+            if (s) rep |= agg[s];
+        }
+        if (threadIdx.x == 0) {
+            if (rep != 0u) {
+#pragma unroll
+                for (int e = 0; e < Op::kErr; ++e)
+                    lb_store(&m.erep[static_cast<size_t>(e) * m.tiles + tile], stream_word(epoch, agg[1 + e]));
+            }
+            lb_store(&m.agg[tile], stream_word(epoch, (rep != 0u ? 1ull << 33 : 0ull) | agg[0]));
+        }
+        const uint32_t next = __builtin_amdgcn_readfirstlane(s_tile);
+        if (next < m.tiles) stream_load<Op, G>(op, first_of(next), lane, left_of(first_of(next)), raw);
+
+        // the counts of the kStreamWindow - 1 tiles before this one, and the prefix before them
+        uint32_t sum[NS] = {};
+        const uint32_t back = threadIdx.x + 1u;
+        if (back < kStreamWindow && back <= tile) {
+            const uint64_t v = stream_poll(m, &m.agg[tile - back], epoch);
+            sum[0] = static_cast<uint32_t>(v);
+            if ((v >> 33) & 1ull) {
+#pragma unroll
+                for (int e = 0; e < Op::kErr; ++e)
+                    sum[1 + e] = static_cast<uint32_t>(
+                        stream_poll(m, &m.erep[static_cast<size_t>(e) * m.tiles + tile - back], epoch));
+            }
+        }
+        if (wave == NW - 1 && tile >= kStreamWindow) {
+#pragma unroll
+            for (int s = 0; s < NS; ++s) {
+                if (lane == static_cast<uint32_t>(s))
+                    sum[s] += static_cast<uint32_t>(
+                        stream_poll(m, &m.incl[static_cast<size_t>(s) * m.tiles + tile - kStreamWindow], epoch));
+            }
+        }
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            const uint32_t t = __ballot(sum[s] != 0u) != 0ull ? wave_sum(sum[s]) : 0u;
+            if (lane == 0) s_sum[s][wave] = t;
+        }
+        __syncthreads();
+        uint32_t excl[NS];
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            excl[s] = 0;
+#pragma unroll
+            for (int w = 0; w < NW; ++w) excl[s] += s_sum[s][w];
+            excl[s] = uniform(excl[s]);
+            if (threadIdx.x == static_cast<uint32_t>(s))
+                lb_store(&m.incl[static_cast<size_t>(s) * m.tiles + tile], stream_word(epoch, excl[s] + agg[s]));
+        }
+
+        const uint64_t pos = static_cast<uint64_t>(excl[0]) + before[0];
+        const uint32_t room = pos >= op.out_cap                   ? 0u
+                              : op.out_cap - pos < kWaveRows ? static_cast<uint32_t>(op.out_cap - pos)
+                                                             : kWaveRows;
+        if (whole && room == kWaveRows) {
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                const uint32_t k = static_cast<uint32_t>(g * 64) + lane;
+                op.emit(st[g], first, pos, k, k);
+            }
+        } else if (kept != 0u) {
+            uint32_t at = 0;
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                const bool on = (keep >> g) & 1u;
+                const uint64_t b = __ballot(on);
+                const uint32_t k = at + wave_rank(b);
+                if (on && k < room) op.emit(st[g], first, pos, static_cast<uint32_t>(g * 64) + lane, k);
+                at += static_cast<uint32_t>(__popcll(b));
+            }
+        }
+        if (reports) {  // rare: the wave's rows are evaluated again, 64 at a time
+            uint64_t idx[Op::kErr];
+#pragma unroll
+            for (int e = 0; e < Op::kErr; ++e) idx[e] = static_cast<uint64_t>(excl[1 + e]) + before[1 + e];
+            for (uint32_t k0 = 0; k0 < left; k0 += 64u) {
+                const uint64_t row = first + k0 + lane;
+                typename Op::State rs{};
+                uint32_t errs = 0;
+                if (k0 + lane < left) op.report(row, rs, errs);
+#pragma unroll
+                for (int e = 0; e < Op::kErr; ++e) {
+                    const bool on = (errs >> e) & 1u;
+                    const uint64_t b = __ballot(on);
+                    if (on) op.emit_err(e, row, rs, idx[e] + wave_rank(b));
+                    idx[e] += static_cast<uint64_t>(__popcll(b));
+                }
+            }
+        }
+        if (tile == m.tiles - 1u && threadIdx.x == 0) {
+            uint64_t totals[NS];
+#pragma unroll
+            for (int s = 0; s < NS; ++s) totals[s] = static_cast<uint64_t>(excl[s]) + agg[s];
+            op.finish(totals);
+        }
+        tile = next;
+    }
+}
+
+}  // namespace ahead_dev
+
+namespace ahead_host {
+
+// Launches the engine for op over op.n rows with `lds` bytes for its tables (at most kStreamLds).
+constexpr size_t kStreamLds = 152 * 1024;
+
+template <class Op>
+int launch_stream(const Op &op, ahead_hip_ws *ws, hipStream_t s, size_t lds = 0) {
+    using namespace ahead_dev;
+    constexpr uint64_t rows = static_cast<uint64_t>(kStreamThreads) * Op::kG;
+    static const uint32_t cus = [] {
+        int dev = 0, c = 0;
+        if (hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || c <= 0)
+            c = 256;
+        return static_cast<uint32_t>(c);
+    }();
+    if (lds > 0) {
+        static const hipError_t set = hipFuncSetAttribute(reinterpret_cast<const void *>(k_stream<Op>),
+                                                          hipFuncAttributeMaxDynamicSharedMemorySize, kStreamLds);
+        AHEAD_HIP_TRY(set);
+    }
+    const uint64_t tiles = op.n == 0 ? 1 : (op.n + rows - 1) / rows;
+    const uint32_t grid = static_cast<uint32_t>(tiles < cus ? tiles : cus);
+    StreamArgs m{};
+    m.tiles = static_cast<uint32_t>(tiles);
+    m.last = m.tiles + grid - 1u;
+    uint64_t *words = nullptr;
+    const int st = stream_state(ws, static_cast<size_t>(tiles) * (2 + 2 * Op::kErr) * 8, s, &m.te, &words);
+    if (st != AHEAD_OK) return st;
+    m.hdr = ws_header(ws);
+    m.agg = words;
+    m.incl = words + tiles;
+    m.erep = words + tiles * (2 + Op::kErr);
+    hipLaunchKernelGGL((k_stream<Op>), dim3(grid), dim3(kStreamThreads), lds, s, op, m);
+    AHEAD_HIP_TRY(hipGetLastError());
+    return AHEAD_OK;
+}
+
+}  // namespace ahead_host

@@ -1,0 +1,108 @@
+"""The single-pass engine (stream.hpp) at the edges of its tiles (1024 threads x 16 rows; 32 for 2-byte
+codes) and of its 512-tile window, against the oracle: outputs, counts and error positions."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import oracle_lib as O
+from ahead_amd import an, capi, datagen
+
+pytestmark = pytest.mark.gpu
+
+KINDS = {2: (an.RESTINY, 233, 0xFF), 4: (an.RESSHORT, 63877, 0xFFFF), 8: (an.RESINT, 65117, 0xFFFFFFFF)}
+TILE = 1024 * 16
+
+
+def codes_of(n, width, bad, seed):
+    t, a, top = KINDS[width]
+    rng = np.random.default_rng(seed)
+    c = datagen.encode(rng.integers(0, top + 1, n).astype(np.uint64), a, width)
+    hit = rng.choice(n, min(bad, n), replace=False)
+    c[hit] ^= (np.ones(hit.size, np.uint64) << rng.integers(0, 8 * width, hit.size).astype(np.uint64)).astype(c.dtype)
+    return c, an.an_meta(t, a)
+
+
+def decode_call(col, cap, ecap, stream=None):
+    lib, ws = capi.load(), capi.workspace()
+    w = col.meta.type.unenc_bits // 8
+    dec, err, cnt = capi.DeviceBuffer(max(8, w * cap)), capi.DeviceBuffer(8 * ecap), capi.DeviceBuffer(16)
+    d = col.desc()
+
+    def launch(s=None):
+        capi.check(lib.ahead_hip_check_and_decode_an(ctypes.byref(d), an.A_OID_ERR, dec.ptr, cap, err.ptr, ecap,
+                                                     cnt.ptr, ws.h, capi.current_stream() if s is None else s))
+    return launch, dec, err, cnt
+
+
+@pytest.mark.parametrize("width", [2, 4, 8])
+@pytest.mark.parametrize("n,bad", [
+    (0, 0), (1, 0), (1, 1), (63, 2), (TILE - 1, 0), (TILE, 1), (TILE + 1, 3), (2 * TILE + 64, 40),
+    (40 * TILE + 777, 0), (40 * TILE + 777, 5000), (511 * TILE + 5, 3), (513 * TILE + 9, 700),
+    (1100 * TILE + 31, 2),
+])
+def test_check_and_decode_tiles(width, n, bad):
+    codes, meta = codes_of(n, width, bad, seed=n + bad + width)
+    col = capi.Column.from_numpy(codes, meta)
+    ref = O.check_and_decode_an(O.Col(codes, meta))
+    print(f"check_and_decode width={width} n={n} bad={bad}", flush=True)
+    launch, dec, err, cnt = decode_call(col, n, max(1, bad))
+    launch()
+    capi.synchronize()
+    c = [int(x) for x in cnt.to_numpy(np.uint64, 2)]
+    assert c == [len(ref[0]), len(ref[1])]
+    assert np.array_equal(dec.to_numpy(f"u{meta.type.unenc_bits // 8}", c[0]), ref[0])
+    assert np.array_equal(err.to_numpy(np.uint64, c[1]), ref[1])
+
+
+@pytest.mark.parametrize("cap,ecap", [(0, 1), (1, 0), (TILE - 3, 7), (2 * TILE + 100, 900)])
+def test_check_and_decode_capacities(cap, ecap):
+    n, bad = 3 * TILE + 11, 800
+    codes, meta = codes_of(n, 8, bad, seed=9)
+    ref = O.check_and_decode_an(O.Col(codes, meta))
+    launch, dec, err, cnt = decode_call(capi.Column.from_numpy(codes, meta), n, bad)
+    guard = 0xAB
+    dec.t.fill_(guard)
+    err.t.fill_(guard)
+    lib, ws = capi.load(), capi.workspace()
+    d = capi.Column.from_numpy(codes, meta)
+    x = d.desc()
+    capi.check(lib.ahead_hip_check_and_decode_an(ctypes.byref(x), an.A_OID_ERR, dec.ptr, cap, err.ptr, ecap, cnt.ptr,
+                                                 ws.h, capi.current_stream()))
+    capi.synchronize()
+    assert [int(v) for v in cnt.to_numpy(np.uint64, 2)] == [len(ref[0]), len(ref[1])]
+    got, e = dec.to_numpy(np.uint32, n), err.to_numpy(np.uint64, bad)
+    k, j = min(cap, len(ref[0])), min(ecap, len(ref[1]))
+    assert np.array_equal(got[:k], ref[0][:k]) and np.array_equal(e[:j], ref[1][:j])
+    assert (got[k:].view(np.uint8) == guard).all() and (e[j:].view(np.uint8) == guard).all()
+
+
+def test_check_and_decode_graph_replays():
+    """The ticket and epoch live on the device: a captured launch gives the right result on every
+    replay, over changed codes, with calls of other sizes between the replays."""
+    import torch
+
+    n = 20 * TILE + 5
+    sets = [codes_of(n, 8, bad, seed=bad) for bad in (0, 3, 900)]
+    meta = sets[0][1]
+    col = capi.Column.from_numpy(sets[0][0], meta)
+    launch, dec, err, cnt = decode_call(col, n, 1000)
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        launch(side.cuda_stream)  # the workspace takes its size before the capture
+        side.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=side):
+            launch(side.cuda_stream)
+        for codes, _ in sets + sets[::-1]:
+            col.buf.t.copy_(torch.from_numpy(codes.view(np.uint8)))
+            small, sm = codes_of(3 * TILE + 1, 8, 2, seed=1)
+            got = capi.check_and_decode_an(capi.Column.from_numpy(small, sm))
+            assert np.array_equal(got[0], O.check_and_decode_an(O.Col(small, sm))[0])
+            g.replay()
+            side.synchronize()
+            ref = O.check_and_decode_an(O.Col(codes, meta))
+            c = [int(v) for v in cnt.to_numpy(np.uint64, 2)]
+            assert c == [len(ref[0]), len(ref[1])]
+            assert np.array_equal(dec.to_numpy(np.uint32, c[0]), ref[0])
+            assert np.array_equal(err.to_numpy(np.uint64, c[1]), ref[1])
