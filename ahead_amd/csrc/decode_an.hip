@@ -83,6 +83,7 @@ struct CheckDecodeOp {
     uint64_t n;
     const CodeT *codes;
     CodeT a_inv, max_u;
+    uint32_t back;  // 8-byte codes of values below 2^32: A (back_factor), else 0
     uint64_t a_oid;
     OutT *dec;
     uint64_t out_cap;
@@ -96,17 +97,36 @@ struct CheckDecodeOp {
         r.c = __builtin_nontemporal_load(codes + first + k);
     }
     template <int G>
-    __device__ __forceinline__ void eval_tile(const char *, uint64_t, uint32_t, const Raw (&raw)[G], uint32_t live,
-                                              State (&st)[G], uint32_t &keep, uint32_t (&errs)[kErr]) const {
-        uint32_t bad = 0;
+    struct Mid {
+        OutT d[G];
+        uint32_t bad;
+    };
+    template <int G>
+    __device__ __forceinline__ void open_tile(const char *, uint64_t, uint32_t, const Raw (&raw)[G], Mid<G> &mid) const {
+        mid.bad = 0;
+        if (sizeof(CodeT) == 8 && back != 0u) {
 #pragma unroll
-        for (int g = 0; g < G; ++g) {
-            const CodeT d = an_mul<CodeT>(raw[g].c, a_inv);
-            st[g] = static_cast<OutT>(d);
-            bad |= (d > max_u ? 1u : 0u) << g;
+            for (int g = 0; g < G; ++g) {
+                const uint32_t d = static_cast<uint32_t>(raw[g].c) * static_cast<uint32_t>(a_inv);
+                mid.d[g] = static_cast<OutT>(d);
+                mid.bad |= (static_cast<uint64_t>(d) * back != raw[g].c || d > max_u ? 1u : 0u) << g;
+            }
+        } else {
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                const CodeT d = an_mul<CodeT>(raw[g].c, a_inv);
+                mid.d[g] = static_cast<OutT>(d);
+                mid.bad |= (d > max_u ? 1u : 0u) << g;
+            }
         }
-        keep = live & ~bad;
-        errs[0] = live & bad;
+    }
+    template <int G>
+    __device__ __forceinline__ void close_tile(const Mid<G> &mid, uint32_t live, State (&st)[G], uint32_t &keep,
+                                               uint32_t (&errs)[kErr]) const {
+#pragma unroll
+        for (int g = 0; g < G; ++g) st[g] = mid.d[g];
+        keep = live & ~mid.bad;
+        errs[0] = live & mid.bad;
     }
     __device__ void report(uint64_t row, State &, uint32_t &errs) const {
         errs = an_mul<CodeT>(codes[row], a_inv) > max_u ? 1u : 0u;
@@ -158,6 +178,7 @@ int launch_check_decode(const ahead_col *col, uint64_t a_oid, void *dec, uint64_
     op.codes = static_cast<const CodeT *>(col->data);
     op.a_inv = static_cast<CodeT>(col->a_inv);
     op.max_u = static_cast<CodeT>(col->max_u);
+    op.back = sizeof(CodeT) == 8 ? ahead_host::back_factor(col->a_inv, col->max_u) : 0u;
     op.a_oid = a_oid;
     op.dec = static_cast<OutT *>(dec);
     op.out_cap = dec == nullptr ? 0 : dec_cap;

@@ -78,6 +78,16 @@ inline uint64_t inverse_mod2k(uint64_t a, uint32_t bits) {
     return bits >= 64 ? x : (x & ((1ull << bits) - 1ull));
 }
 
+// Values below 2^32 in 8-byte codes: d = code * A^-1 mod 2^64 is below 2^32 exactly if its low half
+// times A is the code again (multiplication by the odd A^-1 has one preimage), so a kernel checks with
+// one 32-bit product and one 32 x 32 -> 64-bit product in place of a 64-bit one (four 32-bit multiplies,
+// each a quarter of an addition's rate).  Returns A = the inverse of a_inv, or 0 where that does not
+// apply: values of 2^32 and more are valid, or A needs more than 32 bits.
+inline uint32_t back_factor(uint64_t a_inv, uint64_t max_value) {
+    const uint64_t a = inverse_mod2k(a_inv, 64);
+    return max_value <= 0xFFFFFFFFull && a <= 0xFFFFFFFFull ? static_cast<uint32_t>(a) : 0u;
+}
+
 inline uint64_t width_mask(uint32_t w) { return w >= 8 ? ~0ull : ((1ull << (8 * w)) - 1ull); }
 inline uint64_t bits_mask(uint32_t b) { return b >= 64 ? ~0ull : ((1ull << b) - 1ull); }
 

@@ -8,6 +8,7 @@
 // compare the int-promoted product of 16-bit codes without it (matchjoinAN.tcc:278 and :342,
 // hashjoinAN.tcc:153); no query path feeds 16-bit codes to them.
 #include "maptile.hpp"
+#include "stream.hpp"
 
 using namespace ahead_dev;
 
@@ -16,96 +17,339 @@ namespace {
 constexpr int kG = 8;  // row groups of 256 per tile (2048 rows)
 
 // ---------------------------------------------------------------------------------------------------
+// fetchjoinAN on the single-pass engine.  The gathers bound it: a random 2-byte gather costs a 128-byte
+// line between L1 and L2, so 60M of them take 270 us where the rest of the operator takes 100.  A column
+// that many OIDs point into is therefore looked up in LDS:
+//   kRaw     its codes, when they fit;
+//   kPacked  its decoded values less the smallest, in the fewest bits that hold them, several to a word;
+//            the all-ones field sends the row to the column (corrupt codes; the largest value, where the
+//            bits leave no other field), whose code is checked; the other rows' values are valid.  Rows past the words' capacity read the column too, so a column
+//            of 200,000 8-bit values serves three quarters of its rows from LDS.
+// 60M OIDs into 2-byte columns, the lookups alone with the streaming around them: 40,000 rows 220 us from
+// L2, 104 from LDS; 200,000 rows 264 and 150; without any lookup 97.  The whole operator into 200,000 8-bit
+// values: 408 us before (gathers 340, moving the entries behind a dropped row 67), 205 now.
+enum FetchTable : uint32_t { kFetchNone = 0, kFetchRaw = 1, kFetchPacked = 2 };
+constexpr uint32_t kFetchTableBytes = 150 * 1024;
+struct alignas(16) FetchPack {  // in front of the packed words
+    uint32_t lo, bits, per, magic, covered, full;
+    uint32_t pad[2];
+};
+constexpr uint32_t kFetchWords = (kFetchTableBytes - sizeof(FetchPack)) / 4;
+constexpr uint32_t kRangeBlocks = 64;
+struct FetchRange {
+    uint32_t lo, hi, bad, pad;
+};
+
+// The packed table is built once per call, by the whole card, and then copied by every workgroup (built
+// by each workgroup for itself it took 100 us of a 60M-OID fetch into 200,000 rows).  First the range of the column's valid
+// values, one entry per workgroup ...
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_fetch_range(const T *col, uint32_t n, T a_inv, T max_u, FetchRange *out) {
+    __shared__ uint32_t s_lo, s_hi, s_bad;
+    if (threadIdx.x == 0) {
+        s_lo = 0xFFFFFFFFu;
+        s_hi = 0u;
+        s_bad = 0u;
+    }
+    __syncthreads();
+    constexpr uint32_t U = 8;
+    uint32_t lo = 0xFFFFFFFFu, hi = 0u;
+    bool bad = false;
+    for (uint32_t i0 = blockIdx.x * kBlock * U; i0 < n; i0 += kRangeBlocks * kBlock * U) {
+        T c[U];
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) {
+            const uint32_t i = i0 + u * kBlock + threadIdx.x;
+            c[u] = col[i < n ? i : n - 1u];
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) {
+            const T d = an_mul<T>(c[u], a_inv);
+            const bool ok = d <= max_u;
+            bad |= !ok;
+            lo = ok && d < lo ? d : lo;
+            hi = ok && d > hi ? d : hi;
+        }
+    }
+    atomicMin(&s_lo, lo);
+    atomicMax(&s_hi, hi);
+    if (bad) s_bad = 1u;
+    __syncthreads();
+    if (threadIdx.x == 0) out[blockIdx.x] = FetchRange{s_lo, s_hi, s_bad, 0u};
+}
+// ... then, from all of them, the layout, and every thread the words it comes to.
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_fetch_pack(const T *col, uint32_t n, T a_inv, T max_u,
+                                                       const FetchRange *ranges, FetchPack *p) {
+    __shared__ uint32_t s_r[3];
+    if (threadIdx.x < 64) {
+        FetchRange r = ranges[threadIdx.x];
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) {
+            const uint32_t l = __shfl_xor(r.lo, d, 64), h = __shfl_xor(r.hi, d, 64);
+            r.lo = l < r.lo ? l : r.lo;
+            r.hi = h > r.hi ? h : r.hi;
+            r.bad |= __shfl_xor(r.bad, d, 64);
+        }
+        if (threadIdx.x == 0) {
+            s_r[0] = r.lo;
+            s_r[1] = r.hi;
+            s_r[2] = r.bad;
+        }
+    }
+    __syncthreads();
+    const uint32_t lo = s_r[0], span = s_r[1] - lo;
+    uint32_t bits = 32;  // (no valid value: lo > hi)
+    if (lo <= s_r[1] && span < 0x7FFFFFFFu) {
+        bits = 1;
+        while ((1u << bits) - 1u < span) ++bits;
+        // every field taken: a few values leave one field free, of many the largest shares its own
+        if ((1u << bits) - 1u == span && bits < 6u) ++bits;
+        // where as many fields fit a word, whole bytes
+        if (32u / bits == 4u) bits = 8u;
+        if (32u / bits == 2u) bits = 16u;
+    }
+    const uint32_t ones = bits == 32u ? 0xFFFFFFFFu : (1u << bits) - 1u, per = 32u / bits;
+    const uint32_t cap = per * kFetchWords;
+    const uint32_t covered = cap >= n ? n : (cap >= n / 4u ? cap : 0u);  // below a quarter: the column alone
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        // i / per = mulhi(i, magic) for i < 2^27
+        *p = FetchPack{lo, bits, per, per > 1u ? 0xFFFFFFFFu / per + 1u : 0u, covered,
+                       covered == n && s_r[2] == 0u && ones != span ? 1u : 0u, {0u, 0u}};
+    }
+    uint32_t *w = reinterpret_cast<uint32_t *>(p + 1);
+    const uint32_t q = blockIdx.x * kBlock + threadIdx.x;
+    if (static_cast<uint64_t>(q) * per >= covered || q >= kFetchWords) return;
+    uint32_t v = 0;
+#pragma unroll 4
+    for (uint32_t r = 0; r < per; ++r) {
+        const uint32_t i = q * per + r;
+        const T d = an_mul<T>(col[i < n ? i : n - 1u], a_inv);
+        v |= (d > max_u ? ones : static_cast<uint32_t>(d) - lo) << (r * bits);
+    }
+    w[q] = v;
+}
+
+template <typename T, bool ENC>
 struct FetchOp {
     static constexpr int kErr = 2;
-    static constexpr bool kMulti = false, kMain = true, kAcc = false;
-    using State = uint64_t;
+    static constexpr int kG = 16;
+    struct Raw {
+        uint64_t c;
+    };
+    using Out = std::conditional_t<ENC, T, std::conditional_t<(sizeof(T) >= 4), uint64_t,
+                                                             std::conditional_t<sizeof(T) == 2, uint32_t, uint16_t>>>;
+    using State = Out;
     uint64_t n;
-    DCol oids, col;
-    uint32_t ow;
-    uint64_t omask;
+    const uint64_t *oids;
+    uint64_t o_inv;
+    uint32_t o_back;  // the OIDs' A (back_factor), else 0
+    const T *col;
+    uint32_t col_n;
+    T a, a_inv, max_u;
+    uint32_t table;
+    const FetchPack *pack;  // kFetchPacked: the table in the workspace
     uint32_t reenc;
-    uint64_t f, a_oid;
-    void *out;
+    Out f;
+    uint64_t a_oid;
+    Out *out;
     uint64_t out_cap;
     uint64_t *e1, *e2;
     uint64_t e1_cap, e2_cap;
     uint64_t *d_counts;
 
-    static constexpr bool kBatched = true;
-    static constexpr int kOuts = 1;
-    static constexpr int kMapRows = 8;  // half the steps whose loads wait for the previous step's stores
-    __device__ void out_arrays(void *(&p)[2], uint32_t (&w)[2]) const {
-        p[0] = out;
-        w[0] = ow;
-        p[1] = nullptr;
-        w[1] = 0;
+    __device__ bool skip() const { return false; }
+    __device__ void init(char *lds) const {
+        if (table == kFetchRaw) {
+            T *t = reinterpret_cast<T *>(lds);
+            for (uint32_t i = threadIdx.x; i < col_n; i += kStreamThreads) t[i] = col[i];
+        }
+        if (table == kFetchPacked) {
+            const uint4 *src = reinterpret_cast<const uint4 *>(pack);
+            uint4 *dst = reinterpret_cast<uint4 *>(lds);
+            const uint32_t words = pack->covered / pack->per + 1u;  // read by 16 bytes, within the table
+            const uint32_t quads = (words + sizeof(FetchPack) / 4 + 3u) / 4u;
+            constexpr uint32_t most = kFetchTableBytes / 16;
+            for (uint32_t i = threadIdx.x; i < (quads < most ? quads : most); i += kStreamThreads) dst[i] = src[i];
+        }
+    }
+    __device__ __forceinline__ void load(uint64_t first, uint32_t k, Raw &r) const {
+        r.c = __builtin_nontemporal_load(oids + first + k);
     }
     template <int G>
-    __device__ void eval_n(const uint64_t (&row)[G], const bool (&live)[G], State (&st)[G], uint32_t (&errs)[G],
-                           uint32_t (&cnt)[G], uint64_t &) const {
-        uint64_t o[G], t[G], v[G];
-        bool in[G];
-        oids.raw_n<G>(row, live, o);
+    struct Mid {
+        T v[G];         // the rows' codes
+        uint32_t past;  // OIDs past the column
+        bool clean;     // every code is valid
+    };
+    template <int G>
+    __device__ __forceinline__ void open_tile(const char *lds, uint64_t, uint32_t, const Raw (&raw)[G],
+                                              Mid<G> &mid) const {
+        uint32_t idx[G];
+        mid.past = 0;
+        mid.clean = false;
+        // normative bound (the reference reads one past the end at t == |col|)
+        if (o_back != 0u) {
 #pragma unroll
-        for (int g = 0; g < G; ++g) {
-            t[g] = o[g] * oids.a_inv;
-            in[g] = live[g] && t[g] < col.n;
-        }
-        col.raw_n<G>(t, in, v);
+            for (int g = 0; g < G; ++g) {
+                const uint32_t t = static_cast<uint32_t>(raw[g].c) * static_cast<uint32_t>(o_inv);
+                const bool in = t < col_n && static_cast<uint64_t>(t) * o_back == raw[g].c;
+                mid.past |= (in ? 0u : 1u) << g;
+                idx[g] = in ? t : 0u;
+            }
+        } else {
 #pragma unroll
-        for (int g = 0; g < G; ++g) {
-            errs[g] = 0;
-            cnt[g] = 0;
-            st[g] = 0;
-            if (!live[g]) continue;
-            if (!in[g]) {  // normative bound (the reference reads one past the end at t == |col|)
-                errs[g] = 1u;
-                continue;
+            for (int g = 0; g < G; ++g) {
+                const uint64_t t = raw[g].c * o_inv;
+                const bool in = t < col_n;
+                mid.past |= (in ? 0u : 1u) << g;
+                idx[g] = in ? static_cast<uint32_t>(t) : 0u;
             }
-            const uint64_t x = v[g] & omask;
-            if (col.encoded && ((x * col.a_inv) & omask) > col.max_u) {
-                errs[g] = 2u;
-                st[g] = t[g];
-                continue;
+        }
+        if (table == kFetchRaw) {
+            const T *t = reinterpret_cast<const T *>(lds);
+#pragma unroll
+            for (int g = 0; g < G; ++g) mid.v[g] = t[idx[g]];
+            return;
+        }
+        if constexpr (ENC && sizeof(T) <= 4) {
+            const FetchPack *p = reinterpret_cast<const FetchPack *>(lds);
+            const uint32_t covered = table == kFetchPacked ? uniform(p->covered) : 0u;
+            if (covered != 0u) {
+                const uint32_t bits = uniform(p->bits), base = uniform(p->lo) * a;
+                const uint32_t ones = bits == 32u ? 0xFFFFFFFFu : (1u << bits) - 1u;
+                mid.clean = uniform(p->full) != 0u;
+                uint32_t x[G];
+                if (bits == 8u) {
+                    const uint8_t *t = reinterpret_cast<const uint8_t *>(p + 1);
+#pragma unroll
+                    for (int g = 0; g < G; ++g) x[g] = t[idx[g] < covered ? idx[g] : 0u];
+                } else if (bits == 16u) {
+                    const uint16_t *t = reinterpret_cast<const uint16_t *>(p + 1);
+#pragma unroll
+                    for (int g = 0; g < G; ++g) x[g] = t[idx[g] < covered ? idx[g] : 0u];
+                } else {
+                    const uint32_t *t = reinterpret_cast<const uint32_t *>(p + 1);
+                    const uint32_t per = uniform(p->per), magic = uniform(p->magic);
+#pragma unroll
+                    for (int g = 0; g < G; ++g) {
+                        const uint32_t i = idx[g] < covered ? idx[g] : 0u;
+                        const uint32_t q = per > 1u ? __umulhi(i, magic) : i;
+                        x[g] = (t[q] >> (__umul24(i - q * per, bits))) & ones;
+                    }
+                }
+#pragma unroll
+                for (int g = 0; g < G; ++g) mid.v[g] = static_cast<T>(x[g] * a + base);
+                if (!mid.clean) {
+#pragma unroll
+                    for (int g = 0; g < G; ++g) {
+                        if (idx[g] >= covered || x[g] == ones) mid.v[g] = col[idx[g]];
+                    }
+                }
+                return;
             }
-            st[g] = reenc ? (x * f) & omask : x;
-            cnt[g] = 1;
         }
+#pragma unroll
+        for (int g = 0; g < G; ++g) mid.v[g] = col[idx[g]];
     }
-    __device__ uint32_t eval(uint64_t row, State &st, uint32_t &errs, uint64_t &) const {
-        const uint64_t t = oids.raw(row) * oids.a_inv;
-        if (t >= col.n) {  // normative bound (the reference reads one past the end at t == |col|)
-            errs = 1u;
-            st = 0;
-            return 0;
+    template <int G>
+    __device__ __forceinline__ void close_tile(const Mid<G> &mid, uint32_t live, State (&st)[G], uint32_t &keep,
+                                               uint32_t (&errs)[kErr]) const {
+        uint32_t bad = 0;
+#pragma unroll
+        for (int g = 0; g < G; ++g) st[g] = static_cast<Out>(mid.v[g]);
+        if constexpr (ENC) {
+            if (!mid.clean) {
+#pragma unroll
+                for (int g = 0; g < G; ++g) bad |= (an_mul<T>(mid.v[g], a_inv) > max_u ? 1u : 0u) << g;
+            }
         }
-        const uint64_t v = col.raw(t) & omask;
-        if (col.encoded && ((v * col.a_inv) & omask) > col.max_u) {
-            errs = 2u;
-            st = t;
-            return 0;
+        if (reenc) {
+#pragma unroll
+            for (int g = 0; g < G; ++g) st[g] = an_mul<Out>(st[g], f);
         }
-        st = reenc ? (v * f) & omask : v;
-        return 1;
+        errs[0] = live & mid.past;
+        errs[1] = live & ~mid.past & bad;
+        keep = live & ~mid.past & ~bad;
     }
-    __device__ void emit_main(uint64_t, const State &st, uint64_t pos, uint32_t) const {
-        if (pos < out_cap) store_w(out, pos, ow, st);
+    __device__ void report(uint64_t row, State &, uint32_t &errs) const {
+        const uint64_t t = oids[row] * o_inv;
+        if (t >= col_n) errs = 1u;
+        else if (ENC && an_mul<T>(col[t], a_inv) > max_u) errs = 2u;
     }
-    __device__ void emit_err(int e, uint64_t row, const State &st, uint64_t pos) const {
+    __device__ __forceinline__ void emit(const State &st, uint64_t, uint64_t pos, uint32_t, uint32_t k) const {
+        __builtin_nontemporal_store(st, out + pos + k);
+    }
+    __device__ void emit_err(int e, uint64_t row, const State &, uint64_t pos) const {
         if (e == 0) {
             if (pos < e1_cap) e1[pos] = row * a_oid;
         } else if (pos < e2_cap) {
-            e2[pos] = st * a_oid;
+            e2[pos] = oids[row] * o_inv * a_oid;
         }
     }
-    __device__ void tile_done(uint32_t, uint64_t) const {}
     __device__ void finish(const uint64_t *t) const {
         d_counts[0] = t[0];
         d_counts[1] = t[1];
         d_counts[2] = t[2];
     }
 };
+
+template <typename T, bool ENC>
+int launch_fetch(const ahead_col *oids, const ahead_col *col, int reenc, uint64_t a_reenc, uint64_t a_oid,
+                 ahead_buf out, ahead_buf err1, ahead_buf err2, uint64_t *d_counts, ahead_hip_ws *ws, hipStream_t s) {
+    using Op = FetchOp<T, ENC>;
+    Op op{};
+    op.n = oids->n;
+    op.oids = static_cast<const uint64_t *>(oids->data);
+    op.o_inv = oids->a_inv;
+    op.o_back = ahead_host::back_factor(oids->a_inv, 0xFFFFFFFFull);  // positions are below |col| < 2^32
+    // an empty column is never read, but its row 0 is addressed: any readable element stands in
+    op.col = static_cast<const T *>(col->n ? col->data : oids->data);
+    op.col_n = static_cast<uint32_t>(col->n);
+    op.a = static_cast<T>(col->a);
+    op.a_inv = static_cast<T>(col->a_inv);
+    op.max_u = static_cast<T>(col->max_u);
+    op.reenc = reenc != 0;
+    // matchjoinAN.tcc:323-327: re-encoding factor A_R * inv(A_col) (A_R alone for a plain column)
+    op.f = static_cast<typename Op::Out>(
+        reenc ? (ENC ? a_reenc * ahead_host::inverse_mod2k(col->a, 8 * sizeof(typename Op::Out)) : a_reenc) : 1);
+    op.a_oid = a_oid;
+    op.out = static_cast<typename Op::Out *>(out.data);
+    op.out_cap = out.data ? out.cap : 0;
+    op.e1 = static_cast<uint64_t *>(err1.data);
+    op.e1_cap = err1.data ? err1.cap : 0;
+    op.e2 = static_cast<uint64_t *>(err2.data);
+    op.e2_cap = err2.data ? err2.cap : 0;
+    op.d_counts = d_counts;
+    // A workgroup fills its table from L2 at about 100 KB per microsecond, the packed one after two small
+    // launches; a gather it saves is worth 3 ps over the whole card.  The codes of the column pay from 4
+    // OIDs a byte on, packed values from 16; packing serves columns up to 2 MB (below a quarter of the rows in
+    // LDS the kernel leaves it).  A corrupt value re-encodes differently from its decoded form, so the
+    // packed table needs A^-1 to be A's inverse.
+    const uint64_t bytes = col->n * sizeof(T);
+    size_t lds = 0;
+    if (col->n && bytes <= kFetchTableBytes && op.n / 4 >= bytes) {
+        op.table = kFetchRaw;
+        lds = bytes;
+    } else if (ENC && sizeof(T) <= 4 && bytes <= (2u << 20) && op.n / 16 >= bytes &&
+               static_cast<T>(static_cast<uint64_t>(op.a) * op.a_inv) == 1) {
+        if constexpr (ENC && sizeof(T) <= 4) {
+            const int st = ahead_host::ws_ensure(ws, kFetchTableBytes + kRangeBlocks * sizeof(FetchRange));
+            if (st != AHEAD_OK) return st;
+            FetchPack *pack = reinterpret_cast<FetchPack *>(ahead_host::ws_region(ws, 0));
+            FetchRange *ranges = reinterpret_cast<FetchRange *>(ahead_host::ws_region(ws, kFetchTableBytes));
+            hipLaunchKernelGGL(k_fetch_range<T>, dim3(kRangeBlocks), dim3(kBlock), 0, s, op.col, op.col_n, op.a_inv,
+                               op.max_u, ranges);
+            hipLaunchKernelGGL(k_fetch_pack<T>, dim3((kFetchWords + kBlock - 1) / kBlock), dim3(kBlock), 0, s, op.col,
+                               op.col_n, op.a_inv, op.max_u, ranges, pack);
+            AHEAD_HIP_TRY(hipGetLastError());
+            op.pack = pack;
+            op.table = kFetchPacked;
+            lds = kFetchTableBytes;
+        }
+    }
+    return ahead_host::launch_stream(op, ws, s, lds);
+}
 
 // ---------------------------------------------------------------------------------------------------
 struct MatchPosState {
@@ -473,26 +717,15 @@ extern "C" int ahead_hip_fetchjoin_an(const ahead_col *oids, const ahead_col *co
     if ((st = check_col(col, "fetchjoin.col", false, false)) != AHEAD_OK) return st;
     if (oids->width != 8) return fail(AHEAD_ERR_INVALID, "fetchjoin: OIDs are resoid (8-byte) codes");
     if (d_counts == nullptr) return fail(AHEAD_ERR_INVALID, "fetchjoin: d_counts is NULL");
-    FetchOp op{};
-    op.n = oids->n;
-    op.oids = dcol(*oids);
-    op.col = dcol(*col);
-    op.ow = encoded_width(*col);
-    op.omask = width_mask(op.ow);
-    op.reenc = reenc != 0;
-    // matchjoinAN.tcc:323-327: re-encoding factor A_R * inv(A_col) (A_R alone for a plain column)
-    op.f = reenc ? (col->encoded ? (a_reenc * inverse_mod2k(col->a, 8 * op.ow)) & op.omask : a_reenc & op.omask) : 1;
-    op.a_oid = a_oid;
-    op.out = out.data;
-    op.out_cap = out.data ? out.cap : 0;
-    op.e1 = static_cast<uint64_t *>(err1.data);
-    op.e1_cap = err1.data ? err1.cap : 0;
-    op.e2 = static_cast<uint64_t *>(err2.data);
-    op.e2_cap = err2.data ? err2.cap : 0;
-    op.d_counts = d_counts;
-    // the streaming engine stages entries at their row's place: it needs room for every row
-    if (op.out != nullptr && op.out_cap >= op.n) return launch_map(op, ws, 0, static_cast<hipStream_t>(stream));
-    return launch_rowtile(op, op.n, 3, ws, static_cast<hipStream_t>(stream));
+    hipStream_t s = static_cast<hipStream_t>(stream);
+#define AHEAD_FETCH(T, E) launch_fetch<T, E>(oids, col, reenc, a_reenc, a_oid, out, err1, err2, d_counts, ws, s)
+    switch (col->width) {
+        case 1: return AHEAD_FETCH(uint8_t, false);
+        case 2: return col->encoded ? AHEAD_FETCH(uint16_t, true) : AHEAD_FETCH(uint16_t, false);
+        case 4: return col->encoded ? AHEAD_FETCH(uint32_t, true) : AHEAD_FETCH(uint32_t, false);
+        default: return col->encoded ? AHEAD_FETCH(uint64_t, true) : AHEAD_FETCH(uint64_t, false);
+    }
+#undef AHEAD_FETCH
 }
 
 extern "C" int ahead_hip_matchjoin_pos_an(const ahead_col *h1, const ahead_col *t1, const ahead_col *t2, int reenc_h,

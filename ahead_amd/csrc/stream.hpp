@@ -7,7 +7,7 @@
 // once, at its final place.  Nothing is staged, moved or re-read: the traffic is the inputs once
 // and the outputs once, whether rows are dropped or not.
 //
-// Bound by HBM as long as three latencies stay off the path (60M 8-byte codes checked and decoded
+// Bound by HBM as far as three latencies stay off the path (60M 8-byte codes checked and decoded
 // to 4 bytes, 720 MB, on one MI355X; the same loads and stores without any order take 103 us):
 //  - the place of a tile: a look-back that walks 64 predecessors at a time advances 128 tiles per
 //    device-scope round trip, and a round trip takes several microseconds while HBM is saturated
@@ -15,7 +15,10 @@
 //    and the inclusive prefix just before them; with one workgroup per CU that prefix belongs to a
 //    tile of an earlier generation and is there (170 us).  Windows of 256, 512 and 1024 tiles
 //    measured alike; 512 covers two tickets per CU.
-//  - the next tile's loads go out before the look-back's polls (128 us).
+//  - the next tile's loads go out between this tile's publication and its polls (128 us).  Earlier is
+//    worse: a count published behind loads in flight reaches the other workgroups after them (loads
+//    issued before the publication 172 us; a wave of its own for the places, with the other fifteen
+//    always loading, 209 us).
 //  - tickets come from one address, about 15 ns each: 7325 tiles of 8192 rows take 190 us, 3663 of
 //    16384 rows 128 us.
 //
@@ -30,9 +33,12 @@
 //   struct Raw; using State;            // a row's streamed inputs; what its entry needs
 //   uint64_t out_cap;                   // entries the outputs hold
 //   void load(uint64_t first, uint32_t k, Raw &) const;        // row first + k
-//   template <int G> void eval_tile(const char *lds, uint64_t first, uint32_t lane,
-//            const Raw (&)[G], uint32_t live, State (&)[G], uint32_t &keep, uint32_t (&err)[kErr]) const;
-//       // rows first + 64 g + lane; bit g of live: the row exists (raw is zero where it does not);
+//   template <int G> void open_tile(const char *lds, uint64_t first, uint32_t lane,
+//            const Raw (&)[G], Mid<G> &) const;
+//       // rows first + 64 g + lane: decodes them and issues their lookups (a row past the end has
+//       // the last row's inputs)
+//   template <int G> void close_tile(const Mid<G> &, uint32_t live, State (&)[G], uint32_t &keep,
+//            uint32_t (&err)[kErr]) const;
 //       // sets bit g of keep / err[e] for live rows that emit an entry / report into stream e
 //   void emit(const State &, uint64_t first, uint64_t pos, uint32_t row, uint32_t k) const;
 //       // entry pos + k, of row first + row (first and pos are wave-uniform: scalar bases)
@@ -58,6 +64,8 @@ struct StreamArgs {
     uint32_t tiles;
     uint32_t last;           // the launch's last ticket: tiles + workgroups - 1
 };
+
+__device__ __forceinline__ uint32_t uniform(uint32_t x) { return __builtin_amdgcn_readfirstlane(x); }
 
 // A ticket word's tile; the holder of the launch's last ticket starts the next epoch.
 __device__ __forceinline__ uint32_t stream_tile(const StreamArgs &m, unsigned long long v) {
@@ -90,30 +98,25 @@ __device__ __forceinline__ uint32_t wave_rank(uint64_t ballot) {
                                      __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(ballot), 0u));
 }
 
-// The streamed inputs of a lane's G rows first + 64 g + lane; left: rows of the wave that exist.
+// The streamed inputs of a lane's G rows first + 64 g + lane, of which the wave has `left`; rows past
+// the end repeat the last one (a wave past the end: row 0).
 template <class Op, int G>
 __device__ __forceinline__ void stream_load(const Op &op, uint64_t first, uint32_t lane, uint32_t left,
                                             typename Op::Raw (&raw)[G]) {
-    if (left == 64u * G) {
+    const uint64_t base = left != 0u ? first : 0ull;
+    const uint32_t top = left != 0u ? left - 1u : 0u;
 #pragma unroll
-        for (int g = 0; g < G; ++g) op.load(first, static_cast<uint32_t>(g * 64) + lane, raw[g]);
-    } else {
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-            const uint32_t k = static_cast<uint32_t>(g * 64) + lane;
-            raw[g] = typename Op::Raw{};
-            if (k < left) op.load(first, k, raw[g]);
-        }
+    for (int g = 0; g < G; ++g) {
+        const uint32_t k = static_cast<uint32_t>(g * 64) + lane;
+        op.load(base, k < top ? k : top, raw[g]);
     }
 }
-__device__ __forceinline__ uint32_t uniform(uint32_t x) { return __builtin_amdgcn_readfirstlane(x); }
 
 template <class Op>
 __global__ __launch_bounds__(kStreamThreads) void k_stream(Op op, StreamArgs m) {
     constexpr int G = Op::kG, NS = 1 + Op::kErr, NW = kStreamWaves;
     constexpr uint32_t kWaveRows = 64u * G, kAll = G == 32 ? 0xFFFFFFFFu : (1u << (G & 31)) - 1u;
-    static_assert(NS <= 64, "one wave polls the inclusive prefixes");
-    extern __shared__ char s_op[];
+    extern __shared__ __align__(16) char s_op[];
     __shared__ uint32_t s_cnt[NS][NW], s_sum[NS][NW];
     __shared__ uint32_t s_tile, s_epoch;
     if (op.skip()) return;
@@ -125,34 +128,38 @@ __global__ __launch_bounds__(kStreamThreads) void k_stream(Op op, StreamArgs m) 
     op.init(s_op);
     __syncthreads();
     const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t epoch = __builtin_amdgcn_readfirstlane(s_epoch);
-    uint32_t tile = __builtin_amdgcn_readfirstlane(s_tile);
+    const uint32_t wave = uniform(threadIdx.x >> 6);
+    const uint32_t epoch = uniform(s_epoch);
+    uint32_t tile = uniform(s_tile);
     auto first_of = [&](uint32_t t) { return (static_cast<uint64_t>(t) * NW + wave) * kWaveRows; };
-    auto left_of = [&](uint64_t first) {
+    auto left_of = [&](uint32_t t) {
+        const uint64_t first = first_of(t);
         return first >= op.n ? 0u : op.n - first < kWaveRows ? static_cast<uint32_t>(op.n - first) : kWaveRows;
     };
     typename Op::Raw raw[G];
-    if (tile < m.tiles) stream_load<Op, G>(op, first_of(tile), lane, left_of(first_of(tile)), raw);
+    if (tile < m.tiles && op.n != 0) stream_load<Op, G>(op, first_of(tile), lane, left_of(tile), raw);
     while (tile < m.tiles) {
-        unsigned long long ticket = 0;
+        unsigned long long ticket;  // the next tile's, taken by thread 0 while the inputs arrive
         if (threadIdx.x == 0) ticket = atomicAdd(m.te, 1ull);
         const uint64_t first = first_of(tile);
-        const uint32_t left = left_of(first);
-        uint32_t live = kAll;
-        if (left != kWaveRows) {
-            live = 0;
-#pragma unroll
-            for (int g = 0; g < G; ++g) live |= (static_cast<uint32_t>(g * 64) + lane < left ? 1u : 0u) << g;
-        }
+        const uint32_t left = left_of(tile);
         typename Op::State st[G];
         uint32_t keep = 0, err[Op::kErr] = {};
-        op.template eval_tile<G>(s_op, first, lane, raw, live, st, keep, err);
+        if (left != 0u) {  // (a wave past the last row has nothing to look up: its columns may be empty)
+            typename Op::template Mid<G> mid;
+            uint32_t live = kAll;  // rows of the lane that exist
+            if (left != kWaveRows) {
+                live = 0;
+#pragma unroll
+                for (int g = 0; g < G; ++g) live |= (static_cast<uint32_t>(g * 64) + lane < left ? 1u : 0u) << g;
+            }
+            op.template open_tile<G>(s_op, first, lane, raw, mid);
+            op.template close_tile<G>(mid, live, st, keep, err);
+        }
 
         // what the wave keeps and reports
         const bool whole = __ballot(keep == kAll) == ~0ull;
-        const uint32_t kept = whole ? kWaveRows : __builtin_amdgcn_readfirstlane(wave_sum(
-                                                      static_cast<uint32_t>(__popc(keep))));
+        const uint32_t kept = whole ? kWaveRows : wave_sum(static_cast<uint32_t>(__popc(keep)));
         uint32_t any = 0;
 #pragma unroll
         for (int e = 0; e < Op::kErr; ++e) any |= err[e];
@@ -172,6 +179,8 @@ __global__ __launch_bounds__(kStreamThreads) void k_stream(Op op, StreamArgs m) 
         uint32_t agg[NS], before[NS], rep = 0;
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
+            // (every lane reads every count: independent LDS reads, where a scan over lanes is a chain of
+            // twelve shuffles and cost 10 us)
             agg[s] = 0;
             before[s] = 0;
 #pragma unroll
@@ -192,8 +201,8 @@ __global__ __launch_bounds__(kStreamThreads) void k_stream(Op op, StreamArgs m) 
             }
             lb_store(&m.agg[tile], stream_word(epoch, (rep != 0u ? 1ull << 33 : 0ull) | agg[0]));
         }
-        const uint32_t next = __builtin_amdgcn_readfirstlane(s_tile);
-        if (next < m.tiles) stream_load<Op, G>(op, first_of(next), lane, left_of(first_of(next)), raw);
+        const uint32_t next = uniform(s_tile);
+        if (next < m.tiles) stream_load<Op, G>(op, first_of(next), lane, left_of(next), raw);
 
         // the counts of the kStreamWindow - 1 tiles before this one, and the prefix before them
         uint32_t sum[NS] = {};
@@ -208,13 +217,11 @@ __global__ __launch_bounds__(kStreamThreads) void k_stream(Op op, StreamArgs m) 
                         stream_poll(m, &m.erep[static_cast<size_t>(e) * m.tiles + tile - back], epoch));
             }
         }
-        if (wave == NW - 1 && tile >= kStreamWindow) {
+        if (wave == NW - 1 && tile >= kStreamWindow && lane < static_cast<uint32_t>(NS)) {
+            const uint32_t v = static_cast<uint32_t>(
+                stream_poll(m, &m.incl[static_cast<size_t>(lane) * m.tiles + tile - kStreamWindow], epoch));
 #pragma unroll
-            for (int s = 0; s < NS; ++s) {
-                if (lane == static_cast<uint32_t>(s))
-                    sum[s] += static_cast<uint32_t>(
-                        stream_poll(m, &m.incl[static_cast<size_t>(s) * m.tiles + tile - kStreamWindow], epoch));
-            }
+            for (int s = 0; s < NS; ++s) sum[s] += lane == static_cast<uint32_t>(s) ? v : 0u;
         }
 #pragma unroll
         for (int s = 0; s < NS; ++s) {

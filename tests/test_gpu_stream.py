@@ -106,3 +106,43 @@ def test_check_and_decode_graph_replays():
             assert c == [len(ref[0]), len(ref[1])]
             assert np.array_equal(dec.to_numpy(np.uint32, c[0]), ref[0])
             assert np.array_equal(err.to_numpy(np.uint64, c[1]), ref[1])
+
+
+@pytest.mark.parametrize("t,a,rows,n,span,bad,past", [
+    # 2-byte columns: codes in LDS up to 76,800 rows; packed values beyond, by the bits they need
+    (an.RESTINY, 233, 76_800, 700_001, 256, 0, 3), (an.RESTINY, 233, 76_801, 2_600_000, 256, 0, 0),
+    (an.RESTINY, 29, 200_000, 6_500_003, 256, 9, 5), (an.RESTINY, 29, 200_000, 6_500_003, 25, 4, 1),
+    (an.RESTINY, 29, 200_000, 6_500_003, 4, 0, 0), (an.RESTINY, 233, 1_000_001, 32_100_000, 256, 1, 2),
+    (an.RESTINY, 233, 200_000, 6_400_001, 1, 200_000, 0), (an.RESTINY, 233, 200_000, 6_399_999, 256, 2, 2),
+    # 4-byte columns, an offset far from zero, values too wide to pack
+    (an.RESSHORT, 63877, 38_400, 620_000, 65_536, 3, 1), (an.RESSHORT, 63877, 60_000, 3_900_000, 7, 1, 0),
+    (an.RESSHORT, 63877, 120_000, 7_700_000, 1000, 2, 2), (an.RESSHORT, 63877, 500_000, 32_000_001, 65_536, 2, 2),
+    # 8-byte and plain columns
+    (an.RESINT, 65117, 19_200, 620_000, 1 << 32, 2, 1), (an.RESINT, 65117, 19_201, 620_000, 1 << 32, 2, 1),
+    (an.TINYINT, 1, 150_000, 700_000, 256, 0, 2), (an.SHORTINT, 1, 5_000, 100_000, 65_536, 0, 2),
+    (an.INT, 1, 5_000, 100_000, 1 << 32, 0, 2), (an.RESTINY, 233, 1, 40_000, 256, 0, 7),
+])
+def test_fetch_tables(t, a, rows, n, span, bad, past):
+    """fetchjoinAN with its column in LDS (codes, packed values, in part) and from the column."""
+    rng = np.random.default_rng(rows + n + span)
+    meta = an.an_meta(t, a) if t.encoded else an.plain_meta(t)
+    lo = min(1992, (1 << t.unenc_bits) - span) if span < (1 << t.unenc_bits) else 0
+    v = (lo + rng.integers(0, span, rows)).astype(np.uint64)
+    col = datagen.encode(v, a, t.width) if t.encoded else v.astype(f"u{t.width}")
+    hit = rng.choice(rows, min(bad, rows), replace=False)
+    col[hit] ^= np.asarray(1 << 3, dtype=col.dtype)
+    pos = rng.integers(0, rows, n).astype(np.uint64)
+    if bad < rows:  # one fetch of each corrupt row, and few others
+        clean = np.setdiff1d(np.arange(min(rows, 1000)), hit)[0]
+        pos[np.isin(pos, hit)] = clean
+        pos[rng.choice(n, hit.size, replace=False)] = hit
+    pos[rng.choice(n, past, replace=False)] = rows + 7
+    with np.errstate(over="ignore"):
+        oids = pos * np.uint64(an.A_OID)
+    resoid = an.an_meta(an.RESOID, an.A_OID)
+    print(f"fetch {t.name} rows={rows} n={n} span={span} bad={bad}", flush=True)
+    for reenc, ar in ((0, 0), (1, 13)):
+        ref = O.fetchjoin_an(O.Col(oids, resoid), O.Col(col, meta), reenc, ar)
+        got = capi.fetchjoin_an(capi.Column.from_numpy(oids, resoid), capi.Column.from_numpy(col, meta), reenc, ar)
+        for i, (x, y) in enumerate(zip(got, ref)):
+            assert np.array_equal(np.asarray(x).astype(np.uint64), np.asarray(y).astype(np.uint64)), i
