@@ -92,7 +92,9 @@ struct CheckDecodeOp {
     uint64_t *d_counts;
 
     __device__ bool skip() const { return false; }
+    struct Uniform {};
     __device__ void init(char *) const {}
+    __device__ Uniform begin(const char *) const { return Uniform{}; }
     __device__ __forceinline__ void load(uint64_t first, uint32_t k, Raw &r) const {
         r.c = __builtin_nontemporal_load(codes + first + k);
     }
@@ -102,7 +104,8 @@ struct CheckDecodeOp {
         uint32_t bad;
     };
     template <int G>
-    __device__ __forceinline__ void open_tile(const char *, uint64_t, uint32_t, const Raw (&raw)[G], Mid<G> &mid) const {
+    __device__ __forceinline__ void open_tile(const char *, const Uniform &, uint64_t, uint32_t, uint32_t, const Raw (&raw)[G],
+                                              Mid<G> &mid) const {
         mid.bad = 0;
         if (sizeof(CodeT) == 8 && back != 0u) {
 #pragma unroll
@@ -121,7 +124,7 @@ struct CheckDecodeOp {
         }
     }
     template <int G>
-    __device__ __forceinline__ void close_tile(const Mid<G> &mid, uint32_t live, State (&st)[G], uint32_t &keep,
+    __device__ __forceinline__ void close_tile(const Uniform &, const Mid<G> &mid, uint32_t live, State (&st)[G], uint32_t &keep,
                                                uint32_t (&errs)[kErr]) const {
 #pragma unroll
         for (int g = 0; g < G; ++g) st[g] = mid.d[g];
@@ -131,7 +134,7 @@ struct CheckDecodeOp {
     __device__ void report(uint64_t row, State &, uint32_t &errs) const {
         errs = an_mul<CodeT>(codes[row], a_inv) > max_u ? 1u : 0u;
     }
-    __device__ __forceinline__ void emit(const State &st, uint64_t, uint64_t pos, uint32_t, uint32_t k) const {
+    __device__ __forceinline__ void emit(const Uniform &, const State &st, uint64_t, uint64_t pos, uint32_t, uint32_t k) const {
         __builtin_nontemporal_store(st, dec + pos + k);
     }
     __device__ void emit_err(int, uint64_t row, const State &, uint64_t pos) const {

@@ -22,7 +22,7 @@
 //             every probe row in probe order, build rows in insertion order.
 // Both hash sides (hash_side_t::right / ::left) and the re-encoding variants are supported.
 #include "htable.hpp"
-#include "maptile.hpp"
+#include "stream.hpp"
 
 using namespace ahead_dev;
 
@@ -328,14 +328,6 @@ struct ProbeState {
     uint32_t brow;  // the build row (keys with one row)
 };
 
-// The lean probe's row: the build row and, for 8-byte build payloads, the payload code itself,
-// gathered while the row is evaluated (before any store of the step).
-struct LeanState {
-    uint64_t pay;   // probe-side payload (raw)
-    uint64_t bval;  // build-side payload code (8-byte build payloads)
-    uint32_t brow;  // the build row
-};
-
 struct ProbeOp {
     static constexpr int kErr = 2;  // probe head check, probe tail check
     static constexpr bool kMulti = true, kMain = true, kAcc = false;
@@ -358,14 +350,9 @@ struct ProbeOp {
     uint64_t cap[2];
     uint64_t *counts;         // [0] pairs, error counts at [e_index[0]], [e_index[1]]
     uint32_t e_index[2];
-    uint32_t map_launched;    // a streaming-engine probe (ProbeMapOp, or ProbeLeanOp when lean) was launched before
-    uint32_t lean;            // ... and it was the ProbeLeanOp pair, which takes probes that miss too
 
-    // the tile engine runs this probe when some build key has several rows, when some sampled probe
-    // row finds no key, or when the streaming probe could not be launched
-    __device__ bool skip() const {
-        return map_launched != 0u && t.flags[0] == 0u && (lean != 0u || t.flags[6] == 0u);
-    }
+    // the tile engine runs this probe when some build key has several rows
+    __device__ bool skip() const { return t.flags[0] == 0u; }
 
     static constexpr bool kBatched = true;
     template <int G>
@@ -473,48 +460,62 @@ struct ProbeOp {
     }
 };
 
-// The probe on the streaming engine: when no build key has several rows, a probe row emits at
-// most one pair.  The engine stages each wave's pairs in place and moves them once the offsets are
-// known; when rows emit nothing the waves leave gaps that, beyond kMaxShift rows in all, cannot be
-// closed in place and every row is evaluated twice, so a probe that misses runs on the tile engine.
-struct ProbeMapOp : ProbeOp {
-    static constexpr bool kMulti = false;
-    static constexpr int kOuts = 2;
-    __device__ bool skip() const { return t.flags[0] != 0u || t.flags[6] != 0u; }
-    __device__ void out_arrays(void *(&p)[2], uint32_t (&w)[2]) const {
-        p[0] = out_h;
-        p[1] = out_t;
-        w[0] = build_right ? w_p : w_b;
-        w[1] = build_right ? w_b : w_p;
+// v * f, the product skipped where f is 1 (f is the same for every row: a branch the compiler must not
+// turn into a product for every row)
+__device__ __forceinline__ uint64_t reencode(uint64_t v, uint64_t f) {
+    if (f != 1ull) {
+        asm volatile("" : "+v"(v));
+        v *= f;
     }
+    return v;
+}
+
+// The probe on the single-pass engine: when no build key has several rows, a probe row emits at most one
+// pair.
+struct ProbeOneOp : ProbeOp {
+    static constexpr bool kMulti = false;
+    __device__ bool skip() const { return t.flags[0] != 0u; }
 };
 
-// The probe for its common shapes, on the streaming engine: every build key has one row, the probe
+// The probe for its common shapes, on the single-pass engine: every build key has one row, the probe
 // key column holds KW-byte codes, the probe payload is void (PV) or of 8-byte codes, the build
-// payload is void (BV) or of 8-byte codes, and both outputs are 4 or 8 bytes wide.  The same results as
+// payload is void (BV) or of 8-byte codes, and both outputs are OW (4 or 8) bytes wide.  The same results as
 // ProbeOp (hashjoinAN.tcc:150-220 probe loop), with the widths fixed at compile time: a row costs
-// its loads, one or two products, the lookup and, when it joins, two stores.
-template <bool FILT>
-struct LeanFilter {};
-template <>
-struct LeanFilter<true> {
-    static constexpr int kFilterWords = static_cast<int>(kHjFiltWords);
-};
-
-template <int KW, bool PV, bool BV, bool FILT>
-struct ProbeLeanOp : LeanFilter<FILT> {
+// its loads, two products, the lookup and, when it joins, two stores.  When some sampled probe row
+// found no key (flags[6]), the filter of the build keys is kept in LDS (8-byte keys) and only rows it
+// passes look their key up.
+// 60M foreign keys, 8-byte codes: every row joining a dimension of 200,000 void rows took 215 us and 178
+// for moving the pairs behind the first row that drops, now 235 in one pass; a fifth of them joining
+// 40,000 rows, re-encoded to 8-byte pairs, took 325 us and 135 for the two compaction passes, now 290.
+template <int KW, bool PV, bool BV, int OW>
+struct ProbeLeanOp {
     static constexpr int kErr = 2;  // probe head check, probe tail check
-    static constexpr bool kMulti = false, kMain = true, kAcc = false, kBatched = true;
-    static constexpr int kOuts = 2;
-    // 8 rows per lane and step: half the steps, so half the waits of a step's loads for the
-    // previous step's stores (one counter covers both)
-    static constexpr int kMapRows = 8;
-    using State = LeanState;
+    // void payloads: a row's state is its build row, or the build payload; else two 8-byte codes
+    static constexpr int kG = PV ? 16 : 8;
     using KT = std::conditional_t<KW == 8, uint64_t, uint32_t>;
+    using OT = std::conditional_t<OW == 8, uint64_t, uint32_t>;
+    struct RawV {
+        KT key;
+    };
+    struct RawP {
+        KT key;
+        uint64_t pay;
+    };
+    using Raw = std::conditional_t<PV, RawV, RawP>;
+    using BT = std::conditional_t<BV, uint32_t, uint64_t>;  // the build row, or its payload
+    struct StateV {
+        BT b;
+    };
+    struct StateP {
+        BT b;
+        uint64_t pay;
+    };
+    using State = std::conditional_t<PV, StateV, StateP>;
     uint64_t n;
     HjTable t;
     const KT *key;                            // probe key codes
     uint64_t key_inv, key_cmask, key_maxu;    // decode (key_enc != 0) and the code-width mask
+    uint32_t key_back;                        // the key's A where 32-bit arithmetic decodes it (back_factor), else 0
     uint32_t key_enc, key_err;                // error bit of the key side: 0 probe head, 1 probe tail
     const uint64_t *pay;                      // probe payload codes (PV: void, pay_seq + row)
     uint64_t pay_seq, pay_inv, pay_maxu;
@@ -522,151 +523,185 @@ struct ProbeLeanOp : LeanFilter<FILT> {
     const uint64_t *bpay;                     // build payload codes (BV: void, bpay_seq + row)
     uint64_t bpay_seq;
     uint64_t guard_mask, key_mask, build_max;
-    uint32_t reenc_p, reenc_b;
-    uint64_t f_p, f_b;
-    void *out_p, *out_b;                      // probe / build payload outputs
-    uint32_t ow;                              // their width: 4 or 8 bytes
-    void *out_h, *out_t;
+    uint64_t f_p, f_b;                        // re-encoding factors (1: none)
+    OT *out_p, *out_b;                        // probe / build payload outputs
     uint64_t out_cap;
     uint64_t a_oid;
     uint64_t *err[2];
     uint64_t cap[2];
     uint64_t *counts;
     uint32_t e_index[2];
-    uint32_t pair_launched;  // !FILT: the FILT variant was launched too (it takes probes that miss)
 
-    // a build key with several rows: the tile engine's ProbeOp runs instead.  FILT: only probes in
-    // which some sampled row finds no key (flags[6]); its twin without the filter takes the others.
-    __device__ bool skip() const {
-        if (t.flags[0] != 0u) return true;
-        return FILT ? t.flags[6] == 0u : (pair_launched != 0u && t.flags[6] != 0u);
+    // a build key with several rows: the tile engine's ProbeOp runs instead
+    __device__ bool skip() const { return t.flags[0] != 0u; }
+    struct Uniform {
+        uint32_t lo, hi, filtered, dense, ident;
+    };
+    __device__ Uniform begin(const char *) const {
+        return Uniform{uniform(t.flags[3]), uniform(t.flags[5]), KW == 8 ? uniform(t.flags[6]) : 0u,
+                       uniform(t.flags[4]), uniform(t.flags[7]) == 0u ? 1u : 0u};
     }
-    __device__ void filter_init(uint64_t *s) const {
-        for (uint32_t i = threadIdx.x; i < kHjFiltWords; i += kBlock) s[i] = t.filt[i];
+    __device__ void init(char *lds) const {
+        if (KW != 8 || t.flags[6] == 0u) return;
+        const uint4 *src = reinterpret_cast<const uint4 *>(t.filt);
+        uint4 *dst = reinterpret_cast<uint4 *>(lds);
+        for (uint32_t i = threadIdx.x; i < kHjFiltWords / 2; i += kStreamThreads) dst[i] = src[i];
     }
-    template <int G>
-    __device__ __forceinline__ void eval_f(const uint64_t (&row)[G], const bool (&live)[G], State (&st)[G],
-                                           uint32_t (&errs)[G], uint32_t (&cnt)[G], uint64_t &acc,
-                                           const uint64_t *filt) const {
-        eval_core<G>(row, live, st, errs, cnt, filt);
-    }
-    __device__ void out_arrays(void *(&p)[2], uint32_t (&w)[2]) const {
-        p[0] = out_h;
-        p[1] = out_t;
-        w[0] = ow;
-        w[1] = ow;
+    __device__ __forceinline__ void load(uint64_t first, uint32_t k, Raw &r) const {
+        r.key = __builtin_nontemporal_load(key + first + k);
+        if constexpr (!PV) r.pay = __builtin_nontemporal_load(pay + first + k);
     }
     template <int G>
-    __device__ __forceinline__ void eval_n(const uint64_t (&row)[G], const bool (&live)[G], State (&st)[G],
-                                           uint32_t (&errs)[G], uint32_t (&cnt)[G], uint64_t &) const {
-        eval_core<G>(row, live, st, errs, cnt, nullptr);
-    }
-    // filt: the probe filter in LDS, or NULL
-    template <int G>
-    __device__ __forceinline__ void eval_core(const uint64_t (&row)[G], const bool (&live)[G], State (&st)[G],
-                                              uint32_t (&errs)[G], uint32_t (&cnt)[G], const uint64_t *filt) const {
-        KT x[G];
-        uint64_t p[G];
+    struct Mid {
+        State st[G];
+        uint32_t keep, kbad, pbad;
+    };
+    // build rows of the live rows with a usable key (ok); clears ok of a row without one
+    template <int G, typename K>
+    __device__ __forceinline__ void lookup(const char *lds, const Uniform &u, const K (&k)[G], bool (&ok)[G],
+                                           uint32_t (&brow)[G]) const {
+        const uint32_t span = u.hi - u.lo;
+        if (u.filtered != 0u) {
+            const uint32_t *f = reinterpret_cast<const uint32_t *>(lds);
+            if (u.lo <= u.hi && span < kHjFiltBits) {  // exact: the bit of key - smallest (filt_bit)
+                uint32_t w[G];
 #pragma unroll
-        for (int g = 0; g < G; ++g) {
-            x[g] = key[live[g] ? row[g] : 0ull];
-            p[g] = PV ? static_cast<uint64_t>(static_cast<uint32_t>(pay_seq + row[g])) : pay[live[g] ? row[g] : 0ull];
-        }
-        bool ok[G];
-        uint64_t k[G];
+                for (int g = 0; g < G; ++g) {
+                    const K rel = k[g] - u.lo;
+                    ok[g] = ok[g] && rel <= span;
+                    w[g] = f[ok[g] ? static_cast<uint32_t>(rel) >> 5 : 0u];
+                }
 #pragma unroll
-        for (int g = 0; g < G; ++g) {
-            const uint64_t c = x[g];
-            const uint64_t d = key_enc ? (c * key_inv) & key_cmask : c;
-            const bool kb = key_enc && d > key_maxu;
-            const bool pb = !PV && pay_enc && p[g] * pay_inv > pay_maxu;
-            errs[g] = live[g] ? ((kb ? 1u : 0u) << key_err) | ((pb ? 1u : 0u) << (1u - key_err)) : 0u;
-            st[g].pay = p[g];
-            ok[g] = live[g] && (d & guard_mask) <= build_max;
-            k[g] = d & key_mask;
-            cnt[g] = 0;
-        }
-        if (filt != nullptr) {
+                for (int g = 0; g < G; ++g)
+                    ok[g] = ok[g] && ((w[g] >> (static_cast<uint32_t>(k[g] - u.lo) & 31u)) & 1u);
+            } else {
 #pragma unroll
-            for (int g = 0; g < G; ++g) {
-                const uint32_t b = filt_bit(t.flags, k[g]);
-                ok[g] = ok[g] && b != UINT32_MAX && ((filt[b >> 6] >> (b & 63u)) & 1ull) != 0ull;
-            }
-        }
-        if (t.flags[4] != 0u && t.flags[7] == 0u) {  // identity map: build row = key - smallest
-            const uint64_t lo = t.flags[3], span = t.flags[5] - t.flags[3];
-#pragma unroll
-            for (int g = 0; g < G; ++g) {
-                const uint64_t rel = k[g] - lo;
-                if (ok[g] && rel <= span) {
-                    st[g].brow = static_cast<uint32_t>(rel);
-                    cnt[g] = 1;
+                for (int g = 0; g < G; ++g) {
+                    const uint32_t b = filt_bit(t.flags, k[g]);
+                    ok[g] = ok[g] && b != UINT32_MAX;
+                    ok[g] = ok[g] && ((f[ok[g] ? b >> 5 : 0u] >> (b & 31u)) & 1u);
                 }
             }
-        } else if (t.flags[4] != 0u) {  // direct map: one gather per row (one row per key: no flag bit)
-            const uint64_t lo = t.flags[3], span = t.flags[5] - t.flags[3];
-            uint32_t e[G];
+        }
+        if (u.dense != 0u) {  // direct map (one row per key: no flag bit)
 #pragma unroll
             for (int g = 0; g < G; ++g) {
-                const uint64_t rel = k[g] - lo;
+                const K rel = k[g] - u.lo;
                 ok[g] = ok[g] && rel <= span;
-                e[g] = t.dmap[ok[g] ? rel : 0ull];
+                brow[g] = static_cast<uint32_t>(rel);
             }
+            if (u.ident == 0u) {  // (identity: build row = key - smallest)
 #pragma unroll
-            for (int g = 0; g < G; ++g) {
-                if (ok[g] && e[g] != 0u) {
-                    st[g].brow = e[g] - 1u;
-                    cnt[g] = 1;
+                for (int g = 0; g < G; ++g) {
+                    if (ok[g]) brow[g] = t.dmap[brow[g]] - 1u;  // 0: no row
                 }
+#pragma unroll
+                for (int g = 0; g < G; ++g) ok[g] = ok[g] && brow[g] != UINT32_MAX;
             }
         } else {
-            uint32_t sl[G];
-            t.ht.find_n<G>(k, ok, sl);
-            uint32_t f[G];
+            constexpr int C = 4;  // (more at once do not fit the registers)
 #pragma unroll
-            for (int g = 0; g < G; ++g) f[g] = t.first[sl[g] != UINT32_MAX ? sl[g] : 0u];
+            for (int q = 0; q < G; q += C) {
+                uint32_t sl[C];
+                uint64_t k64[C];
+                bool on[C];
 #pragma unroll
-            for (int g = 0; g < G; ++g) {
-                if (sl[g] != UINT32_MAX) {
-                    st[g].brow = f[g];
-                    cnt[g] = 1;
+                for (int i = 0; i < C; ++i) {
+                    k64[i] = k[q + i];
+                    on[i] = ok[q + i];
+                }
+                t.ht.template find_n<C>(k64, on, sl);
+#pragma unroll
+                for (int i = 0; i < C; ++i) {
+                    brow[q + i] = t.first[sl[i] != UINT32_MAX ? sl[i] : 0u];
+                    ok[q + i] = ok[q + i] && sl[i] != UINT32_MAX;
                 }
             }
         }
-        if constexpr (!BV) {  // the build payloads of the joined rows, all before the step's stores
+    }
+    template <int G>
+    __device__ __forceinline__ void open_tile(const char *lds, const Uniform &u, uint64_t, uint32_t, uint32_t live, const Raw (&raw)[G],
+                                              Mid<G> &mid) const {
+        bool ok[G];
+        uint32_t brow[G];
+        mid.kbad = 0;
+        mid.pbad = 0;
+#pragma unroll
+        for (int g = 0; g < G; ++g) ok[g] = (live >> g) & 1u;
+        if (KW == 8 && key_back != 0u) {
+            uint32_t k[G];
+            const uint32_t inv = static_cast<uint32_t>(key_inv), top = static_cast<uint32_t>(key_maxu),
+                           mask = static_cast<uint32_t>(key_mask);
 #pragma unroll
             for (int g = 0; g < G; ++g) {
-                st[g].bval = 0;
-                if (cnt[g] != 0u) st[g].bval = bpay[st[g].brow];
+                const uint32_t d = static_cast<uint32_t>(raw[g].key) * inv;
+                mid.kbad |= (static_cast<uint64_t>(d) * key_back != raw[g].key || d > top ? 1u : 0u) << g;
+                k[g] = d & mask;
+            }
+            if (guard_mask > build_max) {
+#pragma unroll
+                for (int g = 0; g < G; ++g)
+                    ok[g] = ok[g] && ((static_cast<uint32_t>(raw[g].key) * inv) & static_cast<uint32_t>(guard_mask)) <=
+                                         static_cast<uint32_t>(build_max);
+            }
+            lookup<G, uint32_t>(lds, u, k, ok, brow);
+        } else {
+            uint64_t k[G];
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                const uint64_t c = raw[g].key;
+                const uint64_t d = key_enc ? (c * key_inv) & key_cmask : c;
+                mid.kbad |= (key_enc && d > key_maxu ? 1u : 0u) << g;
+                ok[g] = ok[g] && (d & guard_mask) <= build_max;
+                k[g] = d & key_mask;
+            }
+            lookup<G, uint64_t>(lds, u, k, ok, brow);
+        }
+        if constexpr (!PV) {
+            if (pay_enc) {
+#pragma unroll
+                for (int g = 0; g < G; ++g) mid.pbad |= (raw[g].pay * pay_inv > pay_maxu ? 1u : 0u) << g;
+            }
+#pragma unroll
+            for (int g = 0; g < G; ++g) mid.st[g].pay = raw[g].pay;
+        }
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            mid.st[g].b = BV ? brow[g] : 0u;
+            if constexpr (!BV) {  // the payloads of the joined rows
+                if (ok[g]) mid.st[g].b = bpay[brow[g]];
             }
         }
+        mid.keep = 0;
+#pragma unroll
+        for (int g = 0; g < G; ++g) mid.keep |= (ok[g] ? 1u : 0u) << g;
     }
-    __device__ uint32_t eval(uint64_t row, State &st, uint32_t &errs, uint64_t &acc) const {
-        const uint64_t r[1] = {row};
-        const bool l[1] = {row < n};
-        State s1[1];
-        uint32_t e1[1], c1[1];
-        eval_n<1>(r, l, s1, e1, c1, acc);
-        st = s1[0];
-        errs = e1[0];
-        return c1[0];
+    template <int G>
+    __device__ __forceinline__ void close_tile(const Uniform &, const Mid<G> &mid, uint32_t live, State (&st)[G], uint32_t &keep,
+                                               uint32_t (&errs)[kErr]) const {
+#pragma unroll
+        for (int g = 0; g < G; ++g) st[g] = mid.st[g];
+        keep = live & mid.keep;
+        errs[0] = live & (key_err == 0u ? mid.kbad : mid.pbad);
+        errs[1] = live & (key_err == 0u ? mid.pbad : mid.kbad);
     }
-    __device__ void emit_main(uint64_t, const State &st, uint64_t pos, uint32_t) const {
-        if (pos >= out_cap) return;
-        const uint64_t b = BV ? static_cast<uint64_t>(static_cast<uint32_t>(bpay_seq + st.brow)) : st.bval;
-        const uint64_t pv = reenc_p ? st.pay * f_p : st.pay, bv = reenc_b ? b * f_b : b;
-        if (ow == 8) {
-            static_cast<uint64_t *>(out_p)[pos] = pv;
-            static_cast<uint64_t *>(out_b)[pos] = bv;
-        } else {  // 4-byte outputs keep the low half, as store_w does
-            static_cast<uint32_t *>(out_p)[pos] = static_cast<uint32_t>(pv);
-            static_cast<uint32_t *>(out_b)[pos] = static_cast<uint32_t>(bv);
-        }
+    __device__ void report(uint64_t row, State &, uint32_t &errs) const {
+        const uint64_t c = key[row];
+        if (key_enc && ((c * key_inv) & key_cmask) > key_maxu) errs |= 1u << key_err;
+        if (!PV && pay_enc && pay[row] * pay_inv > pay_maxu) errs |= 1u << (1u - key_err);
+    }
+    __device__ __forceinline__ void emit(const Uniform &, const State &st, uint64_t first, uint64_t pos, uint32_t row, uint32_t k) const {
+        uint64_t p;
+        if constexpr (PV) p = static_cast<uint32_t>(static_cast<uint32_t>(pay_seq + first) + row);
+        else p = st.pay;
+        const uint64_t b = BV ? static_cast<uint64_t>(static_cast<uint32_t>(bpay_seq + st.b)) : st.b;
+        // 4-byte outputs keep the low half, as store_w does
+        __builtin_nontemporal_store(static_cast<OT>(reencode(p, f_p)), out_p + pos + k);
+        __builtin_nontemporal_store(static_cast<OT>(reencode(b, f_b)), out_b + pos + k);
     }
     __device__ void emit_err(int e, uint64_t row, const State &, uint64_t pos) const {
         if (pos < cap[e]) err[e][pos] = row * a_oid;
     }
-    __device__ void tile_done(uint32_t, uint64_t) const {}
     __device__ void finish(const uint64_t *tot) const {
         counts[0] = tot[0];
         counts[e_index[0]] = tot[1];
@@ -674,32 +709,23 @@ struct ProbeLeanOp : LeanFilter<FILT> {
     }
 };
 
-// Calls f with each ProbeLeanOp variant of the given shape: without the filter, and (8-byte keys)
-// with it.  Returns whether the shape has a variant with the filter.
+// Calls f with the ProbeLeanOp of the given shape.
 template <class F>
-bool lean_shape(uint32_t kw, bool pv, bool bv, F &&f) {
-#define AHEAD_LEAN(K, P, B, FL)                     \
-    if (kw == K && pv == P && bv == B) {            \
-        f(ProbeLeanOp<K, P, B, false>{});           \
-        if (FL) f(ProbeLeanOp<K, P, B, FL>{});      \
-        return FL;                                  \
-    }
-    AHEAD_LEAN(8, true, true, true)
-    AHEAD_LEAN(8, true, false, true)
-    AHEAD_LEAN(8, false, true, true)
-    AHEAD_LEAN(8, false, false, true)
-    AHEAD_LEAN(4, true, true, false)
-    AHEAD_LEAN(4, true, false, false)
-    AHEAD_LEAN(4, false, true, false)
-    AHEAD_LEAN(4, false, false, false)
+void lean_shape(uint32_t kw, bool pv, bool bv, uint32_t ow, F &&f) {
+#define AHEAD_LEAN(K, P, B, W) \
+    if (kw == K && pv == P && bv == B && ow == W) f(ProbeLeanOp<K, P, B, W>{});
+#define AHEAD_LEAN_KW(K)                                                                        \
+    AHEAD_LEAN(K, true, true, 4) AHEAD_LEAN(K, true, false, 4) AHEAD_LEAN(K, false, true, 4)    \
+    AHEAD_LEAN(K, false, false, 4) AHEAD_LEAN(K, true, true, 8) AHEAD_LEAN(K, true, false, 8)   \
+    AHEAD_LEAN(K, false, true, 8) AHEAD_LEAN(K, false, false, 8)
+    AHEAD_LEAN_KW(8)
+    AHEAD_LEAN_KW(4)
+#undef AHEAD_LEAN_KW
 #undef AHEAD_LEAN
-    return false;
 }
 
 // Whether every one of kHjSamples evenly spaced probe rows finds a build key: flags[6] = 1 when
-// some do not.  The streaming engine closes the gaps of dropped rows in place only while they total
-// at most kMaxShift rows, so it suits probes where (nearly) every row finds its key, as foreign
-// keys into a whole dimension do.  It only picks the engine; both give the same results.
+// some do not.  It only picks whether the probe keeps the filter in LDS; the results are the same.
 constexpr uint32_t kHjSamples = 4096;  // one per thread of kHjSamples / kBlock workgroups
 __global__ __launch_bounds__(kBlock) void k_hj_sample(ProbeOp p, uint64_t np) {
     const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
@@ -761,18 +787,8 @@ extern "C" int ahead_hip_hashjoin_an(const ahead_col *h1, const ahead_col *t1, c
     const ahead_col &ppay = right ? phead : ptail;
     const uint32_t lean_kw = pkey.data ? pkey.width : 0u;
     const bool lean = (lean_kw == 8 || lean_kw == 4) && (!ppay.data || ppay.width == 8) &&
-                      (!bpay.data || bpay.width == 8) && wout_h == wout_t && (wout_h == 8 || wout_h == 4) && out_h.data && out_t.data &&
-                      (out_h.cap < out_t.cap ? out_h.cap : out_t.cap) >= np;
-    // the streaming probe's tables follow the build's
-    size_t need = o_end + map_scratch_bytes<ProbeMapOp>(np);
-    if (need < o_end + align_up(nb * 4, 256)) need = o_end + align_up(nb * 4, 256);  // long-list merge scratch
-    if (lean) {
-        lean_shape(lean_kw, !ppay.data, !bpay.data, [&](auto proto) {
-            const size_t b = o_end + map_scratch_bytes<decltype(proto)>(np);
-            if (b > need) need = b;
-        });
-    }
-    if ((st = ws_ensure(ws, need)) != AHEAD_OK) return st;
+                      (!bpay.data || bpay.width == 8) && wout_h == wout_t && (wout_h == 8 || wout_h == 4);
+    if ((st = ws_ensure(ws, o_end + align_up(nb * 4, 256))) != AHEAD_OK) return st;  // + long-list merge scratch
 
     HjTable t{};
     t.flags = reinterpret_cast<uint32_t *>(ws_region(ws, o_flags));
@@ -813,7 +829,7 @@ extern "C" int ahead_hip_hashjoin_an(const ahead_col *h1, const ahead_col *t1, c
     off.t = t;
     if ((st = launch_rowtile(off, slots, 1, ws, s)) != AHEAD_OK) return st;
     hipLaunchKernelGGL(k_hj_fill, grid, dim3(kBlock), 0, s, b);
-    // the merge scratch of long row lists shares the probe's scratch region (the build is done first)
+    // the merge scratch of long row lists follows the tables
     hipLaunchKernelGGL(k_hj_sort, dim3(1024), dim3(kBlock), 0, s, t, static_cast<uint32_t>(slots),
                        reinterpret_cast<uint32_t *>(ws_region(ws, o_end)));
     AHEAD_HIP_TRY(hipGetLastError());
@@ -867,27 +883,26 @@ extern "C" int ahead_hip_hashjoin_an(const ahead_col *h1, const ahead_col *t1, c
     p.counts = d_counts;
     p.e_index[0] = right ? 1 : 3;
     p.e_index[1] = right ? 2 : 4;
-    // the streaming engine needs room for a staged pair per probe row
-    const bool map_ok = out_h.data && out_t.data && p.out_cap >= np;
     if (lean) {
         int lst = AHEAD_OK;
-        // the variant with the filter exists for 8-byte keys: the sample picks between the two
-        const bool pair = lean_kw == 8;
-        if (pair) {  // the sample, then the filter (built only when the sample found a missing key)
+        const bool filter = lean_kw == 8;
+        if (filter) {  // the sample, then the filter (built only when the sample found a missing key)
             hipLaunchKernelGGL(k_hj_sample, dim3(kHjSamples / kBlock), dim3(kBlock), 0, s, p, np);
             hipLaunchKernelGGL(k_hj_filter, grid, dim3(kBlock), 0, s, b);
         }
-        lean_shape(lean_kw, !ppay.data, !bpay.data, [&](auto proto) {
-            if (lst != AHEAD_OK) return;
-            auto q = proto;
-            q.pair_launched = pair ? 1u : 0u;
+        lean_shape(lean_kw, !ppay.data, !bpay.data, wout_h, [&](auto q) {
+            using Q = decltype(q);
             q.n = np;
             q.t = t;
-            q.key = static_cast<const typename decltype(q)::KT *>(pkey.data);
+            q.key = static_cast<const typename Q::KT *>(pkey.data);
             q.key_enc = p.key.encoded;
             q.key_inv = p.key.a_inv;
             q.key_cmask = p.key.mask;
             q.key_maxu = p.key.max_u;
+            // 32-bit arithmetic: encoded 8-byte codes whose guard and key take the low 32 bits
+            q.key_back = lean_kw == 8 && p.key.encoded && p.guard_mask <= 0xFFFFFFFFull && p.key_mask <= 0xFFFFFFFFull
+                             ? back_factor(p.key.a_inv, p.key.max_u)
+                             : 0u;
             q.key_err = right ? 1u : 0u;
             q.pay = static_cast<const uint64_t *>(ppay.data);
             q.pay_seq = ppay.seqbase;
@@ -899,15 +914,10 @@ extern "C" int ahead_hip_hashjoin_an(const ahead_col *h1, const ahead_col *t1, c
             q.guard_mask = p.guard_mask;
             q.key_mask = p.key_mask;
             q.build_max = p.build_max;
-            q.reenc_p = p.reenc_p;
-            q.reenc_b = p.reenc_b;
-            q.f_p = p.f_p;
-            q.f_b = p.f_b;
-            q.out_h = out_h.data;
-            q.out_t = out_t.data;
-            q.out_p = right ? out_h.data : out_t.data;
-            q.out_b = right ? out_t.data : out_h.data;
-            q.ow = wout_h;
+            q.f_p = p.reenc_p ? p.f_p : 1ull;
+            q.f_b = p.reenc_b ? p.f_b : 1ull;
+            q.out_p = static_cast<typename Q::OT *>(right ? out_h.data : out_t.data);
+            q.out_b = static_cast<typename Q::OT *>(right ? out_t.data : out_h.data);
             q.out_cap = p.out_cap;
             q.a_oid = a_oid;
             q.err[0] = p.err[0];
@@ -917,17 +927,13 @@ extern "C" int ahead_hip_hashjoin_an(const ahead_col *h1, const ahead_col *t1, c
             q.counts = d_counts;
             q.e_index[0] = p.e_index[0];
             q.e_index[1] = p.e_index[1];
-            lst = launch_map(q, ws, o_end, s);
+            lst = launch_stream(q, ws, s, filter ? kHjFiltWords * 8 : 0);
         });
         if (lst != AHEAD_OK) return lst;
-        p.map_launched = 1u;
-        p.lean = 1u;
-    } else if (map_ok) {
-        hipLaunchKernelGGL(k_hj_sample, dim3(kHjSamples / kBlock), dim3(kBlock), 0, s, p, np);
-        ProbeMapOp pm{};
-        static_cast<ProbeOp &>(pm) = p;
-        if ((st = launch_map(pm, ws, o_end, s)) != AHEAD_OK) return st;
-        p.map_launched = 1u;
+    } else {
+        ProbeOneOp one{};
+        static_cast<ProbeOp &>(one) = p;
+        if ((st = launch_stream(StreamRows<ProbeOneOp>(one), ws, s)) != AHEAD_OK) return st;
     }
     if ((st = launch_rowtile(p, np, 3, ws, s)) != AHEAD_OK) return st;
     hipLaunchKernelGGL(k_hj_status, dim3(1), dim3(1), 0, s, t.flags, d_counts);

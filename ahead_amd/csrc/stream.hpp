@@ -15,7 +15,8 @@
 //    and the inclusive prefix just before them; with one workgroup per CU that prefix belongs to a
 //    tile of an earlier generation and is there (170 us).  Windows of 256, 512 and 1024 tiles
 //    measured alike; 512 covers two tickets per CU.
-//  - the next tile's loads go out between this tile's publication and its polls (128 us).  Earlier is
+//  - the next tile's loads go out between this tile's publication and its polls (128 us).  Half of them
+//    behind the polls took 150 us.  Earlier is
 //    worse: a count published behind loads in flight reaches the other workgroups after them (loads
 //    issued before the publication 172 us; a wave of its own for the places, with the other fifteen
 //    always loading, 209 us).
@@ -29,18 +30,19 @@
 // is running, and a tile waits for lower tickets only, so the chain always drains.
 //
 // Op interface (beside eval / emit_err / finish of rowtile.hpp, which the rare error rows use):
-//   static constexpr int kErr, kG;      // error streams; rows per lane (at most 32)
+//   static constexpr int kErr, kG;      // error streams; rows per lane (even, at most 32)
 //   struct Raw; using State;            // a row's streamed inputs; what its entry needs
 //   uint64_t out_cap;                   // entries the outputs hold
+//   struct Uniform; Uniform begin(const char *lds) const;      // read once per workgroup, after init
 //   void load(uint64_t first, uint32_t k, Raw &) const;        // row first + k
-//   template <int G> void open_tile(const char *lds, uint64_t first, uint32_t lane,
-//            const Raw (&)[G], Mid<G> &) const;
-//       // rows first + 64 g + lane: decodes them and issues their lookups (a row past the end has
-//       // the last row's inputs)
-//   template <int G> void close_tile(const Mid<G> &, uint32_t live, State (&)[G], uint32_t &keep,
-//            uint32_t (&err)[kErr]) const;
+//   template <int G> void open_tile(const char *lds, const Uniform &, uint64_t first, uint32_t lane,
+//            uint32_t live, const Raw (&)[G], Mid<G> &) const;
+//       // rows first + 64 g + lane: decodes them and issues their lookups (bit g of live: the row
+//       // exists; one past the end has the last row's inputs)
+//   template <int G> void close_tile(const Uniform &, const Mid<G> &, uint32_t live, State (&)[G],
+//            uint32_t &keep, uint32_t (&err)[kErr]) const;
 //       // sets bit g of keep / err[e] for live rows that emit an entry / report into stream e
-//   void emit(const State &, uint64_t first, uint64_t pos, uint32_t row, uint32_t k) const;
+//   void emit(const Uniform &, const State &, uint64_t first, uint64_t pos, uint32_t row, uint32_t k) const;
 //       // entry pos + k, of row first + row (first and pos are wave-uniform: scalar bases)
 //   void report(uint64_t row, State &, uint32_t &errs) const;  // the error streams of one row
 //   void init(char *lds) const;         // all threads, before the first tile; a barrier follows
@@ -100,14 +102,14 @@ __device__ __forceinline__ uint32_t wave_rank(uint64_t ballot) {
 
 // The streamed inputs of a lane's G rows first + 64 g + lane, of which the wave has `left`; rows past
 // the end repeat the last one (a wave past the end: row 0).
-template <class Op, int G>
-__device__ __forceinline__ void stream_load(const Op &op, uint64_t first, uint32_t lane, uint32_t left,
-                                            typename Op::Raw (&raw)[G]) {
+template <class Op, int H>
+__device__ __forceinline__ void stream_load(const Op &op, uint64_t first, uint32_t lane, uint32_t left, int half,
+                                            typename Op::Raw (&raw)[H]) {
     const uint64_t base = left != 0u ? first : 0ull;
     const uint32_t top = left != 0u ? left - 1u : 0u;
 #pragma unroll
-    for (int g = 0; g < G; ++g) {
-        const uint32_t k = static_cast<uint32_t>(g * 64) + lane;
+    for (int g = 0; g < H; ++g) {
+        const uint32_t k = static_cast<uint32_t>((half * H + g) * 64) + lane;
         op.load(base, k < top ? k : top, raw[g]);
     }
 }
@@ -136,25 +138,40 @@ __global__ __launch_bounds__(kStreamThreads) void k_stream(Op op, StreamArgs m) 
         const uint64_t first = first_of(t);
         return first >= op.n ? 0u : op.n - first < kWaveRows ? static_cast<uint32_t>(op.n - first) : kWaveRows;
     };
-    typename Op::Raw raw[G];
-    if (tile < m.tiles && op.n != 0) stream_load<Op, G>(op, first_of(tile), lane, left_of(tile), raw);
+    constexpr int H = G / 2;
+    typename Op::Raw raw0[H], raw1[H];
+    const typename Op::Uniform uni = op.begin(s_op);
+    if (tile < m.tiles && op.n != 0) {
+        stream_load<Op, H>(op, first_of(tile), lane, left_of(tile), 0, raw0);
+        stream_load<Op, H>(op, first_of(tile), lane, left_of(tile), 1, raw1);
+    }
     while (tile < m.tiles) {
         unsigned long long ticket;  // the next tile's, taken by thread 0 while the inputs arrive
         if (threadIdx.x == 0) ticket = atomicAdd(m.te, 1ull);
         const uint64_t first = first_of(tile);
         const uint32_t left = left_of(tile);
-        typename Op::State st[G];
+        typename Op::State st0[H], st1[H];
         uint32_t keep = 0, err[Op::kErr] = {};
         if (left != 0u) {  // (a wave past the last row has nothing to look up: its columns may be empty)
-            typename Op::template Mid<G> mid;
             uint32_t live = kAll;  // rows of the lane that exist
             if (left != kWaveRows) {
                 live = 0;
 #pragma unroll
                 for (int g = 0; g < G; ++g) live |= (static_cast<uint32_t>(g * 64) + lane < left ? 1u : 0u) << g;
             }
-            op.template open_tile<G>(s_op, first, lane, raw, mid);
-            op.template close_tile<G>(mid, live, st, keep, err);
+            auto half = [&](int h, const typename Op::Raw (&raw)[H], typename Op::State (&st)[H]) {
+                constexpr uint32_t kHalf = (1u << H) - 1u;
+                const uint32_t on = (live >> (h * H)) & kHalf;
+                typename Op::template Mid<H> mid;
+                uint32_t kp = 0, er[Op::kErr] = {};
+                op.template open_tile<H>(s_op, uni, first + static_cast<uint32_t>(h * H * 64), lane, on, raw, mid);
+                op.template close_tile<H>(uni, mid, on, st, kp, er);
+                keep |= kp << (h * H);
+#pragma unroll
+                for (int e = 0; e < Op::kErr; ++e) err[e] |= er[e] << (h * H);
+            };
+            half(0, raw0, st0);
+            half(1, raw1, st1);
         }
 
         // what the wave keeps and reports
@@ -202,7 +219,10 @@ __global__ __launch_bounds__(kStreamThreads) void k_stream(Op op, StreamArgs m) 
             lb_store(&m.agg[tile], stream_word(epoch, (rep != 0u ? 1ull << 33 : 0ull) | agg[0]));
         }
         const uint32_t next = uniform(s_tile);
-        if (next < m.tiles) stream_load<Op, G>(op, first_of(next), lane, left_of(next), raw);
+        if (next < m.tiles) {
+            stream_load<Op, H>(op, first_of(next), lane, left_of(next), 0, raw0);
+            stream_load<Op, H>(op, first_of(next), lane, left_of(next), 1, raw1);
+        }
 
         // the counts of the kStreamWindow - 1 tiles before this one, and the prefix before them
         uint32_t sum[NS] = {};
@@ -248,7 +268,7 @@ __global__ __launch_bounds__(kStreamThreads) void k_stream(Op op, StreamArgs m) 
 #pragma unroll
             for (int g = 0; g < G; ++g) {
                 const uint32_t k = static_cast<uint32_t>(g * 64) + lane;
-                op.emit(st[g], first, pos, k, k);
+                op.emit(uni, g < H ? st0[g % H] : st1[g % H], first, pos, k, k);
             }
         } else if (kept != 0u) {
             uint32_t at = 0;
@@ -257,7 +277,8 @@ __global__ __launch_bounds__(kStreamThreads) void k_stream(Op op, StreamArgs m) 
                 const bool on = (keep >> g) & 1u;
                 const uint64_t b = __ballot(on);
                 const uint32_t k = at + wave_rank(b);
-                if (on && k < room) op.emit(st[g], first, pos, static_cast<uint32_t>(g * 64) + lane, k);
+                if (on && k < room)
+                    op.emit(uni, g < H ? st0[g % H] : st1[g % H], first, pos, static_cast<uint32_t>(g * 64) + lane, k);
                 at += static_cast<uint32_t>(__popcll(b));
             }
         }
@@ -288,6 +309,68 @@ __global__ __launch_bounds__(kStreamThreads) void k_stream(Op op, StreamArgs m) 
         tile = next;
     }
 }
+
+// An operator of the row-tile interface (at most one entry per row, eval_n) on this engine: the rows
+// are loaded when they are evaluated, not a tile ahead.
+template <class Op>
+struct StreamRows : Op {
+    static constexpr int kErr = Op::kErr, kG = 8;
+    struct Raw {};
+    using State = typename Op::State;
+    StreamRows() = default;
+    explicit StreamRows(const Op &op) : Op(op) {}
+    __device__ bool skip() const {
+        if constexpr (has_skip<Op>::value) return Op::skip();
+        return false;
+    }
+    struct Uniform {};
+    __device__ void init(char *) const {}
+    __device__ Uniform begin(const char *) const { return Uniform{}; }
+    __device__ __forceinline__ void load(uint64_t, uint32_t, Raw &) const {}
+    template <int G>
+    struct Mid {
+        State st[G];
+        uint32_t keep, err[kErr];
+    };
+    template <int G>
+    __device__ __forceinline__ void open_tile(const char *, const Uniform &, uint64_t first, uint32_t lane, uint32_t live,
+                                              const Raw (&)[G], Mid<G> &mid) const {
+        uint64_t rows[G], acc = 0;
+        bool on[G];
+        uint32_t errs[G], cnt[G];
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            rows[g] = first + static_cast<uint32_t>(g * 64) + lane;
+            on[g] = (live >> g) & 1u;
+        }
+        Op::template eval_n<G>(rows, on, mid.st, errs, cnt, acc);
+        mid.keep = 0;
+#pragma unroll
+        for (int e = 0; e < kErr; ++e) mid.err[e] = 0;
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            mid.keep |= (cnt[g] != 0u ? 1u : 0u) << g;
+#pragma unroll
+            for (int e = 0; e < kErr; ++e) mid.err[e] |= ((errs[g] >> e) & 1u) << g;
+        }
+    }
+    template <int G>
+    __device__ __forceinline__ void close_tile(const Uniform &, const Mid<G> &mid, uint32_t live, State (&st)[G], uint32_t &keep,
+                                               uint32_t (&err)[kErr]) const {
+#pragma unroll
+        for (int g = 0; g < G; ++g) st[g] = mid.st[g];
+        keep = live & mid.keep;
+#pragma unroll
+        for (int e = 0; e < kErr; ++e) err[e] = live & mid.err[e];
+    }
+    __device__ void report(uint64_t row, State &st, uint32_t &errs) const {
+        uint64_t acc = 0;
+        (void)Op::eval(row, st, errs, acc);
+    }
+    __device__ __forceinline__ void emit(const Uniform &, const State &st, uint64_t first, uint64_t pos, uint32_t row, uint32_t k) const {
+        Op::emit_main(first + row, st, pos + k, 1u);
+    }
+};
 
 }  // namespace ahead_dev
 
@@ -328,5 +411,4 @@ int launch_stream(const Op &op, ahead_hip_ws *ws, hipStream_t s, size_t lds = 0)
     AHEAD_HIP_TRY(hipGetLastError());
     return AHEAD_OK;
 }
-
 }  // namespace ahead_host

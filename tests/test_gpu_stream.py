@@ -146,3 +146,82 @@ def test_fetch_tables(t, a, rows, n, span, bad, past):
         got = capi.fetchjoin_an(capi.Column.from_numpy(oids, resoid), capi.Column.from_numpy(col, meta), reenc, ar)
         for i, (x, y) in enumerate(zip(got, ref)):
             assert np.array_equal(np.asarray(x).astype(np.uint64), np.asarray(y).astype(np.uint64)), i
+
+
+RESOID = an.an_meta(an.RESOID, an.A_OID)
+KEY = an.an_meta(an.RESINT, 63877)
+
+
+def flipped(codes, count, rng):
+    hit = rng.choice(codes.size, min(count, codes.size), replace=False)
+    codes[hit] ^= np.uint64(1) << rng.integers(0, 64, hit.size).astype(np.uint64)
+    return codes
+
+
+def same(got, ref):
+    assert len(got) == len(ref)
+    for i, (x, y) in enumerate(zip(got, ref)):
+        assert np.array_equal(x, np.asarray(y).astype(x.dtype)), i  # (a 4-byte output keeps the low half)
+
+
+@pytest.mark.parametrize("n,build,step,share,payload,flips", [
+    # payload: "v" void, "c" 8-byte codes, "n" plain 2-byte values (no lean shape): probe then build side
+    (TILE - 1, 500, 1, 1.0, "vv", 0), (3 * TILE + 1, 20_000, 1, 1.0, "vv", 9), (2 * TILE + 63, 3000, 1, 0.2, "vc", 40),
+    (5 * TILE + 7, 3000, 3, 0.5, "vc", 5), (8 * 1024 * 3 + 5, 3000, 1, 0.6, "cv", 5), (40_001, 900, 1, 0.9, "cc", 30),
+    (70_003, 900, 5_000_011, 0.3, "cc", 9), (70_003, 5000, 700, 0.02, "vv", 3), (50_000, 800, 1, 0.7, "nc", 3),
+    (50_000, 800, 1, 0.7, "nn", 3), (9 * TILE + 2, 260_000, 2, 0.4, "vv", 77), (1, 1, 1, 1.0, "cc", 0),
+])
+@pytest.mark.parametrize("wide", [False, True])
+def test_hash_probe_shapes(n, build, step, share, payload, flips, wide):
+    """The probe of unique keys: identity, direct map and hash table, exact and hashed filter."""
+    rng = np.random.default_rng(n + build)
+    keys = (7 + step * np.arange(build, dtype=np.uint64)) & np.uint64(0xFFFFFFFF)
+    if step != 1:
+        rng.shuffle(keys)
+    fk = np.where(rng.random(n) < share, keys[rng.integers(0, build, n)],
+                  (int(keys.max()) + 1 + rng.integers(0, 1000, n)).astype(np.uint64) & np.uint64(0xFFFFFFFF))
+    with np.errstate(over="ignore"):
+        fk_codes, key_codes = flipped(fk * np.uint64(KEY.a), flips, rng), keys * np.uint64(KEY.a)
+        oid = lambda k: flipped(rng.integers(0, 1 << 31, k).astype(np.uint64) * np.uint64(RESOID.a), 2, rng)  # noqa: E731
+
+    def side(kind, k):
+        if kind == "v":
+            return O.void(k), capi.Column.void(k)
+        arr, meta = ((oid(k), RESOID) if kind == "c" else
+                     (rng.integers(0, 1 << 16, k).astype(np.uint16), an.plain_meta(an.SHORTINT)))
+        return O.Col(arr, meta), capi.Column.from_numpy(arr, meta)
+    (oh, gh), (ot, gt) = side(payload[0], n), side(payload[1], build)
+    w = 8 if wide else 4
+    re = (1, 13) if wide else (0, 0)
+    print(f"probe n={n} build={build} step={step} share={share} {payload} w={w}", flush=True)
+    ref = O.hashjoin_an(oh, O.Col(fk_codes, KEY), O.Col(key_codes, KEY), ot, 1, *re, w, *re, w)
+    for cap in (None, max(1, len(ref[0]) // 2)):
+        same(capi.hashjoin_an(gh, capi.Column.from_numpy(fk_codes, KEY), capi.Column.from_numpy(key_codes, KEY), gt, 1,
+                              *re, w, *re, w, out_cap=cap), ref)
+
+
+@pytest.mark.parametrize("head", ["void", "same", "codes", "plain"])
+@pytest.mark.parametrize("t", [an.RESTINY, an.RESSHORT, an.RESINT, an.INT])
+@pytest.mark.parametrize("n,rows,flips", [(0, 5, 0), (1, 1, 0), (8191, 300, 3), (8193, 40_000, 0), (100_001, 5000, 600),
+                                          (5, 0, 0)])
+def test_match_positional_shapes(head, t, n, rows, flips):
+    rng = np.random.default_rng(n + rows + t.width)
+    meta = an.an_meta(t, 233) if t.encoded else an.plain_meta(t)
+    v = rng.integers(0, 1 << t.unenc_bits, rows).astype(np.uint64)
+    col = datagen.encode(v, 233, t.width) if t.encoded else v.astype(f"u{t.width}")
+    if rows > 20:
+        col[17] ^= np.asarray(8, dtype=col.dtype)
+    with np.errstate(over="ignore"):
+        oids = flipped(rng.integers(0, max(1, rows) + 3, n).astype(np.uint64) * np.uint64(RESOID.a), flips, rng)
+        other = flipped(rng.integers(0, 1 << 32, n).astype(np.uint64) * np.uint64(KEY.a), flips, rng)
+    g_oids, g_col = capi.Column.from_numpy(oids, RESOID), capi.Column.from_numpy(col, meta)
+    plain = rng.integers(0, 1 << 16, n).astype(np.uint16)
+    oh, gh, wh = {"void": (O.void(n, 3), capi.Column.void(n, 3), 4), "same": (O.Col(oids, RESOID), g_oids, 8),
+                  "codes": (O.Col(other, KEY), capi.Column.from_numpy(other, KEY), 8),
+                  "plain": (O.Col(plain, an.plain_meta(an.SHORTINT)),
+                            capi.Column.from_numpy(plain, an.plain_meta(an.SHORTINT)), 2)}[head]
+    for re in (0, 1):
+        rh, rt = (re if head in ("same", "codes") else 0), (re if t.encoded else 0)
+        args = (rh, 29 if rh else 0, wh, rt, 7 if rt else 0, t.width)
+        same(capi.matchjoin_pos_an(gh, g_oids, g_col, *args),
+             O.matchjoin_pos_an(oh, O.Col(oids, RESOID), O.Col(col, meta), *args))
