@@ -1,14 +1,16 @@
 // groupby_an.hip -- groupbyAN, unary and binary, for gfx950 (groupbyAN.tcc:51-94 and :99-165).
 //
 // Group ids are numbered by first occurrence in scan order:
-//  k_grp_first   every wave streams one contiguous range of rows, 8 or 16 consecutive rows per
-//                lane and batch (one vector load each), against a wave-private LDS set of the keys it
-//                has listed.  A key the wave has listed costs one LDS read.  A key new to the wave
-//                is listed with its row; the rows a wave visits only ascend, so that row is the
-//                key's first row in the range.  Every 64 listed keys (and at the end) the wave's
-//                lanes publish them to the HBM hash table (htable.hpp): a key's first row is the
-//                atomicMin (after a read) over the waves, and the lane that claims a key's slot
-//                appends the slot to the list of distinct keys.
+//  k_grp_first   (unary keys below 2^16) every wave streams one contiguous range of rows, consecutive
+//                rows per lane and batch (vector loads), against a wave-private bitmap of the keys it
+//                has listed.  A key new to the wave is listed with its row; the rows a wave visits
+//                only ascend, so that row is the key's first row in the range.  Every 64 listed keys
+//                (and at the end) the wave's lanes publish them to the HBM hash table (htable.hpp): a
+//                key's first row is the atomicMin (after a read) over the waves, and the lane that
+//                claims a key's slot appends the slot to the list of distinct keys.
+//  k_grp_first_set (other keys) every workgroup streams one contiguous range of rows against an LDS
+//                hash set of its keys with their first rows, which all lanes extend at once; it
+//                publishes the set at the end.
 //  k_grp_sort    (up to kGrpFastMax distinct keys) one workgroup orders the listed slots by first
 //                row: the position of a key is its group id.  It writes VGIDtoROID, the slot ->
 //                group-id map and a compact dictionary (key, RGID, first row) in group order.
@@ -32,9 +34,11 @@ constexpr uint32_t kGrpFastMax = 8192;      // distinct keys the one-workgroup o
 constexpr uint32_t kDictMax = 512;          // groups the LDS dictionary of AssignOp takes
 constexpr uint32_t kDictBits = 10;
 constexpr uint32_t kDictSlots = 1u << kDictBits;  // at most half full; slot kDictSlots: the all-ones key
-constexpr uint32_t kGfBits = 10;
-constexpr uint32_t kGfSlots = 1u << kGfBits;  // per-wave key set of k_grp_first (key + 1, 0 = free)
-constexpr uint32_t kGfFill = kGfSlots / 2;    // keys in the set before it is cleared
+constexpr uint32_t kGsBits = 11;
+constexpr uint32_t kGsSlots = 1u << kGsBits;  // key set of a k_grp_first_set workgroup (key + 1, 0 = free)
+constexpr uint32_t kGsFill = kGsSlots / 4 * 3;  // keys it takes; rows of further keys go to the HBM table
+constexpr uint64_t kGsRows = 8192;            // rows of a workgroup, at least (its set costs 3 us)
+constexpr uint32_t kGsPerCu = 3;              // workgroups per CU (of 256): each publishes every key it met
 constexpr uint32_t kGfDirectWords = 2048;     // bitmap set of unary keys below 2^16 (one bit a key)
 constexpr uint32_t kDirectKeys = 1024;        // AssignOp's LDS table indexed by the key: keys below 2^10
 // flags: [0] table overflow, [8] distinct keys claimed, [9] more than kGrpFastMax (compaction path)
@@ -142,17 +146,15 @@ struct Run {
     }
 };
 
-// Key word of the per-wave set: 32 bits for unary keys of codes up to 4 bytes.  Runs: 64 bytes of
-// codes per lane (at most 32 rows), 8 rows where a row brings 8 bytes or more.
-template <class T, bool BIN>
+// Runs of k_grp_first: 64 bytes of codes per lane (at most 32 rows).
+template <class T>
 struct GfTraits {
-    using K = std::conditional_t<(!BIN && sizeof(T) <= 4), uint32_t, uint64_t>;
-    static constexpr int R = (BIN || sizeof(T) == 8) ? 8 : (sizeof(T) == 4 ? 16 : 32);
+    static constexpr int R = sizeof(T) == 4 ? 16 : 32;
 };
 
-__device__ __forceinline__ uint32_t gf_slot(uint64_t key) {
+__device__ __forceinline__ uint32_t gs_slot(uint64_t key) {
     const uint32_t x = static_cast<uint32_t>(key) ^ static_cast<uint32_t>(key >> 32);
-    return (x * 0x9E3779B1u) >> (32 - kGfBits);
+    return (x * 0x9E3779B1u) >> (32 - kGsBits);
 }
 
 __device__ __forceinline__ uint32_t dict_slot(uint64_t key) {
@@ -186,118 +188,67 @@ __device__ __forceinline__ void grp_publish(const GrpTable &t, uint32_t *flags, 
     if (t.first[gs] > row) atomicMin(&t.first[gs], row);
 }
 
-// DIRECT (unary keys below 2^16): the wave's set is a bitmap over every key, so a row costs one
-// LDS read and a bit test, and the set never fills.
-template <class T, bool BIN, bool DIRECT>
+// Unary keys below 2^16: the wave's set is a bitmap over every key, so a row costs one LDS read and a
+// bit test, and the set never fills.
+template <class T>
 __global__ __launch_bounds__(kBlock) void k_grp_first(GrpKey k, GrpTable t, uint32_t *flags, uint32_t *list, uint64_t n,
                                                       uint64_t per_wave, uint32_t vec) {
-    using K = typename GfTraits<T, BIN>::K;
-    constexpr int R = GfTraits<T, BIN>::R;
-    static_assert(!DIRECT || sizeof(K) == 4, "direct sets take 32-bit keys");
-    constexpr K kOnes = static_cast<K>(~static_cast<K>(0));  // the key whose key + 1 is 0 (free)
-    constexpr uint32_t kWords = DIRECT ? kGfDirectWords : kGfSlots;
-    __shared__ K s_set[kWaves * kWords];
+    constexpr int R = GfTraits<T>::R;
+    constexpr uint32_t kWords = kGfDirectWords;
+    __shared__ uint32_t s_set[kWaves * kWords];
     const uint32_t lane = threadIdx.x & 63u;
-    K *set = s_set + (threadIdx.x >> 6) * kWords;
+    uint32_t *set = s_set + (threadIdx.x >> 6) * kWords;
     for (uint32_t i = lane; i < kWords; i += 64u) set[i] = 0;
     const uint64_t gw = static_cast<uint64_t>(blockIdx.x) * kWaves + (threadIdx.x >> 6);
     const uint64_t begin = gw * per_wave;
     const uint64_t end = begin + per_wave < n ? begin + per_wave : n;
     const T *tail = static_cast<const T *>(k.tail.data);
-    const uint64_t *grp = static_cast<const uint64_t *>(k.grp.data);
     constexpr uint64_t kStep = 64u * R;
-    // unary keys of codes up to 4 bytes: key = code * ka & km (ka = 1 for plain codes)
+    // key = code * ka & km (ka = 1 for plain codes)
     const uint32_t ka = k.tail.encoded ? static_cast<uint32_t>(k.tail.a_inv) : 1u;
     const uint32_t km = (k.tail.encoded ? static_cast<uint32_t>(k.tail.mask) : ~0u) & static_cast<uint32_t>(k.tail_mask);
-    uint32_t fill = 0, listed = 0;  // wave-uniform
-    bool ones = false;              // wave-uniform: kOnes is listed
-    K my_key = 0;                   // lane i holds the wave's i-th listed key and its first row
+    uint32_t listed = 0;  // wave-uniform
+    uint32_t my_key = 0;  // lane i holds the wave's i-th listed key and its first row
     uint32_t my_row = 0;
-    auto keys_of = [&](const Run<T, R> &c, const Run<uint64_t, R> &g, K (&key)[R]) {
+    auto keys_of = [&](const Run<T, R> &c, uint32_t (&key)[R]) {
 #pragma unroll
         for (int j = 0; j < R; ++j) {
-            if constexpr (!BIN && sizeof(T) <= 2) {  // both factors below 2^16: the 24-bit multiply is exact
-                key[j] = static_cast<K>(__umul24(static_cast<uint32_t>(c.get(j)), ka) & km);
-            } else if constexpr (!BIN && sizeof(T) == 4) {
-                key[j] = static_cast<K>((static_cast<uint32_t>(c.get(j)) * ka) & km);
-            } else if constexpr (BIN) {
-                key[j] = static_cast<K>(k.key_t<T, BIN>(c.get(j), g.get(j)));
+            if constexpr (sizeof(T) <= 2) {  // both factors below 2^16: the 24-bit multiply is exact
+                key[j] = __umul24(static_cast<uint32_t>(c.get(j)), ka) & km;
             } else {
-                key[j] = static_cast<K>(k.key_t<T, BIN>(c.get(j), 0ull));
+                key[j] = (static_cast<uint32_t>(c.get(j)) * ka) & km;
             }
         }
     };
     // one batch: the lanes' keys against the set, then the keys new to the wave
-    auto examine = [&](const K (&key)[R], uint64_t base, uint64_t r0) {
+    auto examine = [&](const uint32_t (&key)[R], uint64_t base, uint64_t r0) {
         // the common case first: a whole run whose keys the wave has all listed.  Every set word is
         // read before any is tested (no per-row branches); nothing of the keys outlives this test.
         bool all = r0 + R <= end;
-        if constexpr (DIRECT) {
+        {
             uint32_t w[R];
 #pragma unroll
-            for (int j = 0; j < R; ++j) w[j] = set[static_cast<uint32_t>(key[j]) >> 5];
+            for (int j = 0; j < R; ++j) w[j] = set[key[j] >> 5];
             uint32_t acc = 1u;  // bit 0 stays set while every key's bit is
 #pragma unroll
-            for (int j = 0; j < R; ++j) acc &= w[j] >> (static_cast<uint32_t>(key[j]) & 31u);
+            for (int j = 0; j < R; ++j) acc &= w[j] >> (key[j] & 31u);
             all = all && (acc & 1u) != 0u;
-        } else {
-            K w[R];
-#pragma unroll
-            for (int j = 0; j < R; ++j) w[j] = set[gf_slot(key[j])];
-#pragma unroll
-            for (int j = 0; j < R; ++j) all = all && (key[j] == kOnes ? ones : w[j] == static_cast<K>(key[j] + 1));
         }
         if (__ballot(!all) == 0ull) return;
         // exact pass: the batch's codes again (cached) and its keys; bit j: row r0 + j
-        K k2[R];
+        uint32_t k2[R];
         {
             Run<T, R> c;
-            Run<uint64_t, R> g;
-            if (vec != 0u && r0 + R <= end) {
-                c.load_vec(tail, r0);
-                if constexpr (BIN) g.load_vec(grp, r0);
-            } else {
-                c.load_elem(tail, r0, end);
-                if constexpr (BIN) g.load_elem(grp, r0, end);
-            }
-            keys_of(c, g, k2);
+            if (vec != 0u && r0 + R <= end) c.load_vec(tail, r0);
+            else c.load_elem(tail, r0, end);
+            keys_of(c, k2);
         }
         const uint32_t live = r0 >= end ? 0u : (end - r0 >= static_cast<uint64_t>(R) ? ~0u >> (32 - R)
                                                                                        : (1u << (end - r0)) - 1u);
-        uint32_t pend = 0, probe = 0;
-        if constexpr (DIRECT) {
+        uint32_t pend = 0;
 #pragma unroll
-            for (int j = 0; j < R; ++j) {
-                const uint32_t w = set[static_cast<uint32_t>(k2[j]) >> 5];
-                pend |= (~(w >> (static_cast<uint32_t>(k2[j]) & 31u)) & 1u) << j;
-            }
-        } else {
-#pragma unroll
-            for (int j = 0; j < R; ++j) {
-                const K w = set[gf_slot(k2[j])];
-                const bool hit = k2[j] == kOnes ? ones : w == static_cast<K>(k2[j] + 1);
-                pend |= static_cast<uint32_t>(!hit) << j;
-                probe |= static_cast<uint32_t>(k2[j] != kOnes && w != 0) << j;
-            }
-        }
+        for (int j = 0; j < R; ++j) pend |= (~(set[k2[j] >> 5] >> (k2[j] & 31u)) & 1u) << j;
         pend &= live;
-        probe &= pend;
-        if (__ballot(pend != 0u) == 0ull) return;
-        // keys stored past their home slot
-#pragma unroll
-        for (int j = 0; j < R; ++j) {
-            if (((probe >> j) & 1u) == 0u) continue;
-            uint32_t s = gf_slot(k2[j]);
-            for (uint32_t p = 1; p < kGfSlots; ++p) {
-                s = (s + 1u) & (kGfSlots - 1u);
-                const K w = set[s];
-                if (w == static_cast<K>(k2[j] + 1)) {
-                    pend &= ~(1u << j);
-                    break;
-                }
-                if (w == 0) break;
-            }
-        }
         // keys new to the wave, one per step: the lowest lane with a pending row holds the batch's
         // smallest pending row (lane l's rows all precede lane l + 1's), and a key is pending in
         // every row of the batch that holds it, so that row is the key's first in the batch.
@@ -306,36 +257,21 @@ __global__ __launch_bounds__(kBlock) void k_grp_first(GrpKey k, GrpTable t, uint
             if (m == 0ull) break;
             const uint32_t L = static_cast<uint32_t>(__builtin_ctzll(m));
             const uint32_t mj = pend != 0u ? static_cast<uint32_t>(__builtin_ctz(pend)) : 0u;
-            K mk = key[0];
+            uint32_t mk = k2[0];
 #pragma unroll
             for (int j = 1; j < R; ++j) mk = mj == static_cast<uint32_t>(j) ? k2[j] : mk;
-            const K k0 = readlane_k<K>(mk, L);
+            const uint32_t k0 = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(mk), L));
             const uint32_t row0 = static_cast<uint32_t>(base) + L * static_cast<uint32_t>(R) +
                                   static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(mj), L));
 #pragma unroll
             for (int j = 0; j < R; ++j) pend &= k2[j] == k0 ? ~(1u << j) : ~0u;
-            if constexpr (DIRECT) {
-                if (lane == 0) set[static_cast<uint32_t>(k0) >> 5] |= 1u << (static_cast<uint32_t>(k0) & 31u);
-            } else if (k0 == kOnes) {
-                ones = true;
-            } else {
-                if (fill == kGfFill) {  // the set is half full: start it again (keys may then be listed twice)
-                    for (uint32_t i = lane; i < kGfSlots; i += 64u) set[i] = 0;
-                    fill = 0;
-                }
-                if (lane == 0) {
-                    uint32_t s = gf_slot(k0);
-                    while (set[s] != 0) s = (s + 1u) & (kGfSlots - 1u);
-                    set[s] = static_cast<K>(k0 + 1);
-                }
-                ++fill;
-            }
+            if (lane == 0) set[k0 >> 5] |= 1u << (k0 & 31u);
             if (lane == listed) {
                 my_key = k0;
                 my_row = row0;
             }
             if (++listed == 64u) {
-                grp_publish(t, flags, list, static_cast<uint64_t>(my_key), my_row);
+                grp_publish(t, flags, list, my_key, my_row);
                 listed = 0;
             }
         }
@@ -346,29 +282,146 @@ __global__ __launch_bounds__(kBlock) void k_grp_first(GrpKey k, GrpTable t, uint
     // batch again), so that no path through the loop leaves a different set of loads in flight.
     const uint64_t nfull = (vec != 0u && end > begin) ? (end - begin) / kStep : 0u;
     Run<T, R> ca;
-    Run<uint64_t, R> ga;
-    if (nfull > 0) {
-        ca.load_vec(tail, rl);
-        if constexpr (BIN) ga.load_vec(grp, rl);
-    }
+    if (nfull > 0) ca.load_vec(tail, rl);
     uint64_t b = 0;
-    K key[R];
+    uint32_t key[R];
     for (; b < nfull; ++b) {
-        keys_of(ca, ga, key);
+        keys_of(ca, key);
         const uint64_t nb = b + 1 < nfull ? b + 1 : b;
         ca.load_vec(tail, rl + nb * kStep);
-        if constexpr (BIN) ga.load_vec(grp, rl + nb * kStep);
         examine(key, begin + b * kStep, rl + b * kStep);
     }
     // the last, partial batch (every batch of an unaligned column): element loads
     for (uint64_t base = begin + b * kStep; base < end; base += kStep) {
         const uint64_t r0 = base + static_cast<uint64_t>(lane) * R;
         ca.load_elem(tail, r0, end);
-        if constexpr (BIN) ga.load_elem(grp, r0, end);
-        keys_of(ca, ga, key);
+        keys_of(ca, key);
         examine(key, base, r0);
     }
-    if (lane < listed) grp_publish(t, flags, list, static_cast<uint64_t>(my_key), my_row);
+    if (lane < listed) grp_publish(t, flags, list, my_key, my_row);
+}
+
+// All other keys.  A workgroup's set holds key + 1 and the smallest row of every key it has met.  A row
+// reads its key's home slot and first row and is done when the key is there with an earlier row; the
+// few others (new keys, keys past their home slot, rows of a key's first batch) probe and insert with
+// LDS atomics, every lane for itself.  The set it replaced belonged to a wave, which listed its new
+// keys one after another: 35 keys in each of 8192 waves took longer than their rows.  12M binary keys,
+// 35 groups: 65 us before, 27 now (145 while the whole table was walked to publish it).
+template <class T, bool BIN>
+__global__ __launch_bounds__(kBlock) void k_grp_first_set(GrpKey k, GrpTable t, uint32_t *flags, uint32_t *list,
+                                                          uint64_t n, uint64_t per_block, uint32_t vec) {
+    constexpr int R = 8;
+    constexpr uint64_t kStep = static_cast<uint64_t>(kBlock) * R;
+    __shared__ unsigned long long s_key[kGsSlots + 1];  // [kGsSlots]: 1 when the all-ones key was met
+    __shared__ uint32_t s_first[kGsSlots + 1];
+    __shared__ uint16_t s_list[kGsSlots];            // the slots taken, in the order they were
+    __shared__ uint32_t s_fill;
+    for (uint32_t i = threadIdx.x; i <= kGsSlots; i += kBlock) {
+        s_key[i] = 0ull;
+        s_first[i] = 0xFFFFFFFFu;
+    }
+    if (threadIdx.x == 0) s_fill = 0u;
+    __syncthreads();
+    const uint64_t begin = static_cast<uint64_t>(blockIdx.x) * per_block;
+    const uint64_t end = begin + per_block < n ? begin + per_block : n;
+    const T *tail = static_cast<const T *>(k.tail.data);
+    const uint64_t *grp = static_cast<const uint64_t *>(k.grp.data);
+    const bool narrow = BIN && sizeof(T) <= 4 && k.lmask <= 0xFFFFFFFFull;  // keys modulo 2^32 or less
+    auto keys_of = [&](const Run<T, R> &c, const Run<uint64_t, R> &g, uint64_t (&key)[R]) {
+        if (narrow) {
+            const uint32_t lm = static_cast<uint32_t>(k.lmask), ng = static_cast<uint32_t>(k.num_groups),
+                           gi = static_cast<uint32_t>(k.grp.a_inv);
+#pragma unroll
+            for (int j = 0; j < R; ++j) {
+                const uint32_t tv = static_cast<uint32_t>(k.dec_t<T>(c.get(j)));
+                key[j] = (tv * ng + static_cast<uint32_t>(g.get(j)) * gi) & lm;
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < R; ++j) key[j] = k.key_t<T, BIN>(c.get(j), BIN ? g.get(j) : 0ull);
+        }
+    };
+    auto examine = [&](const uint64_t (&key)[R], uint64_t r0) {
+        const uint32_t live = r0 >= end ? 0u : (end - r0 >= static_cast<uint64_t>(R) ? (1u << R) - 1u
+                                                                                       : (1u << (end - r0)) - 1u);
+        const uint32_t row = static_cast<uint32_t>(r0);
+        uint32_t pend = 0;
+        {
+            unsigned long long w[R];
+            uint32_t f[R];
+#pragma unroll
+            for (int j = 0; j < R; ++j) {
+                const uint32_t s = key[j] == ~0ull ? kGsSlots : gs_slot(key[j]);
+                w[j] = s_key[s];
+                f[j] = s_first[s];
+            }
+#pragma unroll
+            for (int j = 0; j < R; ++j) {
+                const bool done = w[j] == (key[j] == ~0ull ? 1ull : key[j] + 1ull) && f[j] <= row + static_cast<uint32_t>(j);
+                pend |= (done ? 0u : 1u) << j;
+            }
+        }
+        pend &= live;
+        while (pend != 0u) {
+            const uint32_t j = static_cast<uint32_t>(__builtin_ctz(pend));
+            pend &= pend - 1u;
+            uint64_t kj = key[0];
+#pragma unroll
+            for (int i = 1; i < R; ++i) kj = j == static_cast<uint32_t>(i) ? key[i] : kj;
+            const unsigned long long word = kj == ~0ull ? 1ull : kj + 1ull;
+            uint32_t s = kj == ~0ull ? kGsSlots : gs_slot(kj);
+            bool in = false;
+            for (uint32_t p = 0; p < kGsSlots; ++p) {
+                unsigned long long w = s_key[s];
+                if (w == 0ull) {
+                    if (kj != ~0ull && s_fill >= kGsFill) break;  // the set takes no more keys
+                    w = atomicCAS(&s_key[s], 0ull, word);
+                    if (w == 0ull) {
+                        if (kj != ~0ull) s_list[atomicAdd(&s_fill, 1u)] = static_cast<uint16_t>(s);
+                        in = true;
+                        break;
+                    }
+                }
+                if (w == word) {
+                    in = true;
+                    break;
+                }
+                s = (s + 1u) & (kGsSlots - 1u);
+            }
+            if (!in) grp_publish(t, flags, list, kj, row + j);
+            else if (s_first[s] > row + j) atomicMin(&s_first[s], row + j);
+        }
+    };
+    const uint64_t rl = begin + static_cast<uint64_t>(threadIdx.x) * R;  // this thread's first row
+    const uint64_t nfull = (vec != 0u && end > begin) ? (end - begin) / kStep : 0u;
+    Run<T, R> ca;
+    Run<uint64_t, R> ga;
+    if (nfull > 0) {
+        ca.load_vec(tail, rl);
+        if constexpr (BIN) ga.load_vec(grp, rl);
+    }
+    uint64_t b = 0;
+    uint64_t key[R];
+    for (; b < nfull; ++b) {  // the next batch's loads go out as soon as this batch's keys are taken
+        keys_of(ca, ga, key);
+        const uint64_t nb = b + 1 < nfull ? b + 1 : b;
+        ca.load_vec(tail, rl + nb * kStep);
+        if constexpr (BIN) ga.load_vec(grp, rl + nb * kStep);
+        examine(key, rl + b * kStep);
+    }
+    for (uint64_t base = begin + b * kStep; base < end; base += kStep) {
+        const uint64_t r0 = base + static_cast<uint64_t>(threadIdx.x) * R;
+        ca.load_elem(tail, r0, end);
+        if constexpr (BIN) ga.load_elem(grp, r0, end);
+        keys_of(ca, ga, key);
+        examine(key, r0);
+    }
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < s_fill; i += kBlock) {
+        const uint32_t s = s_list[i];
+        grp_publish(t, flags, list, s_key[s] - 1ull, s_first[s]);
+    }
+    if (threadIdx.x == 0 && s_key[kGsSlots] != 0ull) grp_publish(t, flags, list, ~0ull, s_first[kGsSlots]);
 }
 
 struct GrpSortArgs {
@@ -739,28 +792,39 @@ struct GrpPlan {
     uint32_t vec;
 };
 
-// Persistent grid of k_grp_first: resident workgroups (LDS decides), ranges of whole batches.
+// Launches the first-sightings pass: a persistent grid of resident workgroups (LDS decides), ranges of
+// whole batches.
 template <class T, bool BIN, bool DIRECT>
-uint32_t first_grid(uint64_t n, uint64_t *per_wave) {
-    static uint32_t resident = 0;
-    if (resident == 0) {
+void launch_first(const GrpKey &k, const GrpTable &t, uint32_t *flags, uint32_t *list, uint64_t n, uint32_t vec,
+                  hipStream_t s) {
+    const void *fn;
+    if constexpr (DIRECT) fn = reinterpret_cast<const void *>(k_grp_first<T>);
+    else fn = reinterpret_cast<const void *>(k_grp_first_set<T, BIN>);
+    static const uint32_t resident = [fn] {
         int dev = 0, cus = 0, per_cu = 0;
         if (hipGetDevice(&dev) != hipSuccess ||
             hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
             cus = 256;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void *>(k_grp_first<T, BIN, DIRECT>),
-                                                         kBlock, 0) != hipSuccess ||
-            per_cu <= 0)
-            per_cu = 2;
-        resident = static_cast<uint32_t>(cus) * static_cast<uint32_t>(per_cu);
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, kBlock, 0) != hipSuccess || per_cu <= 0) per_cu = 2;
+        return static_cast<uint32_t>(cus) * static_cast<uint32_t>(per_cu);
+    }();
+    if constexpr (DIRECT) {
+        constexpr uint64_t step = 64u * GfTraits<T>::R;
+        const uint64_t batches = (n + step - 1) / step;
+        const uint64_t most = static_cast<uint64_t>(resident) * kWaves;
+        const uint64_t waves = batches < most ? (batches == 0 ? 1 : batches) : most;
+        const uint64_t per_wave = (batches + waves - 1) / waves * step;
+        hipLaunchKernelGGL(k_grp_first<T>, dim3(static_cast<uint32_t>((waves + kWaves - 1) / kWaves)), dim3(kBlock), 0, s,
+                           k, t, flags, list, n, per_wave, vec);
+    } else {
+        const uint32_t most = resident < 256u * kGsPerCu ? resident : 256u * kGsPerCu;
+        uint64_t per_block = (n + most - 1) / most;
+        if (per_block < kGsRows) per_block = kGsRows;
+        per_block = (per_block + kBlock * 8 - 1) / (kBlock * 8) * (kBlock * 8);
+        const uint32_t grid = static_cast<uint32_t>((n + per_block - 1) / per_block);
+        hipLaunchKernelGGL((k_grp_first_set<T, BIN>), dim3(grid), dim3(kBlock), 0, s, k, t, flags, list, n, per_block,
+                           vec);
     }
-    constexpr uint64_t step = 64u * GfTraits<T, BIN>::R;
-    const uint64_t batches = (n + step - 1) / step;
-    const uint64_t waves_max = static_cast<uint64_t>(resident) * kWaves;
-    const uint64_t waves = batches < waves_max ? (batches == 0 ? 1 : batches) : waves_max;
-    *per_wave = (batches + waves - 1) / waves * step;
-    const uint64_t g = (waves + kWaves - 1) / kWaves;
-    return static_cast<uint32_t>(g);
 }
 
 // D1: k_grp_first's direct bitmap; D2: AssignOp's direct table
@@ -788,10 +852,7 @@ int run_typed(GrpPlan p) {
         AHEAD_HIP_TRY(hipGetLastError());
     }
     if (p.n) {
-        uint64_t per_wave = 0;
-        const uint32_t grid = first_grid<T, BIN, D1>(p.n, &per_wave);
-        hipLaunchKernelGGL((k_grp_first<T, BIN, D1>), dim3(grid), dim3(kBlock), 0, p.s, p.k, p.t, p.flags, p.list, p.n,
-                           per_wave, p.vec);
+        launch_first<T, BIN, D1>(p.k, p.t, p.flags, p.list, p.n, p.vec, p.s);
         AHEAD_HIP_TRY(hipGetLastError());
     }
     GrpSortArgs ga{};

@@ -797,14 +797,17 @@ __global__ __launch_bounds__(kBlock) void k_mulsum_final(const uint64_t *partial
 }
 
 // ---------------------------------------------------------------------------------------------------
-// Grouped sum: LDS-private accumulators per workgroup when the groups fit, merged with 64-bit
-// atomics; otherwise straight 64-bit atomics on the output.
-constexpr uint32_t kAggLds = 2048;
+// Grouped sum: LDS-private accumulators per workgroup when the groups fit, then one partial per group and
+// workgroup and a reduction; otherwise straight 64-bit atomics on the output.
+constexpr uint32_t kAggLds = 4096;  // 64-bit words
 
 struct AggSumArgs {
     uint64_t n;
     DCol head, tail, grp;
     uint64_t num_groups, enc, a_oid;
+    uint32_t grp_back, tail_back;  // the codes' A where 32-bit arithmetic decodes them (back_factor), else 0
+    uint32_t copies;               // accumulators per group in LDS (a power of two; 0: none)
+    uint64_t *partials;            // [num_groups][workgroups] (copies != 0)
     uint64_t *sums;
     uint64_t *err[3];
     uint64_t cap[3];
@@ -812,9 +815,13 @@ struct AggSumArgs {
 };
 
 struct AggSumOp {
-    // checks and sums in one pass: per-workgroup LDS sums when the groups fit (merged into the
-    // output with 64-bit atomics at the end), else 64-bit atomics on the output directly
+    // Checks and sums in one pass.  Few groups make the lanes of a wave meet on the same LDS word, and
+    // same-word atomics run one after another (12M rows into 35 groups: 71 us, 4.5 times what the two
+    // columns take to read).  So a group has up to 32 accumulators side by side, each lane adding to its
+    // own of them, and the workgroups leave partials: 12M rows 52 us.  The codes are summed as they
+    // are and multiplied by the re-encoding factor at the end (sums mod 2^64 are linear).
     static constexpr int kErr = 3;
+    static constexpr int kMapRows = 8;  // twice the loads in flight
     static constexpr int kSharedWords = kAggLds;
     static constexpr bool kMulti = false, kMain = false, kAcc = false;
     using State = uint8_t;
@@ -822,56 +829,70 @@ struct AggSumOp {
     uint64_t n;
     static constexpr bool kBatched = true;
     __device__ void shared_init(unsigned long long *s) const {
-        const uint32_t ng = a.num_groups <= kAggLds ? static_cast<uint32_t>(a.num_groups) : 0u;
-        for (uint32_t i = threadIdx.x; i < ng; i += blockDim.x) s[i] = 0ull;
+        const uint32_t nw = static_cast<uint32_t>(a.num_groups) * a.copies;
+        for (uint32_t i = threadIdx.x; i < nw; i += blockDim.x) s[i] = 0ull;
     }
     __device__ void shared_flush(unsigned long long *s) const {
-        if (a.num_groups > kAggLds) return;
-        for (uint32_t i = threadIdx.x; i < a.num_groups; i += blockDim.x)
-            if (s[i] != 0ull) atomicAdd(reinterpret_cast<unsigned long long *>(&a.sums[i]), s[i]);
+        if (a.copies == 0u) return;
+        for (uint32_t i = threadIdx.x; i < a.num_groups; i += blockDim.x) {
+            unsigned long long x = 0ull;
+            for (uint32_t c = 0; c < a.copies; ++c) x += s[i * a.copies + ((c + i) & (a.copies - 1u))];
+            a.partials[static_cast<size_t>(i) * gridDim.x + blockIdx.x] = x;
+        }
     }
     // aggregateAN.tcc:84-112: a corrupt tail is still added (and reported); a row whose group id
     // is corrupt or out of range is reported and skipped
     template <int G>
     __device__ void eval_shared(const uint64_t (&row)[G], const bool (&live)[G], State (&st)[G], uint32_t (&errs)[G],
                                 uint32_t (&cnt)[G], uint64_t &acc, unsigned long long *s) const {
-        uint64_t t[G], gr[G];
-        eval_rows<G>(row, live, errs, t, gr);
-        const bool lds = a.num_groups <= kAggLds;
+        uint64_t t[G], gi[G];
+        eval_rows<G>(row, live, errs, t, gi);
+        const uint32_t copy = threadIdx.x & (a.copies - 1u);
 #pragma unroll
         for (int g = 0; g < G; ++g) {
             cnt[g] = 0;
             if (!live[g] || (errs[g] & 4u)) continue;
-            const uint64_t gi = gr[g] * a.grp.a_inv;
-            const unsigned long long add = t[g] * a.enc;
-            if (lds) atomicAdd(&s[gi], add);
-            else atomicAdd(reinterpret_cast<unsigned long long *>(&a.sums[gi]), add);
+            if (a.copies != 0u) atomicAdd(&s[static_cast<uint32_t>(gi[g]) * a.copies + copy], static_cast<unsigned long long>(t[g]));
+            else atomicAdd(reinterpret_cast<unsigned long long *>(&a.sums[gi[g]]), static_cast<unsigned long long>(t[g] * a.enc));
         }
         (void)st;
         (void)acc;
     }
+    // error bits, tail codes and group ids of G rows
     template <int G>
     __device__ void eval_rows(const uint64_t (&row)[G], const bool (&live)[G], uint32_t (&errs)[G], uint64_t (&t)[G],
-                              uint64_t (&gr)[G]) const {
-        uint64_t h[G];
+                              uint64_t (&gi)[G]) const {
+        uint64_t h[G], gr[G];
         if (a.head.encoded) a.head.raw_n<G>(row, live, h);
         a.tail.raw_n<G>(row, live, t);
         a.grp.raw_n<G>(row, live, gr);
 #pragma unroll
         for (int g = 0; g < G; ++g) {
-            errs[g] = 0;
-            if (!live[g]) continue;
-            if (a.head.encoded && a.head.bad_of(h[g])) errs[g] |= 1u;
-            if (a.tail.bad_of(t[g])) errs[g] |= 2u;
-            const uint64_t gi = gr[g] * a.grp.a_inv;
-            if (gi > a.grp.max_u || gi >= a.num_groups) errs[g] |= 4u;
+            bool ok, bad;
+            if (a.grp_back != 0u) {
+                const uint32_t x = static_cast<uint32_t>(gr[g]) * static_cast<uint32_t>(a.grp.a_inv);
+                ok = x < a.num_groups && static_cast<uint64_t>(x) * a.grp_back == gr[g] && x <= a.grp.max_u;
+                gi[g] = x;
+            } else {
+                const uint64_t x = gr[g] * a.grp.a_inv;
+                ok = x <= a.grp.max_u && x < a.num_groups;
+                gi[g] = x;
+            }
+            if (a.tail_back != 0u) {
+                const uint32_t d = static_cast<uint32_t>(t[g]) * static_cast<uint32_t>(a.tail.a_inv);
+                bad = static_cast<uint64_t>(d) * a.tail_back != t[g] || d > a.tail.max_u;
+            } else {
+                bad = a.tail.bad_of(t[g]);
+            }
+            errs[g] = !live[g] ? 0u
+                               : (a.head.encoded && a.head.bad_of(h[g]) ? 1u : 0u) | (bad ? 2u : 0u) | (ok ? 0u : 4u);
         }
     }
     template <int G>
     __device__ void eval_n(const uint64_t (&row)[G], const bool (&live)[G], State (&)[G], uint32_t (&errs)[G],
                            uint32_t (&cnt)[G], uint64_t &) const {
-        uint64_t t[G], gr[G];
-        eval_rows<G>(row, live, errs, t, gr);
+        uint64_t t[G], gi[G];
+        eval_rows<G>(row, live, errs, t, gi);
 #pragma unroll
         for (int g = 0; g < G; ++g) cnt[g] = 0;
     }
@@ -893,6 +914,18 @@ struct AggSumOp {
     }
 };
 
+
+// The group's partials of all workgroups, re-encoded.  (Added to the output with atomics by every
+// workgroup, 1280 of them meeting on each group's word cost 20 us.)
+__global__ __launch_bounds__(kBlock) void k_aggsum_final(AggSumArgs a, uint32_t parts) {
+    __shared__ uint64_t s_red[kWaves];
+    for (uint64_t g = blockIdx.x; g < a.num_groups; g += gridDim.x) {
+        uint64_t x = 0;
+        for (uint32_t i = threadIdx.x; i < parts; i += kBlock) x += a.partials[g * parts + i];
+        x = block_sum<uint64_t>(x, s_red);
+        if (threadIdx.x == 0) a.sums[g] = x * a.enc;
+    }
+}
 
 __global__ void k_fill_u64(uint64_t *p, uint64_t n, uint64_t v) {
     const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
@@ -1075,6 +1108,13 @@ extern "C" int ahead_hip_aggregate_sum_grouped_an(const ahead_col *head, const a
     // aggregateAN.tcc:74-75: A_result * inv(A_tail) mod 2^64
     a.enc = a_result * (tail->encoded ? inverse_mod2k(tail->a, 64) : 1ull);
     a.a_oid = a_oid;
+    // (a group id in range is below 2^32 unless there are more groups than that)
+    a.grp_back = num_groups <= 0xFFFFFFFFull ? back_factor(grouping->a_inv, 0xFFFFFFFFull) : 0u;
+    a.tail_back = a.tail.encoded && a.tail.width == 8 ? back_factor(a.tail.a_inv, a.tail.max_u) : 0u;
+    if (num_groups && num_groups <= kAggLds) {
+        a.copies = 1;
+        while (a.copies < 32u && 2ull * a.copies * num_groups <= kAggLds) a.copies *= 2;
+    }
     a.sums = sums;
     const ahead_buf e[3] = {e_head, e_tail, e_group};
     for (int i = 0; i < 3; ++i) {
@@ -1083,12 +1123,24 @@ extern "C" int ahead_hip_aggregate_sum_grouped_an(const ahead_col *head, const a
     }
     a.d_counts = d_counts;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (num_groups) {
+    AggSumOp op{};
+    op.n = a.n;
+    size_t o_map = 0;
+    const uint32_t parts = map_waves<AggSumOp>(op.n) / kWaves;  // one partial per workgroup and group
+    if (a.copies != 0u) {
+        o_map = align_up(num_groups * parts * 8ull, 256);
+        if ((st = ws_ensure(ws, o_map + map_scratch_bytes<AggSumOp>(op.n))) != AHEAD_OK) return st;
+        a.partials = reinterpret_cast<uint64_t *>(ws_region(ws, 0));
+    } else if (num_groups) {
         hipLaunchKernelGGL(k_fill_u64, dim3(64), dim3(256), 0, s, sums, num_groups, 0ull);
         AHEAD_HIP_TRY(hipGetLastError());
     }
-    AggSumOp op{};
     op.a = a;
-    op.n = a.n;
-    return launch_map(op, ws, 0, s);
+    if ((st = launch_map(op, ws, o_map, s)) != AHEAD_OK) return st;
+    if (a.copies != 0u) {
+        hipLaunchKernelGGL(k_aggsum_final, dim3(static_cast<uint32_t>(num_groups < 1024 ? num_groups : 1024)), dim3(kBlock),
+                           0, s, a, parts);
+        AHEAD_HIP_TRY(hipGetLastError());
+    }
+    return AHEAD_OK;
 }

@@ -139,3 +139,29 @@ def test_groupby_dictionary_overflow_retry(card):
     got2 = capi.groupby2_an(capi.Column.void(n), gcol(codes, meta), gcol(ref[0], RESOID), ng,
                             an.RESSHORT.larger_bits, err_cap=4, table_bits=4)
     same(got2, ref2)
+
+
+@pytest.mark.parametrize("n,card", [(8191, 3), (8192, 1535), (8193, 1536), (20_000, 1537), (40_000, 2047), (70_001, 2600),
+                                    (2_000_003, 900)])
+def test_groupby_workgroup_set_edges(n, card):
+    """Row counts around a workgroup's least range, distinct keys around what its LDS set takes (1536 of
+    2048 slots; further keys go to the HBM table row by row), the all-ones key among them; and the
+    grouped sum over as many groups (LDS accumulators in 32 copies down to one, then none)."""
+    rng = np.random.default_rng(n + card)
+    vals = rng.integers(0, card, n).astype(np.uint64) * np.uint64(0x100000001) + np.uint64(5)
+    vals[rng.choice(n, 5, replace=False)] = ~np.uint64(0)
+    meta = an.plain_meta(an.BIGINT)
+    ref = O.groupby_an(O.void(n), O.Col(vals, meta))
+    same(capi.groupby_an(capi.Column.void(n), gcol(vals, meta), err_cap=2), ref)
+    small = (vals % np.uint64(251)).astype(np.uint8)
+    mt = an.plain_meta(an.TINYINT)
+    ng = ref[1].size
+    ref2 = O.groupby2_an(O.void(n), O.Col(small, mt), O.Col(ref[0], RESOID), ng, 64)
+    same(capi.groupby2_an(capi.Column.void(n), gcol(small, mt), gcol(ref[0], RESOID), ng, 64, err_cap=2), ref2)
+    m = datagen.encode(rng.integers(0, 1 << 32, n).astype(np.uint64), 65117, 8)
+    datagen.inject_flips(m, n, 2, datagen.flip_threshold(1e-3))
+    mm = an.an_meta(an.RESINT, 65117)
+    for g, k in ((ref[0], ng), (ref2[0], ref2[1].size), (ref[0], max(1, ng // 2))):
+        a = O.aggregate_sum_grouped_an(O.void(n), O.Col(m, mm), O.Col(g, RESOID), k)
+        b = capi.aggregate_sum_grouped_an(capi.Column.void(n), gcol(m, mm), gcol(g, RESOID), k)
+        same(b, a)
