@@ -29,7 +29,7 @@
 // every check holds the pieces are the reference's walk.  If any fails (the inputs are not sorted
 // in decoded value, e.g. a corrupted key), k_mm_gscan's first thread walks the whole input
 // instead: slower, same results.
-#include "rowtile.hpp"
+#include "stream.hpp"
 
 namespace {
 
@@ -69,8 +69,11 @@ struct MergeArgs {
     uint64_t prov_cap;
     uint32_t *flags;    // [0]: a piece of the walk disagreed with its successor's entry state
     uint64_t *d_counts;
-    const uint32_t *fast;  // nonzero: the intersection path wrote every output (the sub-tile kernels return)
+    const uint32_t *fast;  // [0] the intersection path ran, [1] its pass over list 1 found it does not apply
 };
+
+// The intersection path wrote every output: the sub-tile kernels return.
+__device__ __forceinline__ bool fast_path(const MergeArgs &a) { return a.fast[0] != 0u && a.fast[1] == 0u; }
 
 __device__ __forceinline__ uint64_t dec_at(const DCol &c, uint64_t i) { return c.dec_of(c.raw(i)); }
 
@@ -136,7 +139,7 @@ struct SplitArgs {
 };
 
 __global__ __launch_bounds__(kBlock) void k_mm_split(MergeArgs a, SplitArgs sp) {
-    if (*a.fast != 0u) return;
+    if (fast_path(a)) return;
     const uint64_t b = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     // the sub-tile kernels' flag and group sums start at zero
     if (b == 0) a.flags[0] = 0u;
@@ -624,7 +627,7 @@ __global__ __launch_bounds__(kMmThreads) void k_mm_count(MergeArgs a) {
     __shared__ uint16_t s_os[kMmDiag];  // local list-1 row of each output pair
     __shared__ uint64_t s_bound[kMmWaves];
     __shared__ uint32_t s_red[kMmWaves];
-    if (*a.fast != 0u) return;
+    if (fast_path(a)) return;
     const uint64_t sub = blockIdx.x;
     const uint32_t t = threadIdx.x;
     SubTile T;
@@ -707,7 +710,7 @@ __global__ __launch_bounds__(kMmThreads) void k_mm_count(MergeArgs a) {
 // Exclusive prefixes of the group sums, per stream (one block), and the totals.
 __global__ __launch_bounds__(kBlock) void k_mm_gscan(MergeArgs a) {
     __shared__ uint64_t s_red[kWaves];
-    if (*a.fast != 0u) return;
+    if (fast_path(a)) return;
     for (int s = 0; s < kMmStreams; ++s) {
         uint64_t *g = a.grp + s * a.num_grp;
         uint64_t carry = 0;
@@ -782,7 +785,7 @@ __global__ __launch_bounds__(kMmThreads) void k_mm_move(MergeArgs a) {
     __shared__ uint64_t s_red[kMmWaves];
     __shared__ uint32_t s_red32[kMmWaves];
     __shared__ uint64_t s_bound[kMmWaves];
-    if (a.flags[0] != 0u || *a.fast != 0u) return;  // the one-thread walk (or the intersection path) writes everything
+    if (a.flags[0] != 0u || fast_path(a)) return;  // the one-thread walk (or the intersection path) writes everything
     const uint32_t t = threadIdx.x, lane = t & 63u, wv = t >> 6;
     const uint64_t s0 = static_cast<uint64_t>(blockIdx.x) * kMmMoveSubs;
     const uint32_t nsub = static_cast<uint32_t>(a.num_sub - s0 < kMmMoveSubs ? a.num_sub - s0 : kMmMoveSubs);
@@ -848,28 +851,24 @@ __global__ __launch_bounds__(kMmThreads) void k_mm_move(MergeArgs a) {
 //              are gathered from t2, per 64-key word the list-2 row of its first key (the row of
 //              a key is that plus the set bits below it);
 //  k_mi_tails  the words the build waves share, ORed in;
-//  k_mi_count  per wave of list 1: the rows whose key is set;
-//  k_mi_scan   the waves' prefixes and the counts;
-//  k_mi_write  the pairs at the waves' prefixes.
-// The build and count passes check the conditions on every row they read (valid codes, each key
-// above the one before it); any failure clears the path's flag, the later passes return, and the
-// sub-tile kernels (which return while the flag is set) compute the outputs instead.
+//  IntersectOp on the single-pass engine (stream.hpp): the pairs of list 1's rows whose key is set.
+// Both passes check the conditions on every row they read (valid codes, each key above the one
+// before it); after a failure the sub-tile kernels, which otherwise return, write all outputs.
 constexpr uint64_t kMiBitsPerRow = 16;
-constexpr uint32_t kMiNone = 0xFFFFFFFFu;  // no bitmap word (words < 2^30)
+constexpr uint64_t kMiWordsMax = 1ull << 26;  // a key's bit number fits 32 bits: all 32-bit OIDs
+constexpr uint32_t kMiNone = 0xFFFFFFFFu;  // no bitmap word
 constexpr int kMiG = 4;  // rows per lane per step
 
 struct MiArgs {
-    uint32_t *ok;       // [0] nonzero while the path applies
+    uint32_t *ok;       // [0] nonzero while the path applies, [1] list 1 failed a check, [2] its keys need 64 bits
     uint64_t *range;    // [0] lo2, [1] bitmap words in use
     uint64_t *bits;     // [words_cap]
     uint32_t *first;    // [words_cap] list-2 row of the first key in each word that holds one
     uint64_t words_cap;
-    uint32_t *wcnt;     // [waves1] matches per wave of list 1
-    uint32_t *wpre;     // [waves1] their exclusive prefixes
     uint32_t *tail_w;   // [waves2] the last bitmap word of each build wave (kMiNone: none) ...
     uint64_t *tail_m;   // [waves2] ... and the wave's bits of it, ORed in by k_mi_tails
-    uint32_t waves1, waves2;
-    uint64_t per1, per2;  // rows per wave of list 1 / list 2 (multiples of 64 * kMiG)
+    uint32_t waves2;
+    uint64_t per2;      // rows per wave of list 2 (a multiple of 64 * kMiG)
 };
 
 // The key range of list 2 from its first and last codes (every thread of k_mi_clear computes it;
@@ -893,6 +892,8 @@ __global__ __launch_bounds__(kBlock) void k_mi_clear(MergeArgs a, MiArgs mi, uin
         mi.range[0] = lo;
         mi.range[1] = words;
         mi.ok[0] = ok;
+        mi.ok[1] = 0u;
+        mi.ok[2] = ok && a.t1.dec_of(a.t1.raw(a.n1 - 1)) > 0xFFFFFFFFull ? 1u : 0u;
     }
     const uint64_t stride = static_cast<uint64_t>(gridDim.x) * kBlock;
     for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * kBlock + threadIdx.x; i < words; i += stride) mi.bits[i] = 0ull;
@@ -1089,199 +1090,187 @@ __global__ __launch_bounds__(kBlock) void k_mi_tails(MergeArgs a, MiArgs mi) {
     if (w < mi.range[1]) atomicOr(reinterpret_cast<unsigned long long *>(mi.bits + w), static_cast<unsigned long long>(mi.tail_m[gw]));
 }
 
-// List 1, count pass: order and validity checks and, per wave, the rows whose key is set.  Each
-// lane takes kMiR consecutive rows of a step.
-template <typename K>
-__global__ __launch_bounds__(kBlock) void k_mi_count(MergeArgs a, MiArgs mi) {
-    if (mi.ok[0] == 0u) return;
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t gw = blockIdx.x * kWaves + (threadIdx.x >> 6);
-    if (gw >= mi.waves1) return;
-    const uint64_t begin = static_cast<uint64_t>(gw) * mi.per1;
-    const uint64_t end = begin < a.n1 ? mi_rows_end(begin, mi.per1, a.n1) : begin;
-    const uint64_t lo = mi.range[0], words = mi.range[1];
-    const bool chk_h1 = mi_own_check(a.h1, a.t1);  // h1's codes are checked too
-    bool bad = false;
-    bool has_prev = begin > 0 && begin < end;
-    uint64_t prev = has_prev ? a.t1.dec_of(a.t1.raw(begin - 1)) : 0ull;
-    uint32_t cnt = 0;
-    K cn[kMiR];
-    uint64_t chn[kMiR] = {};
-    {
-        uint64_t rows[kMiR];
-        bool live[kMiR];
-#pragma unroll
-        for (int k = 0; k < kMiR; ++k) {
-            rows[k] = begin + static_cast<uint64_t>(lane) * kMiR + k;
-            live[k] = rows[k] < end;
-        }
-        mi_load<K, kMiR>(a.t1.data, rows, live, cn);
-        if (chk_h1) a.h1.raw_n<kMiR>(rows, live, chn);
-    }
-    for (uint64_t seg = begin; seg < end; seg += 64u * kMiR) {
-        uint64_t rows[kMiR], c[kMiR], ch[kMiR], v[kMiR], word[kMiR];
-        bool live[kMiR], in[kMiR];
-#pragma unroll
-        for (int k = 0; k < kMiR; ++k) {
-            rows[k] = seg + static_cast<uint64_t>(lane) * kMiR + k;
-            live[k] = rows[k] < end;
-            c[k] = cn[k];
-            ch[k] = chn[k];
-        }
-        {  // the next step's codes, in flight with this step's bitmap reads
-            uint64_t nrows[kMiR];
-            bool nlive[kMiR];
-#pragma unroll
-            for (int k = 0; k < kMiR; ++k) {
-                nrows[k] = seg + 64u * kMiR + static_cast<uint64_t>(lane) * kMiR + k;
-                nlive[k] = nrows[k] < end;
-            }
-            mi_load<K, kMiR>(a.t1.data, nrows, nlive, cn);
-            if (chk_h1) a.h1.raw_n<kMiR>(nrows, nlive, chn);
-        }
-#pragma unroll
-        for (int k = 0; k < kMiR; ++k) {
-            v[k] = a.t1.dec_of(c[k]);
-            in[k] = live[k] && v[k] >= lo && ((v[k] - lo) >> 6) < words;
-        }
-#pragma unroll
-        for (int k = 0; k < kMiR; ++k) word[k] = in[k] ? mi.bits[(v[k] - lo) >> 6] : 0ull;
-        const uint64_t last_row = (end < seg + 64u * kMiR ? end : seg + 64u * kMiR) - 1u;
-        const uint32_t last_lane = static_cast<uint32_t>((last_row - seg) / kMiR);
-        const int last_k = static_cast<int>((last_row - seg) % kMiR);
-        const uint64_t up = __shfl_up(v[kMiR - 1], 1, 64);
-        const uint64_t pv0 = lane == 0 ? prev : up;
-        const bool hp0 = lane > 0 || has_prev;
-#pragma unroll
-        for (int k = 0; k < kMiR; ++k) {
-            if (!live[k]) continue;
-            const uint64_t pv = k == 0 ? pv0 : v[k - 1];
-            if (a.t1.bad_of(c[k]) || (chk_h1 && a.h1.bad_of(ch[k]))) bad = true;
-            if ((k > 0 || hp0) && !(pv < v[k])) bad = true;
-            if (in[k] && ((word[k] >> ((v[k] - lo) & 63u)) & 1ull) != 0ull) ++cnt;
-        }
-        uint64_t vl_own = v[0];
-#pragma unroll
-        for (int k = 1; k < kMiR; ++k) vl_own = k == last_k ? v[k] : vl_own;
-        prev = __shfl(vl_own, static_cast<int>(last_lane), 64);
-        has_prev = true;
-    }
-    cnt = wave_sum(cnt);
-    if (lane == 0) mi.wcnt[gw] = cnt;
-    if (bad) mi.ok[0] = 0u;
+// The value of the lane below (DPP wave shift); lane 0: `edge`.
+template <typename V>
+__device__ __forceinline__ V mi_lane_below(V x, V edge) {
+    auto one = [](uint32_t v, uint32_t e) {
+        return static_cast<uint32_t>(
+            __builtin_amdgcn_update_dpp(static_cast<int>(e), static_cast<int>(v), 0x138, 0xf, 0xf, false));
+    };
+    const uint32_t lo = one(static_cast<uint32_t>(x), static_cast<uint32_t>(edge));
+    if constexpr (sizeof(V) == 4) return lo;
+    else return static_cast<V>(one(static_cast<uint32_t>(x >> 32), static_cast<uint32_t>(edge >> 32))) << 32 | lo;
 }
 
-// Exclusive prefixes of the per-wave matches (one workgroup of 1024 threads) and the counts.
-__global__ __launch_bounds__(1024) void k_mi_scan(MergeArgs a, MiArgs mi) {
-    __shared__ uint32_t s_w[16];
-    if (mi.ok[0] == 0u) return;
-    const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;
-    uint64_t carry = 0;
-    for (uint32_t base = 0; base < mi.waves1; base += 8192u) {
-        uint32_t v[8], t = 0;
-#pragma unroll
-        for (int q = 0; q < 8; ++q) {
-            const uint32_t i = base + threadIdx.x * 8u + q;
-            v[q] = i < mi.waves1 ? mi.wcnt[i] : 0u;
-            t += v[q];
-        }
-        const uint32_t inc = wave_incl_scan(t);
-        if (lane == 63u) s_w[wv] = inc;
-        __syncthreads();
-        uint64_t pre = carry, tot = 0;
-#pragma unroll
-        for (int w = 0; w < 16; ++w) {
-            if (w < static_cast<int>(wv)) pre += s_w[w];
-            tot += s_w[w];
-        }
-        __syncthreads();
-        pre += inc - t;
-#pragma unroll
-        for (int q = 0; q < 8; ++q) {
-            const uint32_t i = base + threadIdx.x * 8u + q;
-            if (i < mi.waves1) mi.wpre[i] = static_cast<uint32_t>(pre);
-            pre += v[q];
-        }
-        carry += tot;
+template <typename V>
+__device__ __forceinline__ V mi_last_lane(V x) {
+    const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(x), 63));
+    if constexpr (sizeof(V) == 4) return lo;
+    else return static_cast<V>(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(x >> 32), 63))) << 32 | lo;
+}
+
+// List 1, on the single-pass engine: order and validity checks, and the pairs of the rows whose key is set.
+// A failed check sets the path's second flag; the sub-tile kernels then write all outputs (and counts) again.
+// V: keys are compared in 32 bits where every valid key fits (codes of up to 4 bytes, 8-byte codes whose
+// values fit and check by multiplying back, void ranges below 2^32).  VOID1: the keys are seqbase + row (a
+// whole dimension meets a selection of it).  GATHER: the right tails are read from t2 at the keys' rows.
+// Two ascending lists of 30.0M and 16.4M 8-byte OIDs, 8.2M matches: a count, a scan and a write pass over
+// list 1 took 184 us together, this pass 151 (174 with keys compared in 64 bits).
+// W8: both outputs are 8 bytes wide; a run-time width makes eight stores of each row's two, so much code
+// that a small call waits for its instructions, and takes fewer rows per lane (one tile of 2,556 void rows:
+// 21 us with 16 rows per lane, 11 with 8 and fixed widths).
+template <typename K, typename V, bool VOID1, bool GATHER, bool W8>
+struct IntersectOp {
+    static constexpr int kErr = 1;  // (no error on this path)
+    static constexpr int kG = !W8 ? 4 : sizeof(V) == 8 || VOID1 || GATHER ? 8 : 10;
+    struct RawK {
+        K c;
+    };
+    struct RawV {};
+    using Raw = std::conditional_t<VOID1, RawV, RawK>;
+    struct StateO {
+        uint32_t off;  // key - lo2 (the bitmap holds at most 2^32 bits)
+    };
+    struct StateJ {
+        uint32_t off, j;  // j: the set bits below the key's in its word
+    };
+    using State = std::conditional_t<GATHER, StateJ, StateO>;
+    uint64_t n;
+    MergeArgs a;
+    MiArgs mi;
+    const K *t1;
+    uint32_t back;    // 8-byte codes in 32 bits: their A (back_factor)
+    uint32_t chk_h1;  // h1's codes are checked too
+    uint32_t choose;  // the key width is decided by k_mi_clear: the form of the other width stands down
+    uint64_t out_cap;
+
+    struct Uniform {
+        uint64_t lo;
+        V lo_v;
+        uint32_t top;  // the bitmap's last bit
+        bool any;      // keys of type V reach the bitmap
+    };
+    __device__ bool skip() const { return mi.ok[0] == 0u || (choose && (mi.ok[2] != 0u) != (sizeof(V) == 8)); }
+    __device__ void init(char *) const {}
+    __device__ Uniform begin(const char *) const {
+        const uint64_t lo = mi.range[0];
+        return Uniform{lo, static_cast<V>(lo), static_cast<uint32_t>(mi.range[1] * 64ull - 1ull), lo <= static_cast<V>(~static_cast<V>(0))};
     }
-    if (threadIdx.x == 0) {
-        a.d_counts[0] = carry;
+    __device__ __forceinline__ void load(uint64_t first, uint32_t k, Raw &r) const {
+        if constexpr (!VOID1) r.c = __builtin_nontemporal_load(t1 + first + k);
+    }
+    template <int G>
+    struct Mid {
+        V v[G];
+        uint64_t word[G];
+        uint32_t in, bad;
+    };
+    template <int G>
+    __device__ __forceinline__ void open_tile(const char *, const Uniform &u, uint64_t first, uint32_t lane, uint32_t live,
+                                              const Raw (&raw)[G], Mid<G> &mid) const {
+        mid.in = 0;
+        mid.bad = 0;
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            V v;
+            if constexpr (VOID1) {
+                v = static_cast<V>(a.t1.raw(first + static_cast<uint32_t>(g * 64) + lane));
+            } else {
+                const uint64_t c = raw[g].c;
+                bool bad;
+                if constexpr (sizeof(K) == 8 && sizeof(V) == 4) {
+                    v = static_cast<uint32_t>(c) * static_cast<uint32_t>(a.t1.a_inv);
+                    bad = static_cast<uint64_t>(v) * back != c || v > a.t1.max_u;
+                } else {
+                    v = static_cast<V>(a.t1.dec_of(c));
+                    bad = a.t1.bad_of(c);
+                }
+                mid.bad |= (bad ? 1u : 0u) << g;
+            }
+            mid.v[g] = v;
+            const V off = v - u.lo_v;
+            const bool in = u.any && v >= u.lo_v && off <= u.top;
+            mid.in |= (in ? 1u : 0u) << g;
+            mid.word[g] = mi.bits[in ? off >> 6 : 0];
+        }
+        // the key before each row: the lane below's, the last lane's of the 64 rows before, the row before's
+        // (the first row has none; a half without rows, which may begin past the end, looks at nothing)
+        V edge = 0;
+        const bool has = first > 0 && first - 1 < n;
+        if (has) edge = static_cast<V>(a.t1.dec_of(a.t1.raw(first - 1)));
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            const V prev = mi_lane_below(mid.v[g], edge);
+            const bool check = g > 0 || lane != 0u || has;
+            mid.bad |= (check && !(prev < mid.v[g]) ? 1u : 0u) << g;
+            edge = mi_last_lane(mid.v[g]);
+        }
+        if (chk_h1) {
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                if (((live >> g) & 1u) && a.h1.bad_of(a.h1.raw(first + static_cast<uint32_t>(g * 64) + lane)))
+                    mid.bad |= 1u << g;
+            }
+        }
+    }
+    template <int G>
+    __device__ __forceinline__ void close_tile(const Uniform &u, const Mid<G> &mid, uint32_t live, State (&st)[G],
+                                               uint32_t &keep, uint32_t (&err)[kErr]) const {
+        keep = 0;
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            st[g].off = static_cast<uint32_t>(mid.v[g] - u.lo_v);
+            const uint32_t b = st[g].off & 63u;
+            keep |= (static_cast<uint32_t>(mid.word[g] >> b) & 1u) << g;
+            if constexpr (GATHER) st[g].j = static_cast<uint32_t>(__popcll(mid.word[g] & ((1ull << b) - 1ull)));
+        }
+        keep &= live & mid.in;
+        err[0] = 0;
+        // (a flag of its own: every workgroup of this launch decides to run by ok[0])
+        if ((live & mid.bad) != 0u) mi.ok[1] = 1u;
+    }
+    __device__ void report(uint64_t, State &, uint32_t &) const {}
+    __device__ __forceinline__ void emit(const Uniform &u, const State &st, uint64_t first, uint64_t pos, uint32_t row,
+                                         uint32_t k) const {
+        const uint64_t v = u.lo + st.off;
+        const uint64_t h = a.h1_from_t1 ? enc_key(a.t1, a.a_t1, v) : a.h1.raw(first + row);
+        uint64_t t;
+        if constexpr (GATHER) t = a.t2.raw(static_cast<uint64_t>(mi.first[st.off >> 6]) + st.j);
+        else t = enc_key(a.h2, a.a_h2, v);
+        const uint64_t oh = a.reenc_h ? h * a.f_h1 : h, ot = a.reenc_t ? t * a.f_t2 : t;
+        if constexpr (W8) {
+            static_cast<uint64_t *>(a.out_h)[pos + k] = oh;
+            static_cast<uint64_t *>(a.out_t)[pos + k] = ot;
+        } else {
+            store_w(a.out_h, pos + k, a.wout_h, oh);
+            store_w(a.out_t, pos + k, a.wout_t, ot);
+        }
+    }
+    __device__ void emit_err(int, uint64_t, const State &, uint64_t) const {}
+    __device__ void finish(const uint64_t *t) const {
+        a.d_counts[0] = t[0];
 #pragma unroll
         for (int s = 1; s < kMmStreams; ++s) a.d_counts[s] = 0ull;
     }
-}
+};
 
-// List 1, write pass: the pairs of the rows whose key is set, at the wave's prefix + their rank
-// (rows seg + g * 64 + lane, ranks from ballots).  The next step's keys are loaded while this
-// step's bitmap words are read.
-template <typename K>
-__global__ __launch_bounds__(kBlock) void k_mi_write(MergeArgs a, MiArgs mi) {
-    if (mi.ok[0] == 0u) return;
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t gw = blockIdx.x * kWaves + (threadIdx.x >> 6);
-    if (gw >= mi.waves1) return;
-    const uint64_t begin = static_cast<uint64_t>(gw) * mi.per1;
-    if (begin >= a.n1) return;
-    const uint64_t end = mi_rows_end(begin, mi.per1, a.n1);
-    const uint64_t lo = mi.range[0], words = mi.range[1];
-    uint64_t pos = mi.wpre[gw];
-    K c[kMiG];
-    {
-        uint64_t rows[kMiG];
-        bool live[kMiG];
-#pragma unroll
-        for (int g = 0; g < kMiG; ++g) {
-            rows[g] = begin + static_cast<uint64_t>(g) * 64u + lane;
-            live[g] = rows[g] < end;
-        }
-        mi_load<K, kMiG>(a.t1.data, rows, live, c);
-    }
-    for (uint64_t seg = begin; seg < end; seg += 64u * kMiG) {
-        uint64_t rows[kMiG], v[kMiG], word[kMiG];
-        bool live[kMiG], in[kMiG];
-#pragma unroll
-        for (int g = 0; g < kMiG; ++g) {
-            rows[g] = seg + static_cast<uint64_t>(g) * 64u + lane;
-            live[g] = rows[g] < end;
-            v[g] = a.t1.dec_of(static_cast<uint64_t>(c[g]));
-            in[g] = live[g] && v[g] >= lo && ((v[g] - lo) >> 6) < words;
-        }
-#pragma unroll
-        for (int g = 0; g < kMiG; ++g) word[g] = in[g] ? mi.bits[(v[g] - lo) >> 6] : 0ull;
-        {  // the next step's keys
-            uint64_t nrows[kMiG];
-            bool nlive[kMiG];
-#pragma unroll
-            for (int g = 0; g < kMiG; ++g) {
-                nrows[g] = seg + 64u * kMiG + static_cast<uint64_t>(g) * 64u + lane;
-                nlive[g] = nrows[g] < end;
-            }
-            mi_load<K, kMiG>(a.t1.data, nrows, nlive, c);
-        }
-#pragma unroll
-        for (int g = 0; g < kMiG; ++g) {
-            const uint32_t b = static_cast<uint32_t>((v[g] - lo) & 63u);
-            const bool hit = in[g] && ((word[g] >> b) & 1ull) != 0ull;
-            const uint64_t bal = __ballot(hit);
-            if (hit) {
-                const uint64_t p = pos + mi_below(bal);
-                if (p < a.out_cap) {
-                    const uint64_t h = a.h1_from_t1 ? enc_key(a.t1, a.a_t1, v[g]) : a.h1.raw(rows[g]);
-                    uint64_t t;
-                    if (a.t2_from_h2) {
-                        t = enc_key(a.h2, a.a_h2, v[g]);
-                    } else {
-                        const uint64_t j = static_cast<uint64_t>(mi.first[(v[g] - lo) >> 6]) +
-                                           static_cast<uint64_t>(__popcll(word[g] & ((1ull << b) - 1ull)));
-                        t = a.t2.raw(j);
-                    }
-                    store_w(a.out_h, p, a.wout_h, a.reenc_h ? h * a.f_h1 : h);
-                    store_w(a.out_t, p, a.wout_t, a.reenc_t ? t * a.f_t2 : t);
-                }
-            }
-            pos += static_cast<uint64_t>(__popcll(bal));
-        }
-    }
+template <typename K, typename V, bool VOID1>
+int launch_intersect(const MergeArgs &a, const MiArgs &mi, uint32_t back, bool choose, ahead_hip_ws *ws, hipStream_t s) {
+    auto run = [&](auto op) {
+        op.n = a.n1;
+        op.a = a;
+        op.mi = mi;
+        op.t1 = static_cast<const K *>(a.t1.data);
+        op.back = back;
+        op.choose = choose ? 1u : 0u;
+        op.chk_h1 = a.h1.encoded && (VOID1 || !(a.h1.data == a.t1.data && a.h1.width == a.t1.width && a.t1.encoded &&
+                                                a.h1.a_inv == a.t1.a_inv && a.h1.max_u == a.t1.max_u));
+        op.out_cap = a.out_cap;
+        return ahead_host::launch_stream(op, ws, s);
+    };
+    if (a.wout_h == 8 && a.wout_t == 8)
+        return a.t2_from_h2 ? run(IntersectOp<K, V, VOID1, false, true>{}) : run(IntersectOp<K, V, VOID1, true, true>{});
+    return a.t2_from_h2 ? run(IntersectOp<K, V, VOID1, false, false>{}) : run(IntersectOp<K, V, VOID1, true, false>{});
 }
 
 }  // namespace
@@ -1319,13 +1308,6 @@ void by_width(uint32_t w, F f) {
         case 4: f(uint32_t{}); break;
         default: f(uint64_t{}); break;
     }
-}
-
-template <typename K>
-uint32_t mi_cap1() {
-    static const uint32_t c = std::min(mi_resident(reinterpret_cast<const void *>(k_mi_count<K>)),
-                                       mi_resident(reinterpret_cast<const void *>(k_mi_write<K>)));
-    return c;
 }
 
 template <typename K>
@@ -1416,16 +1398,15 @@ extern "C" int ahead_hip_matchjoin_merge_an(const ahead_col *h1, const ahead_col
     // path's flag intact
     MiArgs mi{};
     mi.words_cap = kMiBitsPerRow * a.n2 / 64u + 2u;
-    // the path streams the key columns' codes: void key columns take the sub-tile path
-    const bool mi_eligible = t1->data != nullptr && h2->data != nullptr;
-    by_width(a.t1.width, [&](auto k) { mi.waves1 = mi_waves(a.n1, mi_cap1<decltype(k)>()); });
+    // list 2's keys are streamed into the bitmap: a void list 2 takes the sub-tile path.  Against a void
+    // list 1 (a dimension's rows) the bitmap may span them all, however few of them list 2 has.
+    const bool mi_eligible = h2->data != nullptr && a.n1 != 0 && a.n2 != 0;
+    if (t1->data == nullptr && a.n1 / 64u + 2u > mi.words_cap) mi.words_cap = a.n1 / 64u + 2u;
+    if (mi.words_cap > kMiWordsMax) mi.words_cap = kMiWordsMax;
     by_width(a.h2.width, [&](auto k) { mi.waves2 = mi_waves(a.n2, mi_cap2<decltype(k)>()); });
-    mi.per1 = mi_per(a.n1, mi.waves1);
     mi.per2 = mi_per(a.n2, mi.waves2);
     const size_t o_mi = o_end, o_bits = o_mi + 256, o_first = o_bits + align_up(mi.words_cap * 8, 256),
-                 o_wcnt = o_first + align_up(mi.words_cap * 4, 256),
-                 o_wpre = o_wcnt + align_up(static_cast<size_t>(mi.waves1) * 4, 256),
-                 o_tw = o_wpre + align_up(static_cast<size_t>(mi.waves1) * 4, 256),
+                 o_tw = o_first + align_up(mi.words_cap * 4, 256),
                  o_tm = o_tw + align_up(static_cast<size_t>(mi.waves2) * 4, 256),
                  o_all = o_tm + align_up(static_cast<size_t>(mi.waves2) * 8, 256);
     if ((st = ws_ensure(ws, o_all)) != AHEAD_OK) return st;
@@ -1433,8 +1414,6 @@ extern "C" int ahead_hip_matchjoin_merge_an(const ahead_col *h1, const ahead_col
     mi.range = reinterpret_cast<uint64_t *>(ws_region(ws, o_mi + 64));
     mi.bits = reinterpret_cast<uint64_t *>(ws_region(ws, o_bits));
     mi.first = reinterpret_cast<uint32_t *>(ws_region(ws, o_first));
-    mi.wcnt = reinterpret_cast<uint32_t *>(ws_region(ws, o_wcnt));
-    mi.wpre = reinterpret_cast<uint32_t *>(ws_region(ws, o_wpre));
     mi.tail_w = reinterpret_cast<uint32_t *>(ws_region(ws, o_tw));
     mi.tail_m = reinterpret_cast<uint64_t *>(ws_region(ws, o_tm));
     a.fast = mi.ok;
@@ -1462,13 +1441,18 @@ extern "C" int ahead_hip_matchjoin_merge_an(const ahead_col *h1, const ahead_col
             hipLaunchKernelGGL(k_mi_build<decltype(k)>, dim3(mi.waves2 / kWaves), dim3(kBlock), 0, s, a, mi);
         });
         hipLaunchKernelGGL(k_mi_tails, dim3((mi.waves2 + kBlock - 1) / kBlock), dim3(kBlock), 0, s, a, mi);
-        by_width(a.t1.width, [&](auto k) {
-            hipLaunchKernelGGL(k_mi_count<decltype(k)>, dim3(mi.waves1 / kWaves), dim3(kBlock), 0, s, a, mi);
-        });
-        hipLaunchKernelGGL(k_mi_scan, dim3(1), dim3(1024), 0, s, a, mi);
-        by_width(a.t1.width, [&](auto k) {
-            hipLaunchKernelGGL(k_mi_write<decltype(k)>, dim3(mi.waves1 / kWaves), dim3(kBlock), 0, s, a, mi);
-        });
+        // 8-byte codes of a small A: values of 2^32 and more, where the type has them, take a form of their own
+        const uint32_t back = t1->data != nullptr && a.t1.encoded && a.t1.width == 8 ? back_factor(a.t1.a_inv, 0xFFFFFFFFull) : 0u;
+        const bool choose = back != 0u && a.t1.max_u > 0xFFFFFFFFull;
+        if (t1->data == nullptr) {
+            st = launch_intersect<uint32_t, uint32_t, true>(a, mi, 0u, false, ws, s);
+        } else {
+            if (a.t1.width != 8 || back != 0u)
+                by_width(a.t1.width, [&](auto k) { st = launch_intersect<decltype(k), uint32_t, false>(a, mi, back, choose, ws, s); });
+            if (st == AHEAD_OK && a.t1.width == 8 && (back == 0u || choose))
+                st = launch_intersect<uint64_t, uint64_t, false>(a, mi, 0u, choose, ws, s);
+        }
+        if (st != AHEAD_OK) return st;
     }
     // the sub-tile path: its kernels return when the intersection path applied
     hipLaunchKernelGGL(k_mm_split, dim3((subs + kBlock) / kBlock), dim3(kBlock), 0, s, a, sp);

@@ -46,7 +46,8 @@
 //       // entry pos + k, of row first + row (first and pos are wave-uniform: scalar bases)
 //   void report(uint64_t row, State &, uint32_t &errs) const;  // the error streams of one row
 //   void init(char *lds) const;         // all threads, before the first tile; a barrier follows
-//   bool skip() const;                  // the whole launch stands down (decided from device state)
+//   bool skip() const;                  // the whole launch stands down (from device state that no
+//                                       // workgroup of this launch changes)
 #pragma once
 
 #include "rowtile.hpp"

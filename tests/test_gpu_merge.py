@@ -254,3 +254,37 @@ def test_merge_ascending_lists_of_every_key_width(kind):
     ref = run_both(h1, c1, c2, t2, RESOID, meta, meta, RESOID)
     assert ref[0].size == np.intersect1d(k1, k2).size and ref[0].size > 0
     run_both(c1, c1, c2, c2, meta, meta, meta, meta)
+
+
+@pytest.mark.parametrize("n1", [1, 63, 64, 512, 513, 767, 769, 1023, 1025, 12_288, 12_289, 16_383, 16_385, 200_003])
+@pytest.mark.parametrize("void1", [True, False])
+def test_merge_list1_tile_edges(n1, void1):
+    """List 1 at the edges of a wave's halves and of a workgroup's tile, as a void column (a whole
+    dimension met by a few of its rows, and by keys past its end) and as 8-byte codes of two types, with
+    gathered and with mirrored right sides and with heads of their own."""
+    seed = 7 * n1
+    m_int = an.an_meta(an.RESINT, 32417)
+    k2 = np.unique(np.concatenate([datagen.uniform(n1 // 9 + 2, seed, 1, 5, n1 + 40), np.array([5, n1 + 4])])).astype(np.uint64)
+    h2 = oid_list(k2, seed, 2)
+    t2 = oid_list(np.arange(k2.size, dtype=np.uint64) + 11, seed, 3)
+    h1 = oid_list(np.arange(n1, dtype=np.uint64) * 3, seed, 4)
+    bad_h1 = h1.copy()
+    bad_h1[n1 - 1] ^= np.uint64(2)
+    k1 = np.arange(n1, dtype=np.uint64) + 5
+
+    def both(head, tail, right, ref_head, ref_tail):
+        ref = O.matchjoin_merge_an(ref_head, ref_tail, O.Col(h2, RESOID), O.Col(right, RESOID))
+        c_h2 = capi.Column.from_numpy(h2, RESOID)
+        c_t2 = c_h2 if right is h2 else capi.Column.from_numpy(right, RESOID)
+        same(capi.matchjoin_merge_an(head, tail, c_h2, c_t2, err_cap=4), ref)
+        assert ref[0].size == np.intersect1d(k1, k2).size
+
+    for right in (h2, t2):
+        if void1:
+            for h in (h1, bad_h1):
+                both(capi.Column.from_numpy(h, RESOID), capi.Column.void(n1, 5), right, O.Col(h, RESOID), O.void(n1, 5))
+            both(capi.Column.void(n1, 5), capi.Column.void(n1, 5), right, O.void(n1, 5), O.void(n1, 5))
+        else:
+            for codes, meta in ((oid_list(k1, seed, 5), RESOID), (datagen.encode(k1, 32417, 8), m_int)):
+                both(capi.Column.from_numpy(h1, RESOID), capi.Column.from_numpy(codes, meta), right,
+                     O.Col(h1, RESOID), O.Col(codes, meta))
