@@ -1115,13 +1115,14 @@ __device__ __forceinline__ V mi_last_lane(V x) {
 // values fit and check by multiplying back, void ranges below 2^32).  VOID1: the keys are seqbase + row (a
 // whole dimension meets a selection of it).  GATHER: the right tails are read from t2 at the keys' rows.
 // Two ascending lists of 30.0M and 16.4M 8-byte OIDs, 8.2M matches: a count, a scan and a write pass over
-// list 1 took 184 us together, this pass 151 (174 with keys compared in 64 bits).
+// list 1 took 184 us together, this pass 129.
 // W8: both outputs are 8 bytes wide; a run-time width makes eight stores of each row's two, so much code
 // that a small call waits for its instructions, and takes fewer rows per lane (one tile of 2,556 void rows:
-// 21 us with 16 rows per lane, 11 with 8 and fixed widths).
+// 21 us with 16 rows per lane, 9 with 8 and fixed widths).
 template <typename K, typename V, bool VOID1, bool GATHER, bool W8>
 struct IntersectOp {
     static constexpr int kErr = 1;  // (no error on this path)
+    static constexpr bool kPack = true;  // (8.2M of 30M rows kept: 151 -> 129 us)
     static constexpr int kG = !W8 ? 4 : sizeof(V) == 8 || VOID1 || GATHER ? 8 : 10;
     struct RawK {
         K c;
@@ -1141,6 +1142,7 @@ struct IntersectOp {
     const K *t1;
     uint32_t back;    // 8-byte codes in 32 bits: their A (back_factor)
     uint32_t chk_h1;  // h1's codes are checked too
+    uint32_t same;    // both lists' codes of a key are the same
     uint32_t choose;  // the key width is decided by k_mi_clear: the form of the other width stands down
     uint64_t out_cap;
 
@@ -1236,7 +1238,7 @@ struct IntersectOp {
         const uint64_t h = a.h1_from_t1 ? enc_key(a.t1, a.a_t1, v) : a.h1.raw(first + row);
         uint64_t t;
         if constexpr (GATHER) t = a.t2.raw(static_cast<uint64_t>(mi.first[st.off >> 6]) + st.j);
-        else t = enc_key(a.h2, a.a_h2, v);
+        else t = same ? h : enc_key(a.h2, a.a_h2, v);
         const uint64_t oh = a.reenc_h ? h * a.f_h1 : h, ot = a.reenc_t ? t * a.f_t2 : t;
         if constexpr (W8) {
             static_cast<uint64_t *>(a.out_h)[pos + k] = oh;
@@ -1263,6 +1265,7 @@ int launch_intersect(const MergeArgs &a, const MiArgs &mi, uint32_t back, bool c
         op.t1 = static_cast<const K *>(a.t1.data);
         op.back = back;
         op.choose = choose ? 1u : 0u;
+        op.same = a.h1_from_t1 && a.t1.encoded == a.h2.encoded && (!a.t1.encoded || (a.a_t1 == a.a_h2 && a.t1.mask == a.h2.mask));
         op.chk_h1 = a.h1.encoded && (VOID1 || !(a.h1.data == a.t1.data && a.h1.width == a.t1.width && a.t1.encoded &&
                                                 a.h1.a_inv == a.t1.a_inv && a.h1.max_u == a.t1.max_u));
         op.out_cap = a.out_cap;

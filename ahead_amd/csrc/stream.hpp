@@ -45,6 +45,8 @@
 //   void emit(const Uniform &, const State &, uint64_t first, uint64_t pos, uint32_t row, uint32_t k) const;
 //       // entry pos + k, of row first + row (first and pos are wave-uniform: scalar bases)
 //   void report(uint64_t row, State &, uint32_t &errs) const;  // the error streams of one row
+//   static constexpr bool kPack = true; // (optional) a wave that drops rows packs its entries in LDS and
+//                                       // emits them 64 at a time; its op takes no tables (lds = 0)
 //   void init(char *lds) const;         // all threads, before the first tile; a barrier follows
 //   bool skip() const;                  // the whole launch stands down (from device state that no
 //                                       // workgroup of this launch changes)
@@ -115,6 +117,11 @@ __device__ __forceinline__ void stream_load(const Op &op, uint64_t first, uint32
     }
 }
 
+template <class Op, class = void>
+struct packs : std::false_type {};
+template <class Op>
+struct packs<Op, std::enable_if_t<Op::kPack>> : std::true_type {};
+
 template <class Op>
 __global__ __launch_bounds__(kStreamThreads) void k_stream(Op op, StreamArgs m) {
     constexpr int G = Op::kG, NS = 1 + Op::kErr, NW = kStreamWaves;
@@ -122,6 +129,9 @@ __global__ __launch_bounds__(kStreamThreads) void k_stream(Op op, StreamArgs m) 
     extern __shared__ __align__(16) char s_op[];
     __shared__ uint32_t s_cnt[NS][NW], s_sum[NS][NW];
     __shared__ uint32_t s_tile, s_epoch;
+    constexpr uint32_t kPackRows = packs<Op>::value ? kWaveRows : 1u;
+    __shared__ typename Op::State s_pack[packs<Op>::value ? NW : 1][kPackRows];
+    __shared__ uint16_t s_row[packs<Op>::value ? NW : 1][kPackRows];
     if (op.skip()) return;
     if (threadIdx.x == 0) {
         const unsigned long long v = atomicAdd(m.te, 1ull);
@@ -270,6 +280,31 @@ __global__ __launch_bounds__(kStreamThreads) void k_stream(Op op, StreamArgs m) 
             for (int g = 0; g < G; ++g) {
                 const uint32_t k = static_cast<uint32_t>(g * 64) + lane;
                 op.emit(uni, g < H ? st0[g % H] : st1[g % H], first, pos, k, k);
+            }
+        } else if (packs<Op>::value && kept != 0u) {
+            if constexpr (packs<Op>::value) {
+                // (a wave reads what its own lanes wrote: LDS operations of one wave keep their order)
+                uint32_t at = 0;
+#pragma unroll
+                for (int g = 0; g < G; ++g) {
+                    const bool on = (keep >> g) & 1u;
+                    const uint64_t b = __ballot(on);
+                    if (on) {
+                        const uint32_t k = at + wave_rank(b);
+                        s_pack[wave][k] = g < H ? st0[g % H] : st1[g % H];
+                        s_row[wave][k] = static_cast<uint16_t>(g * 64 + lane);
+                    }
+                    at += static_cast<uint32_t>(__popcll(b));
+                }
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                const uint32_t out = kept < room ? kept : room;
+                for (uint32_t k0 = 0; k0 < out; k0 += 64u) {
+                    const uint32_t k = k0 + lane;
+                    if (k < out) op.emit(uni, s_pack[wave][k], first, pos, s_row[wave][k], k);
+                }
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
             }
         } else if (kept != 0u) {
             uint32_t at = 0;
