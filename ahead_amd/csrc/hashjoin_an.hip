@@ -511,6 +511,9 @@ struct ProbeLeanOp {
         uint64_t pay;
     };
     using State = std::conditional_t<PV, StateV, StateP>;
+    // packed entries: all of a wave's rows where they and the filter fit the LDS, else half of them (60M
+    // foreign keys against a fifth of a dimension, the whole join: 349 -> 332 us)
+    static constexpr uint32_t kPack = sizeof(State) == 4 ? 64u * kG : 32u * kG;
     uint64_t n;
     HjTable t;
     const KT *key;                            // probe key codes

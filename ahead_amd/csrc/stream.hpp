@@ -45,8 +45,8 @@
 //   void emit(const Uniform &, const State &, uint64_t first, uint64_t pos, uint32_t row, uint32_t k) const;
 //       // entry pos + k, of row first + row (first and pos are wave-uniform: scalar bases)
 //   void report(uint64_t row, State &, uint32_t &errs) const;  // the error streams of one row
-//   static constexpr bool kPack = true; // (optional) a wave that drops rows packs its entries in LDS and
-//                                       // emits them 64 at a time; its op takes no tables (lds = 0)
+//   static constexpr uint32_t kPack;    // (optional) a wave that drops rows and keeps at most kPack packs
+//                                       // its entries in LDS and emits them 64 at a time
 //   void init(char *lds) const;         // all threads, before the first tile; a barrier follows
 //   bool skip() const;                  // the whole launch stands down (from device state that no
 //                                       // workgroup of this launch changes)
@@ -118,9 +118,19 @@ __device__ __forceinline__ void stream_load(const Op &op, uint64_t first, uint32
 }
 
 template <class Op, class = void>
-struct packs : std::false_type {};
+struct pack_rows : std::integral_constant<uint32_t, 0> {};
 template <class Op>
-struct packs<Op, std::enable_if_t<Op::kPack>> : std::true_type {};
+struct pack_rows<Op, std::enable_if_t<(Op::kPack > 0)>> : std::integral_constant<uint32_t, Op::kPack> {};
+template <class Op>
+struct StreamPack {  // a wave's packed entries
+    static constexpr uint32_t kRows = pack_rows<Op>::value ? pack_rows<Op>::value : 1u;
+    typename Op::State st[kRows];
+    uint16_t row[kRows];
+};
+template <class Op>
+constexpr size_t stream_pack_bytes() {
+    return pack_rows<Op>::value ? sizeof(StreamPack<Op>) * kStreamWaves : 0;
+}
 
 template <class Op>
 __global__ __launch_bounds__(kStreamThreads) void k_stream(Op op, StreamArgs m) {
@@ -129,9 +139,8 @@ __global__ __launch_bounds__(kStreamThreads) void k_stream(Op op, StreamArgs m) 
     extern __shared__ __align__(16) char s_op[];
     __shared__ uint32_t s_cnt[NS][NW], s_sum[NS][NW];
     __shared__ uint32_t s_tile, s_epoch;
-    constexpr uint32_t kPackRows = packs<Op>::value ? kWaveRows : 1u;
-    __shared__ typename Op::State s_pack[packs<Op>::value ? NW : 1][kPackRows];
-    __shared__ uint16_t s_row[packs<Op>::value ? NW : 1][kPackRows];
+    constexpr uint32_t kPack = pack_rows<Op>::value;
+    __shared__ StreamPack<Op> s_pack[kPack ? NW : 1];
     if (op.skip()) return;
     if (threadIdx.x == 0) {
         const unsigned long long v = atomicAdd(m.te, 1ull);
@@ -281,8 +290,8 @@ __global__ __launch_bounds__(kStreamThreads) void k_stream(Op op, StreamArgs m) 
                 const uint32_t k = static_cast<uint32_t>(g * 64) + lane;
                 op.emit(uni, g < H ? st0[g % H] : st1[g % H], first, pos, k, k);
             }
-        } else if (packs<Op>::value && kept != 0u) {
-            if constexpr (packs<Op>::value) {
+        } else if (kPack != 0u && kept != 0u && kept <= kPack) {
+            if constexpr (kPack != 0u) {
                 // (a wave reads what its own lanes wrote: LDS operations of one wave keep their order)
                 uint32_t at = 0;
 #pragma unroll
@@ -291,8 +300,8 @@ __global__ __launch_bounds__(kStreamThreads) void k_stream(Op op, StreamArgs m) 
                     const uint64_t b = __ballot(on);
                     if (on) {
                         const uint32_t k = at + wave_rank(b);
-                        s_pack[wave][k] = g < H ? st0[g % H] : st1[g % H];
-                        s_row[wave][k] = static_cast<uint16_t>(g * 64 + lane);
+                        s_pack[wave].st[k] = g < H ? st0[g % H] : st1[g % H];
+                        s_pack[wave].row[k] = static_cast<uint16_t>(g * 64 + lane);
                     }
                     at += static_cast<uint32_t>(__popcll(b));
                 }
@@ -301,12 +310,12 @@ __global__ __launch_bounds__(kStreamThreads) void k_stream(Op op, StreamArgs m) 
                 const uint32_t out = kept < room ? kept : room;
                 for (uint32_t k0 = 0; k0 < out; k0 += 64u) {
                     const uint32_t k = k0 + lane;
-                    if (k < out) op.emit(uni, s_pack[wave][k], first, pos, s_row[wave][k], k);
+                    if (k < out) op.emit(uni, s_pack[wave].st[k], first, pos, s_pack[wave].row[k], k);
                 }
                 __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
                 __builtin_amdgcn_wave_barrier();
             }
-        } else if (kept != 0u) {
+        } else if (kPack < kWaveRows && kept != 0u) {
             uint32_t at = 0;
 #pragma unroll
             for (int g = 0; g < G; ++g) {
@@ -412,7 +421,8 @@ struct StreamRows : Op {
 
 namespace ahead_host {
 
-// Launches the engine for op over op.n rows with `lds` bytes for its tables (at most kStreamLds).
+// Launches the engine for op over op.n rows with `lds` bytes for its tables (at most kStreamLds less the
+// packed entries).
 constexpr size_t kStreamLds = 152 * 1024;
 
 template <class Op>
@@ -428,7 +438,8 @@ int launch_stream(const Op &op, ahead_hip_ws *ws, hipStream_t s, size_t lds = 0)
     }();
     if (lds > 0) {
         static const hipError_t set = hipFuncSetAttribute(reinterpret_cast<const void *>(k_stream<Op>),
-                                                          hipFuncAttributeMaxDynamicSharedMemorySize, kStreamLds);
+                                                          hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                          static_cast<int>(kStreamLds - stream_pack_bytes<Op>()));
         AHEAD_HIP_TRY(set);
     }
     const uint64_t tiles = op.n == 0 ? 1 : (op.n + rows - 1) / rows;
