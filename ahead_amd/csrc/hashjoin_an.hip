@@ -178,8 +178,8 @@ struct OffsetOp {
     using State = uint8_t;
     uint64_t n;
     HjTable t;
+    __device__ bool skip() const { return t.flags[0] == 0u; }  // no key has several rows
     __device__ uint32_t eval(uint64_t row, State &, uint32_t &, uint64_t &) const {
-        if (t.flags[0] == 0u) return 0;
         const uint32_t c = t.cnt[row];
         return c > 1u ? c : 0u;
     }
@@ -457,6 +457,7 @@ struct ProbeOp {
         counts[0] = tot[0];
         counts[e_index[0]] = tot[1];
         counts[e_index[1]] = tot[2];
+        counts[5] = t.flags[1] ? 1u : 0u;  // the table's status
     }
 };
 
@@ -485,8 +486,8 @@ struct ProbeOneOp : ProbeOp {
 // found no key (flags[6]), the filter of the build keys is kept in LDS (8-byte keys) and only rows it
 // passes look their key up.
 // 60M foreign keys, 8-byte codes: every row joining a dimension of 200,000 void rows took 215 us and 178
-// for moving the pairs behind the first row that drops, now 235 in one pass; a fifth of them joining
-// 40,000 rows, re-encoded to 8-byte pairs, took 325 us and 135 for the two compaction passes, now 290.
+// for moving the pairs behind the first row that drops, now 240 in one pass; a fifth of them joining
+// 40,000 rows, re-encoded to 8-byte pairs, took 325 us and 135 for the two compaction passes, now 274.
 template <int KW, bool PV, bool BV, int OW>
 struct ProbeLeanOp {
     static constexpr int kErr = 2;  // probe head check, probe tail check
@@ -709,6 +710,7 @@ struct ProbeLeanOp {
         counts[0] = tot[0];
         counts[e_index[0]] = tot[1];
         counts[e_index[1]] = tot[2];
+        counts[5] = t.flags[1] ? 1u : 0u;  // the table's status
     }
 };
 
@@ -737,10 +739,6 @@ __global__ __launch_bounds__(kBlock) void k_hj_sample(ProbeOp p, uint64_t np) {
     uint32_t errs = 0;
     uint64_t aux = 0;
     if (row < np && p.eval(row, st, errs, aux) == 0u) atomicOr(&p.t.flags[6], 1u);
-}
-
-__global__ void k_hj_status(const uint32_t *flags, uint64_t *d_counts) {
-    d_counts[5] = flags[1] ? 1u : 0u;
 }
 
 }  // namespace
@@ -837,6 +835,8 @@ extern "C" int ahead_hip_hashjoin_an(const ahead_col *h1, const ahead_col *t1, c
                        reinterpret_cast<uint32_t *>(ws_region(ws, o_end)));
     AHEAD_HIP_TRY(hipGetLastError());
 
+    // (The status is the probe's last store, and the offsets stand down where no key has several rows: a
+    // launch of its own and a scan of empty slots cost 8 us of a 297 us join.)
     // build-side checks, in build-scan order: e3/e4 for a right build, e1/e2 for a left build
     Check2Op chk{};
     chk.n = nb;
@@ -939,7 +939,6 @@ extern "C" int ahead_hip_hashjoin_an(const ahead_col *h1, const ahead_col *t1, c
         if ((st = launch_stream(StreamRows<ProbeOneOp>(one), ws, s)) != AHEAD_OK) return st;
     }
     if ((st = launch_rowtile(p, np, 3, ws, s)) != AHEAD_OK) return st;
-    hipLaunchKernelGGL(k_hj_status, dim3(1), dim3(1), 0, s, t.flags, d_counts);
     AHEAD_HIP_TRY(hipGetLastError());
     return AHEAD_OK;
 }
