@@ -138,13 +138,15 @@ __global__ __launch_bounds__(kStreamThreads) void k_stream(Op op, StreamArgs m) 
     constexpr uint32_t kWaveRows = 64u * G, kAll = G == 32 ? 0xFFFFFFFFu : (1u << (G & 31)) - 1u;
     extern __shared__ __align__(16) char s_op[];
     __shared__ uint32_t s_cnt[NS][NW], s_sum[NS][NW];
-    __shared__ uint32_t s_tile, s_epoch;
+    // (the first tile has a word of its own: thread 0 stores the second one before the next barrier, when
+    // other waves may still have to read the first)
+    __shared__ uint32_t s_begin, s_tile, s_epoch;
     constexpr uint32_t kPack = pack_rows<Op>::value;
     __shared__ StreamPack<Op> s_pack[kPack ? NW : 1];
     if (op.skip()) return;
     if (threadIdx.x == 0) {
         const unsigned long long v = atomicAdd(m.te, 1ull);
-        s_tile = stream_tile(m, v);
+        s_begin = stream_tile(m, v);
         s_epoch = static_cast<uint32_t>(v >> 32) % ((1u << 30) - 1u) + 1u;
     }
     op.init(s_op);
@@ -152,7 +154,7 @@ __global__ __launch_bounds__(kStreamThreads) void k_stream(Op op, StreamArgs m) 
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wave = uniform(threadIdx.x >> 6);
     const uint32_t epoch = uniform(s_epoch);
-    uint32_t tile = uniform(s_tile);
+    uint32_t tile = uniform(s_begin);
     auto first_of = [&](uint32_t t) { return (static_cast<uint64_t>(t) * NW + wave) * kWaveRows; };
     auto left_of = [&](uint32_t t) {
         const uint64_t first = first_of(t);
