@@ -603,7 +603,7 @@ struct ProbeLeanOp {
                 for (int g = 0; g < G; ++g) ok[g] = ok[g] && brow[g] != UINT32_MAX;
             }
         } else {
-            constexpr int C = 4;  // (more at once do not fit the registers)
+            constexpr int C = G < 4 ? G : 4;  // (more at once do not fit the registers)
 #pragma unroll
             for (int q = 0; q < G; q += C) {
                 uint32_t sl[C];

@@ -2,7 +2,7 @@
 // ordered main output: check-and-decode, fetch, positional match, hash probe of unique keys.
 //
 // A persistent grid (one workgroup of 1024 threads per CU) takes tiles of 1024 x G rows in ticket
-// order.  Per tile, every lane evaluates its G rows, the tile publishes how many rows it keeps and
+// order (G: the operator's kG, or fewer for smaller calls, see launch_stream).  Per tile, every lane evaluates its G rows, the tile publishes how many rows it keeps and
 // reports, takes its place among all tiles from its predecessors' counts, and writes every entry
 // once, at its final place.  Nothing is staged, moved or re-read: the traffic is the inputs once
 // and the outputs once, whether rows are dropped or not.
@@ -30,7 +30,7 @@
 // is running, and a tile waits for lower tickets only, so the chain always drains.
 //
 // Op interface (beside eval / emit_err / finish of rowtile.hpp, which the rare error rows use):
-//   static constexpr int kErr, kG;      // error streams; rows per lane (even, at most 32)
+//   static constexpr int kErr, kG;      // error streams; rows per lane, at most (even, up to 32)
 //   struct Raw; using State;            // a row's streamed inputs; what its entry needs
 //   uint64_t out_cap;                   // entries the outputs hold
 //   struct Uniform; Uniform begin(const char *lds) const;      // read once per workgroup, after init
@@ -117,32 +117,33 @@ __device__ __forceinline__ void stream_load(const Op &op, uint64_t first, uint32
     }
 }
 
-template <class Op, class = void>
+template <class Op, int G, class = void>
 struct pack_rows : std::integral_constant<uint32_t, 0> {};
-template <class Op>
-struct pack_rows<Op, std::enable_if_t<(Op::kPack > 0)>> : std::integral_constant<uint32_t, Op::kPack> {};
-template <class Op>
+template <class Op, int G>
+struct pack_rows<Op, G, std::enable_if_t<(Op::kPack > 0)>>
+    : std::integral_constant<uint32_t, (Op::kPack < 64u * G ? Op::kPack : 64u * G)> {};
+template <class Op, int G>
 struct StreamPack {  // a wave's packed entries
-    static constexpr uint32_t kRows = pack_rows<Op>::value ? pack_rows<Op>::value : 1u;
+    static constexpr uint32_t kRows = pack_rows<Op, G>::value ? pack_rows<Op, G>::value : 1u;
     typename Op::State st[kRows];
     uint16_t row[kRows];
 };
-template <class Op>
+template <class Op, int G>
 constexpr size_t stream_pack_bytes() {
-    return pack_rows<Op>::value ? sizeof(StreamPack<Op>) * kStreamWaves : 0;
+    return pack_rows<Op, G>::value ? sizeof(StreamPack<Op, G>) * kStreamWaves : 0;
 }
 
-template <class Op>
+template <class Op, int G>
 __global__ __launch_bounds__(kStreamThreads) void k_stream(Op op, StreamArgs m) {
-    constexpr int G = Op::kG, NS = 1 + Op::kErr, NW = kStreamWaves;
+    constexpr int NS = 1 + Op::kErr, NW = kStreamWaves;
     constexpr uint32_t kWaveRows = 64u * G, kAll = G == 32 ? 0xFFFFFFFFu : (1u << (G & 31)) - 1u;
     extern __shared__ __align__(16) char s_op[];
     __shared__ uint32_t s_cnt[NS][NW], s_sum[NS][NW];
     // (the first tile has a word of its own: thread 0 stores the second one before the next barrier, when
     // other waves may still have to read the first)
     __shared__ uint32_t s_begin, s_tile, s_epoch;
-    constexpr uint32_t kPack = pack_rows<Op>::value;
-    __shared__ StreamPack<Op> s_pack[kPack ? NW : 1];
+    constexpr uint32_t kPack = pack_rows<Op, G>::value;
+    __shared__ StreamPack<Op, G> s_pack[kPack ? NW : 1];
     if (op.skip()) return;
     if (threadIdx.x == 0) {
         const unsigned long long v = atomicAdd(m.te, 1ull);
@@ -427,21 +428,25 @@ namespace ahead_host {
 // packed entries).
 constexpr size_t kStreamLds = 152 * 1024;
 
-template <class Op>
-int launch_stream(const Op &op, ahead_hip_ws *ws, hipStream_t s, size_t lds = 0) {
+// Rows per lane by the size of a call.  An operator's own kG suits tens of millions of rows, where the
+// tickets (15 ns each) ask for large tiles; 16,384 rows a tile keep 256 CUs busy from 4.2M rows on only.
+// One MI355X, us per call with 16 / 8 / 4 / 2 rows a lane:
+//   fetch of 4-byte codes, 400,000-row column: 500,000 rows 29 / 18 / 12 / 16, 1M 31 / 20 / 20 / 21,
+//   2M 33 / 27 / 26 / 33, 4M 51 / 42 / 44 / 57, 8M 68 / 67 / 75 / 100;
+//   check and decode of 8-byte codes: 500,000 rows 11 / 9 / 8 / 11, 1M 11 / 9 / 12 / 15, 2M 13 / 13 / 15 / 22,
+//   4M 18 / 18 / 23 / 36, 8M 25 / 28 / 38 / 63.
+// So 8 rows a lane below one and a half of the operator's own tiles per CU, and 4 where tiles of 8 would
+// reach fewer than three eighths of the CUs.  (2 are never better than 4 by more than 2 us.)
+constexpr int kStreamMidG = 8, kStreamSmallG = 4;
+
+template <class Op, int G>
+int launch_stream_g(const Op &op, ahead_hip_ws *ws, hipStream_t s, size_t lds, uint32_t cus) {
     using namespace ahead_dev;
-    constexpr uint64_t rows = static_cast<uint64_t>(kStreamThreads) * Op::kG;
-    static const uint32_t cus = [] {
-        int dev = 0, c = 0;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || c <= 0)
-            c = 256;
-        return static_cast<uint32_t>(c);
-    }();
+    constexpr uint64_t rows = static_cast<uint64_t>(kStreamThreads) * G;
     if (lds > 0) {
-        static const hipError_t set = hipFuncSetAttribute(reinterpret_cast<const void *>(k_stream<Op>),
+        static const hipError_t set = hipFuncSetAttribute(reinterpret_cast<const void *>(k_stream<Op, G>),
                                                           hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                          static_cast<int>(kStreamLds - stream_pack_bytes<Op>()));
+                                                          static_cast<int>(kStreamLds - stream_pack_bytes<Op, G>()));
         AHEAD_HIP_TRY(set);
     }
     const uint64_t tiles = op.n == 0 ? 1 : (op.n + rows - 1) / rows;
@@ -456,8 +461,32 @@ int launch_stream(const Op &op, ahead_hip_ws *ws, hipStream_t s, size_t lds = 0)
     m.agg = words;
     m.incl = words + tiles;
     m.erep = words + tiles * (2 + Op::kErr);
-    hipLaunchKernelGGL((k_stream<Op>), dim3(grid), dim3(kStreamThreads), lds, s, op, m);
+    hipLaunchKernelGGL((k_stream<Op, G>), dim3(grid), dim3(kStreamThreads), lds, s, op, m);
     AHEAD_HIP_TRY(hipGetLastError());
     return AHEAD_OK;
+}
+
+template <class Op>
+int launch_stream(const Op &op, ahead_hip_ws *ws, hipStream_t s, size_t lds = 0) {
+    using namespace ahead_dev;
+    static const uint32_t cus = [] {
+        int dev = 0, c = 0;
+        if (hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || c <= 0)
+            c = 256;
+        return static_cast<uint32_t>(c);
+    }();
+    // Tiles of fewer rows for calls that leave CUs idle otherwise, or give them one tile each, whose loads,
+    // lookups and places then follow one another (see kStreamMidG).
+    if constexpr (Op::kG > kStreamSmallG) {
+        constexpr int mid = Op::kG >= 2 * kStreamMidG ? kStreamMidG : Op::kG;
+        if (op.n < static_cast<uint64_t>(cus) * 3 / 8 * kStreamThreads * mid)
+            return launch_stream_g<Op, kStreamSmallG>(op, ws, s, lds, cus);
+        if constexpr (mid < Op::kG) {
+            if (op.n < static_cast<uint64_t>(cus) * 3 / 2 * kStreamThreads * Op::kG)
+                return launch_stream_g<Op, mid>(op, ws, s, lds, cus);
+        }
+    }
+    return launch_stream_g<Op, Op::kG>(op, ws, s, lds, cus);
 }
 }  // namespace ahead_host

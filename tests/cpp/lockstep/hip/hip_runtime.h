@@ -59,7 +59,7 @@ inline hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int *n, const voi
 }
 
 namespace lockstep {
-enum Op : int { kNone, kBarrier, kBallot, kShfl, kFirst, kRead, kDpp };
+enum Op : int { kNone, kBarrier, kBallot, kShfl, kFirst, kRead, kDpp, kSync };
 void launch(const char *name, dim3 grid, dim3 block, const std::function<void()> &kernel);
 uint32_t thread_id();
 uint32_t block_id();
@@ -101,6 +101,10 @@ inline uint32_t first_lane(uint32_t v) {
     const uint64_t *x = wave_op(kFirst, v, &on);
     return static_cast<uint32_t>(x[__builtin_ctzll(on)]);
 }
+inline void wave_sync() {
+    uint64_t on = 0;
+    wave_op(kSync, 0, &on);
+}
 inline uint32_t mbcnt(uint32_t mask, uint32_t base, uint32_t from) {
     const uint32_t l = lane();
     const uint32_t below = l <= from ? 0u : l - from >= 32u ? ~0u : (1u << (l - from)) - 1u;
@@ -132,7 +136,7 @@ inline uint32_t mbcnt(uint32_t mask, uint32_t base, uint32_t from) {
 #define __builtin_amdgcn_mbcnt_lo(m, b) lockstep::mbcnt(m, b, 0)
 #define __builtin_amdgcn_mbcnt_hi(m, b) lockstep::mbcnt(m, b, 32)
 #define __builtin_amdgcn_fence(order, scope) ((void)0)
-#define __builtin_amdgcn_wave_barrier() ((void)0)
+#define __builtin_amdgcn_wave_barrier() lockstep::wave_sync()
 #define __builtin_amdgcn_s_sleep(n) ((void)0)
 template <bool OK>
 inline void static_assert_dpp() {

@@ -55,6 +55,26 @@ def test_check_and_decode_tiles(width, n, bad):
     assert np.array_equal(err.to_numpy(np.uint64, c[1]), ref[1])
 
 
+@pytest.mark.parametrize("width", [2, 4, 8])
+@pytest.mark.parametrize("tiles,past", [(1, 1), (96, -1), (96, 0), (384, -1), (384, 0), (384, 1)])
+def test_check_and_decode_where_the_tile_changes(width, tiles, past):
+    """Rows per lane follow the size of a call: 4, 8 or the operator's own (launch_stream)."""
+    import torch
+
+    per_cu = torch.cuda.get_device_properties(0).multi_processor_count / 256
+    rows = 8 if tiles <= 96 else 32 if width == 2 else 16
+    n = int(tiles * per_cu) * 1024 * rows + past
+    codes, meta = codes_of(n, width, 5, seed=n)
+    print(f"check_and_decode width={width} n={n}", flush=True)
+    ref = O.check_and_decode_an(O.Col(codes, meta))
+    launch, dec, err, cnt = decode_call(capi.Column.from_numpy(codes, meta), n, 5)
+    launch()
+    capi.synchronize()
+    assert [int(x) for x in cnt.to_numpy(np.uint64, 2)] == [len(ref[0]), len(ref[1])]
+    assert np.array_equal(dec.to_numpy(f"u{meta.type.unenc_bits // 8}", len(ref[0])), ref[0])
+    assert np.array_equal(err.to_numpy(np.uint64, len(ref[1])), ref[1])
+
+
 @pytest.mark.parametrize("cap,ecap", [(0, 1), (1, 0), (TILE - 3, 7), (2 * TILE + 100, 900)])
 def test_check_and_decode_capacities(cap, ecap):
     n, bad = 3 * TILE + 11, 800

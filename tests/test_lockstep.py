@@ -7,17 +7,20 @@ import pytest
 
 import lockstep_lib as L
 import oracle_lib as O
-from ahead_amd import an, datagen
+from ahead_amd import an, capi, datagen
 
 pytestmark = pytest.mark.skipif(not L.available(), reason="no clang++ of ROCm to compile the kernels for the CPU")
+
+
+CUS = 256
 
 
 @pytest.fixture(params=[0, 1], ids=["ascending", "descending"])
 def waves(request):
     lib = L.lib()
-    lib.lockstep_set(request.param, 0, 1)
+    lib.lockstep_set(request.param, 0, CUS)
     yield request.param
-    lib.lockstep_set(0, 0, 4)
+    lib.lockstep_set(0, 0, CUS)
 
 
 @pytest.mark.parametrize("n,bad", [(5, 1), (16 * 1024 * 2 + 77, 3)])
@@ -36,3 +39,59 @@ def test_single_pass_engine_under_uneven_waves(waves, n, bad):
         assert cnt.tolist() == [n - bad, bad]
         assert np.array_equal(dec[:n - bad], ref[0]) and np.array_equal(err, ref[1])
         cnt[:] = 77
+
+
+
+@pytest.fixture
+def recorded():
+    """Launches are recorded, not run, on a card of 256 CUs."""
+    lib = L.lib()
+    lib.lockstep_set(0, 1, CUS)
+    L.launches()
+    yield lib
+    lib.lockstep_set(0, 0, CUS)
+
+
+def _somewhere(n, meta, **kw):
+    return L.column(None, meta, n, data=4096 if n else None, **kw)
+
+
+RESOID = an.an_meta(an.RESOID, an.A_OID)
+
+
+def _calls(n, ws):
+    """One call of n rows per operator of the single-pass engine: (name, rows of its streamed input, call)."""
+    lib, ref, b = L.lib(), ctypes.byref, capi.Buf(4096, n)
+    key, void = an.an_meta(an.RESINT, 65117), L.column(None, an.plain_meta(an.VOID), n)
+    oid, short = _somewhere(n, RESOID), _somewhere(n, an.an_meta(an.RESSHORT, 233))
+    out = []
+    for t, a in ((an.RESTINY, 233), (an.RESSHORT, 233), (an.RESINT, 65117)):
+        d = _somewhere(n, an.an_meta(t, a))
+        out.append((f"decode {t.name}", lambda d=d: lib.ahead_hip_check_and_decode_an(
+            ref(d), 1, 4096, n, 4096, n, 4096, ws.h, None)))
+    out.append(("fetch", lambda: lib.ahead_hip_fetchjoin_an(ref(oid), ref(short), 0, 0, 1, b, b, b, 4096, ws.h, None)))
+    out.append(("match", lambda: lib.ahead_hip_matchjoin_pos_an(
+        ref(void), ref(oid), ref(short), 0, 0, 4, 0, 0, 4, 1, b, b, b, b, b, 4096, ws.h, None)))
+    fk, bk, bv = _somewhere(n, key), _somewhere(500, key), L.column(None, an.plain_meta(an.VOID), 500)
+    out.append(("probe", lambda: lib.ahead_hip_hashjoin_an(
+        ref(void), ref(fk), ref(bk), ref(bv), 1, 0, 0, 4, 0, 0, 4, 1, *[b] * 6, 4096, ws.h, None)))
+    out.append(("merge", lambda: lib.ahead_hip_matchjoin_merge_an(
+        ref(oid), ref(oid), ref(oid), ref(oid), 0, 0, 8, 0, 0, 8, 1, *[b] * 6, 4096, ws.h, None)))
+    return out
+
+
+@pytest.mark.parametrize("n", [1, 4096, 4097, 20_000, 100_000, 500_000, 786_431, 786_433, 1_000_000, 2_000_000, 4_000_000,
+                               6_291_455, 6_291_456, 12_582_911, 12_582_912, 60_000_000])
+def test_single_pass_engine_spreads_a_call_over_the_card(recorded, n):
+    """Every workgroup a call of n rows can fill with 4 rows a lane runs, up to three eighths of the CUs; from
+    three eighths of the CUs x 8 rows a lane on, no fewer."""
+    ws = L.Workspace()
+    for name, call in _calls(n, ws):
+        L.launches()
+        L.check(call())
+        grids = [g for k, g, t in L.launches() if k.startswith("k_stream")]
+        assert grids, name
+        for g in grids:
+            assert min(-(-n // 4096), CUS * 3 // 8) <= g <= CUS, (name, n, g)
+            if n >= 60_000_000:
+                assert g == CUS
