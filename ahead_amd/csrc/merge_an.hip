@@ -941,6 +941,13 @@ __device__ __forceinline__ uint64_t mi_wave_or(uint64_t x) {
     return x;
 }
 
+// The steps of k_mi_build on the wave's LDS slice: LDS operations of one wave keep their order on the
+// card; the compiler keeps it across this too.
+__device__ __forceinline__ void mi_wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 template <typename K>
 __global__ __launch_bounds__(kBlock) void k_mi_build(MergeArgs a, MiArgs mi) {
     __shared__ unsigned long long s_bits[kWaves][kMiLdsWords];
@@ -1032,12 +1039,15 @@ __global__ __launch_bounds__(kBlock) void k_mi_build(MergeArgs a, MiArgs mi) {
                 const uint32_t o = w[k] - wf;
                 if (in[k] && o < span) atomicOr(sb + o, 1ull << ((v[k] - lo) & 63u));
             }
+            mi_wave_sync();
             const uint64_t x0 = sb[0], xl = sb[span - 1u];
+            mi_wave_sync();
             for (uint32_t o = lane; o < span; o += 64u) {
                 const unsigned long long x = sb[o];
                 sb[o] = 0ull;
                 if (o > 0u && o + 1u < span && x != 0ull) mi.bits[wf + o] = x;  // all of the word's keys are in this step
             }
+            mi_wave_sync();
             if (ow == wf) {
                 om |= x0;
             } else {
@@ -1153,6 +1163,7 @@ struct IntersectOp {
         bool any;      // keys of type V reach the bitmap
     };
     __device__ bool skip() const { return mi.ok[0] == 0u || (choose && (mi.ok[2] != 0u) != (sizeof(V) == 8)); }
+    __device__ bool stop() const { return __hip_atomic_load(&mi.ok[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u; }
     __device__ void init(char *) const {}
     __device__ Uniform begin(const char *) const {
         const uint64_t lo = mi.range[0];
@@ -1229,7 +1240,7 @@ struct IntersectOp {
         keep &= live & mid.in;
         err[0] = 0;
         // (a flag of its own: every workgroup of this launch decides to run by ok[0])
-        if ((live & mid.bad) != 0u) mi.ok[1] = 1u;
+        if ((live & mid.bad) != 0u) __hip_atomic_store(&mi.ok[1], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     __device__ void report(uint64_t, State &, uint32_t &) const {}
     __device__ __forceinline__ void emit(const Uniform &u, const State &st, uint64_t first, uint64_t pos, uint32_t row,

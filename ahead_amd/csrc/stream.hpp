@@ -50,6 +50,8 @@
 //   void init(char *lds) const;         // all threads, before the first tile; a barrier follows
 //   bool skip() const;                  // the whole launch stands down (from device state that no
 //                                       // workgroup of this launch changes)
+//   bool stop() const;                  // (optional) nothing this launch writes will be used: read by one thread
+//                                       // with every ticket; the tiles still to come are counted as empty
 #pragma once
 
 #include "rowtile.hpp"
@@ -117,6 +119,11 @@ __device__ __forceinline__ void stream_load(const Op &op, uint64_t first, uint32
     }
 }
 
+template <class Op, class = void>
+struct has_stop : std::false_type {};
+template <class Op>
+struct has_stop<Op, std::void_t<decltype(std::declval<const Op &>().stop())>> : std::true_type {};
+
 template <class Op, int G, class = void>
 struct pack_rows : std::integral_constant<uint32_t, 0> {};
 template <class Op, int G>
@@ -141,7 +148,7 @@ __global__ __launch_bounds__(kStreamThreads) void k_stream(Op op, StreamArgs m) 
     __shared__ uint32_t s_cnt[NS][NW], s_sum[NS][NW];
     // (the first tile has a word of its own: thread 0 stores the second one before the next barrier, when
     // other waves may still have to read the first)
-    __shared__ uint32_t s_begin, s_tile, s_epoch;
+    __shared__ uint32_t s_begin, s_tile, s_epoch, s_stop;
     constexpr uint32_t kPack = pack_rows<Op, G>::value;
     __shared__ StreamPack<Op, G> s_pack[kPack ? NW : 1];
     if (op.skip()) return;
@@ -170,7 +177,11 @@ __global__ __launch_bounds__(kStreamThreads) void k_stream(Op op, StreamArgs m) 
     }
     while (tile < m.tiles) {
         unsigned long long ticket;  // the next tile's, taken by thread 0 while the inputs arrive
-        if (threadIdx.x == 0) ticket = atomicAdd(m.te, 1ull);
+        bool stop = false;
+        if (threadIdx.x == 0) {
+            ticket = atomicAdd(m.te, 1ull);
+            if constexpr (has_stop<Op>::value) stop = op.stop();
+        }
         const uint64_t first = first_of(tile);
         const uint32_t left = left_of(tile);
         typename Op::State st0[H], st1[H];
@@ -214,7 +225,10 @@ __global__ __launch_bounds__(kStreamThreads) void k_stream(Op op, StreamArgs m) 
 #pragma unroll
             for (int e = 0; e < Op::kErr; ++e) s_cnt[1 + e][wave] = ecnt[e];
         }
-        if (threadIdx.x == 0) s_tile = stream_tile(m, ticket);
+        if (threadIdx.x == 0) {
+            s_tile = stream_tile(m, ticket);
+            if constexpr (has_stop<Op>::value) s_stop = stop ? 1u : 0u;
+        }
         __syncthreads();
         uint32_t agg[NS], before[NS], rep = 0;
 #pragma unroll
@@ -242,6 +256,7 @@ __global__ __launch_bounds__(kStreamThreads) void k_stream(Op op, StreamArgs m) 
             lb_store(&m.agg[tile], stream_word(epoch, (rep != 0u ? 1ull << 33 : 0ull) | agg[0]));
         }
         const uint32_t next = uniform(s_tile);
+        if constexpr (has_stop<Op>::value) stop = uniform(s_stop) != 0u;
         if (next < m.tiles) {
             stream_load<Op, H>(op, first_of(next), lane, left_of(next), 0, raw0);
             stream_load<Op, H>(op, first_of(next), lane, left_of(next), 1, raw1);
@@ -355,6 +370,17 @@ __global__ __launch_bounds__(kStreamThreads) void k_stream(Op op, StreamArgs m) 
             op.finish(totals);
         }
         tile = next;
+        if constexpr (has_stop<Op>::value) {
+            if (stop) {  // the workgroup's further tiles: empty, so that no other one waits for them
+                while (threadIdx.x == 0 && tile < m.tiles) {
+                    lb_store(&m.agg[tile], stream_word(epoch, 0));
+#pragma unroll
+                    for (int s = 0; s < NS; ++s) lb_store(&m.incl[static_cast<size_t>(s) * m.tiles + tile], stream_word(epoch, 0));
+                    tile = stream_tile(m, atomicAdd(m.te, 1ull));
+                }
+                return;
+            }
+        }
     }
 }
 

@@ -37,6 +37,7 @@ char *stacks;
 const std::function<void()> *body;
 uint32_t cur, bid, bdim, gdim;
 bool bar_any, bar_out;
+uint64_t steps;  // wave-wide operations and barriers, summed over the waves, of the launch
 int descending, dry, cus = 4, device;
 std::string log_;
 std::vector<std::string> attrs;
@@ -67,6 +68,7 @@ bool run_wave(uint32_t w) {
         }
         Op op = kNone;
         uint64_t on = 0;
+        ++steps;
         for (uint32_t i = b; i < e; ++i) {
             if (lanes[i].done) continue;
             if (op == kNone) op = lanes[i].op;
@@ -134,7 +136,11 @@ const uint64_t *wave_op(Op op, uint64_t v, uint64_t *on) {
 }
 
 void launch(const char *name, dim3 grid, dim3 block, const std::function<void()> &kernel) {
-    log_ += std::string(name) + " " + std::to_string(grid.x) + " " + std::to_string(block.x) + "\n";
+    struct Log {
+        std::string head;
+        ~Log() { log_ += head + std::to_string(steps) + "\n"; }
+    } log{std::string(name) + " " + std::to_string(grid.x) + " " + std::to_string(block.x) + " "};
+    steps = 0;
     if (dry) return;
     if (block.x > kMost) bad("workgroup too large");
     if (stacks == nullptr) {
@@ -186,7 +192,7 @@ void lockstep_set(int descending, int dry, int cus) {
     lockstep::cus = cus;
 }
 void lockstep_device(int device) { lockstep::device = device; }
-// The launches since the last call, one line each: kernel, workgroups, threads.
+// The launches since the last call, one line each: kernel, workgroups, threads, steps run.
 const char *lockstep_launches(void) {
     static std::string out;
     out.swap(lockstep::log_);

@@ -85,16 +85,16 @@ class Workspace:
         lib().ahead_hip_ws_destroy(self.h)
 
 
-def launches() -> list[tuple[str, int, int]]:
-    """(kernel, workgroups, threads) of every launch since the last call; ("attribute", device, 0) for each
-    hipFuncSetAttribute."""
+def launches() -> list[tuple[str, int, int, int]]:
+    """(kernel, workgroups, threads, steps) of every launch since the last call, the steps being the wave-wide
+    operations and barriers its waves went through; ("attribute", device, 0, 0) for each hipFuncSetAttribute."""
     out = []
     for line in lib().lockstep_launches().decode().splitlines():
         if line.startswith("attribute"):
-            out.append(("attribute", int(line.split()[1]), 0))
+            out.append(("attribute", int(line.split()[1]), 0, 0))
         else:
-            name, grid, block = line.rsplit(" ", 2)
-            out.append((name.strip("()"), int(grid), int(block)))
+            name, grid, block, steps = line.rsplit(" ", 3)
+            out.append((name.strip("()"), int(grid), int(block), int(steps)))
     return out
 
 

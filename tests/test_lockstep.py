@@ -89,9 +89,42 @@ def test_single_pass_engine_spreads_a_call_over_the_card(recorded, n):
     for name, call in _calls(n, ws):
         L.launches()
         L.check(call())
-        grids = [g for k, g, t in L.launches() if k.startswith("k_stream")]
+        grids = [x[1] for x in L.launches() if x[0].startswith("k_stream")]
         assert grids, name
         for g in grids:
             assert min(-(-n // 4096), CUS * 3 // 8) <= g <= CUS, (name, n, g)
             if n >= 60_000_000:
                 assert g == CUS
+
+
+def _merge(t1, h2, ws):
+    """The pairs and counts of a merge of two OID lists against themselves, and the launches it made."""
+    cap = max(1, min(t1.size, h2.size))
+    oh, ot, cnt = np.zeros(cap, np.uint64), np.zeros(cap, np.uint64), np.zeros(5, np.uint64)
+    errs = [np.zeros(4 * (t1.size + h2.size), np.uint64) for _ in range(4)]
+    d1, d2 = L.column(t1, RESOID), L.column(h2, RESOID)
+    L.launches()
+    L.check(L.lib().ahead_hip_matchjoin_merge_an(
+        *[ctypes.byref(x) for x in (d1, d1, d2, d2)], 0, 0, 8, 0, 0, 8, an.A_OID_ERR, L.buf(oh), L.buf(ot),
+        *[L.buf(e) for e in errs], cnt.ctypes.data, ws.h, None))
+    k = cnt.tolist()
+    got = [oh[:k[0]], ot[:k[0]], *[e[:c] for e, c in zip(errs, k[1:])]]
+    ref = O.matchjoin_merge_an(O.Col(t1, RESOID), O.Col(t1, RESOID), O.Col(h2, RESOID), O.Col(h2, RESOID))
+    for i, (x, y) in enumerate(zip(got, ref)):
+        assert np.array_equal(x, y), i
+    return L.launches()
+
+
+def test_merge_stops_when_list_1_fails_a_check():
+    """The pass over list 1 ends soon after a row fails; the walk that writes the outputs is not its concern."""
+    n = 200_000
+    L.lib().lockstep_set(0, 0, CUS)
+    ws, keys = L.Workspace(), np.arange(n, dtype=np.uint64) * np.uint64(3)
+    lists = keys * np.uint64(an.A_OID), keys[::2] * np.uint64(an.A_OID)
+    steps = []
+    for bad in (False, True):
+        t1 = lists[0].copy()
+        if bad:
+            t1[700] = t1[699] - np.uint64(an.A_OID)
+        steps.append(sum(x[3] for x in _merge(t1, lists[1], ws) if "k_stream" in x[0]))
+    assert steps[1] * 4 < steps[0]
