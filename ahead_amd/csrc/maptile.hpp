@@ -302,6 +302,22 @@ size_t map_scratch_bytes(uint64_t n) {
     return 2 * align_up(NS * waves * 4, 256) + align_up(waves * 4, 256) + align_up(waves * kMapErrList * 8, 256) + 256;
 }
 
+// Rows of a wave's range for n rows: whole steps.
+template <class Op>
+uint64_t map_rows_per_wave(uint64_t n) {
+    using namespace ahead_dev;
+    const uint64_t waves = static_cast<uint64_t>(map_grid<Op>(n)) * kWaves;
+    constexpr uint64_t step = 64u * MapG<Op>::value;
+    return ((n + waves - 1) / waves + step - 1) / step * step;
+}
+
+// Workgroups of the map engine's grid that have rows: the first ones.
+template <class Op>
+uint32_t map_parts(uint64_t n) {
+    const uint64_t rows = map_rows_per_wave<Op>(n) * ahead_dev::kWaves;
+    return n == 0 ? 1u : static_cast<uint32_t>((n + rows - 1) / rows);
+}
+
 // Launches the map engine for op over op.n rows.  Scratch: per-wave tables in the workspace region
 // at `offset`.  A caller that keeps regions of its own before `offset` must have grown the
 // workspace to offset + map_scratch_bytes<Op>(n) beforehand (growing moves the workspace).
@@ -311,9 +327,6 @@ int launch_map(const Op &op, ahead_hip_ws *ws, size_t offset, hipStream_t s) {
     constexpr int NS = MapTraits<Op>::NS;
     const uint32_t grid = map_grid<Op>(op.n);
     const uint32_t waves = grid * kWaves;
-    uint64_t per = (op.n + waves - 1) / waves;
-    constexpr uint64_t step = 64u * MapG<Op>::value;
-    per = (per + step - 1) / step * step;
     const size_t o_cnt = offset, o_pre = o_cnt + align_up(static_cast<size_t>(NS) * waves * 4, 256),
                  o_erows = o_pre + align_up(static_cast<size_t>(NS) * waves * 4, 256),
                  o_elist = o_erows + align_up(static_cast<size_t>(waves) * 4, 256),
@@ -324,7 +337,7 @@ int launch_map(const Op &op, ahead_hip_ws *ws, size_t offset, hipStream_t s) {
         return fail(AHEAD_ERR_INVALID, "map engine: the workspace was not grown before its regions were placed");
     if ((st = ws_ensure(ws, o_end)) != AHEAD_OK) return st;
     MapArgs m{};
-    m.rows_per_wave = per;
+    m.rows_per_wave = map_rows_per_wave<Op>(op.n);
     m.waves = waves;
     m.wcnt = reinterpret_cast<uint32_t *>(ws_region(ws, o_cnt));
     m.wpre = reinterpret_cast<uint32_t *>(ws_region(ws, o_pre));

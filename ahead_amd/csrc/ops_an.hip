@@ -798,7 +798,7 @@ __global__ __launch_bounds__(kBlock) void k_mulsum_final(const uint64_t *partial
 
 // ---------------------------------------------------------------------------------------------------
 // Grouped sum: LDS-private accumulators per workgroup when the groups fit, then one partial per group and
-// workgroup and a reduction; otherwise straight 64-bit atomics on the output.
+// workgroup with rows and a reduction; otherwise straight 64-bit atomics on the output.
 constexpr uint32_t kAggLds = 4096;  // 64-bit words
 
 struct AggSumArgs {
@@ -807,7 +807,8 @@ struct AggSumArgs {
     uint64_t num_groups, enc, a_oid;
     uint32_t grp_back, tail_back;  // the codes' A where 32-bit arithmetic decodes them (back_factor), else 0
     uint32_t copies;               // accumulators per group in LDS (a power of two; 0: none)
-    uint64_t *partials;            // [num_groups][workgroups] (copies != 0)
+    uint32_t parts;                // workgroups with rows: those that leave partials
+    uint64_t *partials;            // [parts][num_groups] (copies != 0)
     uint64_t *sums;
     uint64_t *err[3];
     uint64_t cap[3];
@@ -818,8 +819,11 @@ struct AggSumOp {
     // Checks and sums in one pass.  Few groups make the lanes of a wave meet on the same LDS word, and
     // same-word atomics run one after another (12M rows into 35 groups: 71 us, 4.5 times what the two
     // columns take to read).  So a group has up to 32 accumulators side by side, each lane adding to its
-    // own of them, and the workgroups leave partials: 12M rows 52 us.  The codes are summed as they
+    // own of them, and the workgroups leave partials: 12M rows 57 us.  The codes are summed as they
     // are and multiplied by the re-encoding factor at the end (sums mod 2^64 are linear).
+    // Many groups make the partials the cost: only workgroups with rows leave them, side by side
+    // (4096 groups: 250,000 rows 74 us when all 977 workgroups of the grid did, each group's in a row of
+    // its own, 23 now; 4M rows 86 and 49; 30M rows 128, by atomics on the output 1230).
     static constexpr int kErr = 3;
     static constexpr int kMapRows = 8;  // twice the loads in flight
     static constexpr int kSharedWords = kAggLds;
@@ -833,11 +837,11 @@ struct AggSumOp {
         for (uint32_t i = threadIdx.x; i < nw; i += blockDim.x) s[i] = 0ull;
     }
     __device__ void shared_flush(unsigned long long *s) const {
-        if (a.copies == 0u) return;
+        if (a.copies == 0u || blockIdx.x >= a.parts) return;
         for (uint32_t i = threadIdx.x; i < a.num_groups; i += blockDim.x) {
             unsigned long long x = 0ull;
             for (uint32_t c = 0; c < a.copies; ++c) x += s[i * a.copies + ((c + i) & (a.copies - 1u))];
-            a.partials[static_cast<size_t>(i) * gridDim.x + blockIdx.x] = x;
+            a.partials[blockIdx.x * a.num_groups + i] = x;
         }
     }
     // aggregateAN.tcc:84-112: a corrupt tail is still added (and reported); a row whose group id
@@ -915,15 +919,28 @@ struct AggSumOp {
 };
 
 
-// The group's partials of all workgroups, re-encoded.  (Added to the output with atomics by every
-// workgroup, 1280 of them meeting on each group's word cost 20 us.)
-__global__ __launch_bounds__(kBlock) void k_aggsum_final(AggSumArgs a, uint32_t parts) {
-    __shared__ uint64_t s_red[kWaves];
-    for (uint64_t g = blockIdx.x; g < a.num_groups; g += gridDim.x) {
-        uint64_t x = 0;
-        for (uint32_t i = threadIdx.x; i < parts; i += kBlock) x += a.partials[g * parts + i];
-        x = block_sum<uint64_t>(x, s_red);
-        if (threadIdx.x == 0) a.sums[g] = x * a.enc;
+// The groups' partials of all workgroups, re-encoded: kAggFinal groups per workgroup, whose threads read
+// them side by side.  (Added to the output with atomics by every workgroup, 1280 of them meeting on each
+// group's word cost 20 us.)
+constexpr uint32_t kAggFinal = 4;
+__global__ __launch_bounds__(kBlock) void k_aggsum_final(AggSumArgs a) {
+    __shared__ uint64_t s_sum[kWaves][kAggFinal];
+    const uint32_t lane = threadIdx.x & 63u, sub = threadIdx.x % kAggFinal;
+    const uint64_t g = static_cast<uint64_t>(blockIdx.x) * kAggFinal + sub;
+    uint64_t x = 0;
+    if (g < a.num_groups) {
+#pragma unroll 4
+        for (uint32_t i = threadIdx.x / kAggFinal; i < a.parts; i += kBlock / kAggFinal) x += a.partials[i * a.num_groups + g];
+    }
+#pragma unroll
+    for (int d = 32; d >= static_cast<int>(kAggFinal); d >>= 1) x += __shfl_xor(x, d, 64);
+    if (lane < kAggFinal) s_sum[threadIdx.x >> 6][lane] = x;
+    __syncthreads();
+    if (threadIdx.x < kAggFinal && g < a.num_groups) {
+        uint64_t t = 0;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) t += s_sum[w][threadIdx.x];
+        a.sums[g] = t * a.enc;
     }
 }
 
@@ -1111,10 +1128,6 @@ extern "C" int ahead_hip_aggregate_sum_grouped_an(const ahead_col *head, const a
     // (a group id in range is below 2^32 unless there are more groups than that)
     a.grp_back = num_groups <= 0xFFFFFFFFull ? back_factor(grouping->a_inv, 0xFFFFFFFFull) : 0u;
     a.tail_back = a.tail.encoded && a.tail.width == 8 ? back_factor(a.tail.a_inv, a.tail.max_u) : 0u;
-    if (num_groups && num_groups <= kAggLds) {
-        a.copies = 1;
-        while (a.copies < 32u && 2ull * a.copies * num_groups <= kAggLds) a.copies *= 2;
-    }
     a.sums = sums;
     const ahead_buf e[3] = {e_head, e_tail, e_group};
     for (int i = 0; i < 3; ++i) {
@@ -1126,9 +1139,11 @@ extern "C" int ahead_hip_aggregate_sum_grouped_an(const ahead_col *head, const a
     AggSumOp op{};
     op.n = a.n;
     size_t o_map = 0;
-    const uint32_t parts = map_waves<AggSumOp>(op.n) / kWaves;  // one partial per workgroup and group
-    if (a.copies != 0u) {
-        o_map = align_up(num_groups * parts * 8ull, 256);
+    if (num_groups && num_groups <= kAggLds) {
+        a.copies = 1;
+        while (a.copies < 32u && 2ull * a.copies * num_groups <= kAggLds) a.copies *= 2;
+        a.parts = map_parts<AggSumOp>(op.n);
+        o_map = align_up(num_groups * a.parts * 8ull, 256);
         if ((st = ws_ensure(ws, o_map + map_scratch_bytes<AggSumOp>(op.n))) != AHEAD_OK) return st;
         a.partials = reinterpret_cast<uint64_t *>(ws_region(ws, 0));
     } else if (num_groups) {
@@ -1138,8 +1153,8 @@ extern "C" int ahead_hip_aggregate_sum_grouped_an(const ahead_col *head, const a
     op.a = a;
     if ((st = launch_map(op, ws, o_map, s)) != AHEAD_OK) return st;
     if (a.copies != 0u) {
-        hipLaunchKernelGGL(k_aggsum_final, dim3(static_cast<uint32_t>(num_groups < 1024 ? num_groups : 1024)), dim3(kBlock),
-                           0, s, a, parts);
+        hipLaunchKernelGGL(k_aggsum_final, dim3(static_cast<uint32_t>((num_groups + kAggFinal - 1) / kAggFinal)), dim3(kBlock), 0,
+                           s, a);
         AHEAD_HIP_TRY(hipGetLastError());
     }
     return AHEAD_OK;

@@ -208,6 +208,19 @@ def test_aggregate_sum_grouped_parity(n, G):
     same(got, ref)
 
 
+@pytest.mark.parametrize("n,G", [(600_001, 4096), (3_000_001, 1), (700_000, 2048), (2_700_000, 35), (2048 * 300, 4095)])
+def test_aggregate_sum_grouped_partials(n, G):
+    """One partial per group and workgroup with rows, for some and for all workgroups of the grid."""
+    meta = an.an_meta(an.RESINT, 65117)
+    codes = datagen.encode(datagen.uniform(n, G, 1, 90_000, 10_500_000), 65117, 8)
+    gcodes = enc_oids(datagen.uniform(n, G, 3, 0, G - 1))
+    codes[n // 2] ^= np.uint64(1 << 40)
+    print(f"grouped sum n={n} groups={G}", flush=True)
+    ref = O.aggregate_sum_grouped_an(O.void(n), O.Col(codes, meta), O.Col(gcodes, RESOID), G)
+    for _ in range(2):
+        same(capi.aggregate_sum_grouped_an(capi.Column.void(n), gcol(codes, meta), gcol(gcodes, RESOID), G), ref)
+
+
 @pytest.mark.parametrize("n", SIZES)
 def test_mul_sum_parity(n):
     p = datagen.encode(datagen.uniform(n, 41, 1, 0, 10**6), 65117, 8)

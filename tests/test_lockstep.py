@@ -128,3 +128,41 @@ def test_merge_stops_when_list_1_fails_a_check():
             t1[700] = t1[699] - np.uint64(an.A_OID)
         steps.append(sum(x[3] for x in _merge(t1, lists[1], ws) if "k_stream" in x[0]))
     assert steps[1] * 4 < steps[0]
+
+
+def _sums(n, groups, ws, run=True):
+    rng = np.random.default_rng(n + groups)
+    meas = an.an_meta(an.RESINT, 65117)
+    gi = rng.integers(0, groups, n).astype(np.uint64)
+    t = datagen.encode(rng.integers(0, 1 << 32, n).astype(np.uint64), meas.a, 8)
+    g = gi * np.uint64(an.A_OID)
+    if n > 100:
+        t[[3, 70]] ^= np.uint64(1 << 35)
+        g[[5, n - 1]] = np.uint64(groups) * np.uint64(an.A_OID)
+    sums, cnt, errs = np.full(groups, 77, np.uint64), np.zeros(4, np.uint64), [np.zeros(8, np.uint64) for _ in range(3)]
+    void = L.column(None, an.plain_meta(an.VOID), n)
+    ct, cg = L.column(t, meas), L.column(g, RESOID)
+    L.check(L.lib().ahead_hip_aggregate_sum_grouped_an(
+        ctypes.byref(void), ctypes.byref(ct), ctypes.byref(cg), groups, an.A_RESULT, an.A_OID, sums.ctypes.data,
+        *[L.buf(e) for e in errs], cnt.ctypes.data, ws.h, None))
+    if run:
+        ref = O.aggregate_sum_grouped_an(O.void(n), O.Col(t, meas), O.Col(g, RESOID), groups)
+        got = [sums, *[e[:int(c)] for e, c in zip(errs, cnt[1:])]]
+        for i, (x, y) in enumerate(zip(got, ref)):
+            assert np.array_equal(x, y), i
+
+
+@pytest.mark.parametrize("n,groups", [(0, 7), (1, 1), (2047, 3), (2049, 5), (4097, 4096), (6000, 4097), (5000, 130)])
+def test_grouped_sum_partials(n, groups):
+    """Workgroups without rows leave no partials, and none of another call's are summed."""
+    L.lib().lockstep_set(0, 0, CUS)
+    ws = L.Workspace()
+    _sums(9000, min(groups, 4096), ws, run=False)
+    _sums(n, groups, ws)
+
+
+def test_grouped_sum_partials_follow_the_rows(recorded):
+    n, groups = 250_000, 4096
+    ws = L.Workspace()
+    _sums(n, groups, ws, run=False)
+    assert ws.bytes() < 2 * 8 * groups * (n // 2048 + 1) + (4 << 20)
