@@ -800,14 +800,12 @@ void launch_first(const GrpKey &k, const GrpTable &t, uint32_t *flags, uint32_t 
     const void *fn;
     if constexpr (DIRECT) fn = reinterpret_cast<const void *>(k_grp_first<T>);
     else fn = reinterpret_cast<const void *>(k_grp_first_set<T, BIN>);
-    static const uint32_t resident = [fn] {
-        int dev = 0, cus = 0, per_cu = 0;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-            cus = 256;
+    static ahead_host::PerDevice kept;
+    const uint32_t resident = ahead_host::per_device(kept, [fn] {
+        int per_cu = 0;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, kBlock, 0) != hipSuccess || per_cu <= 0) per_cu = 2;
-        return static_cast<uint32_t>(cus) * static_cast<uint32_t>(per_cu);
-    }();
+        return ahead_host::device_cus() * static_cast<uint32_t>(per_cu);
+    });
     if constexpr (DIRECT) {
         constexpr uint64_t step = 64u * GfTraits<T>::R;
         const uint64_t batches = (n + step - 1) / step;

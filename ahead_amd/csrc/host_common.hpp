@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
 #include <string>
 
 #include "../../include/ahead_hip.h"
@@ -44,6 +45,23 @@ int hip_fail(hipError_t e, const char *what);
 constexpr size_t kHeaderBytes = sizeof(ahead_dev::WsHeader);
 
 inline size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
+
+// What f() says about the current device, asked at the first use there and again while it says 0.
+constexpr int kMaxDevices = 64;
+using PerDevice = std::atomic<uint32_t>[kMaxDevices];
+template <class F>
+uint32_t per_device(PerDevice &kept, F &&f) {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return f();
+    uint32_t v = kept[dev].load(std::memory_order_relaxed);
+    if (v == 0) {
+        v = f();
+        kept[dev].store(v, std::memory_order_relaxed);
+    }
+    return v;
+}
+// CUs of the current device.
+uint32_t device_cus();
 
 // Ensures the scratch allocation holds `bytes` beyond the header.  Growing frees the old
 // allocation (hipFree waits for the device) and zero-fills the new one.

@@ -22,6 +22,17 @@ int hip_fail(hipError_t e, const char *what) {
     return e == hipErrorOutOfMemory ? AHEAD_ERR_NOMEM : AHEAD_ERR_HIP;
 }
 
+uint32_t device_cus() {
+    static PerDevice kept;
+    return per_device(kept, [] {
+        int dev = 0, c = 0;
+        if (hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || c <= 0)
+            c = 256;
+        return static_cast<uint32_t>(c);
+    });
+}
+
 // Grows a zero-filled device allocation of the workspace to at least `need` bytes (by half more than
 // it held); hipFree waits for the device before the old one goes.
 static int grow(ahead_hip_ws *ws, void **mem, size_t *held, size_t need, const char *what) {

@@ -470,10 +470,14 @@ int launch_stream_g(const Op &op, ahead_hip_ws *ws, hipStream_t s, size_t lds, u
     using namespace ahead_dev;
     constexpr uint64_t rows = static_cast<uint64_t>(kStreamThreads) * G;
     if (lds > 0) {
-        static const hipError_t set = hipFuncSetAttribute(reinterpret_cast<const void *>(k_stream<Op, G>),
-                                                          hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                          static_cast<int>(kStreamLds - stream_pack_bytes<Op, G>()));
-        AHEAD_HIP_TRY(set);
+        static PerDevice kept;
+        hipError_t e = hipSuccess;
+        per_device(kept, [&] {
+            e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_stream<Op, G>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    static_cast<int>(kStreamLds - stream_pack_bytes<Op, G>()));
+            return e == hipSuccess ? 1u : 0u;
+        });
+        AHEAD_HIP_TRY(e);
     }
     const uint64_t tiles = op.n == 0 ? 1 : (op.n + rows - 1) / rows;
     const uint32_t grid = static_cast<uint32_t>(tiles < cus ? tiles : cus);
@@ -495,13 +499,7 @@ int launch_stream_g(const Op &op, ahead_hip_ws *ws, hipStream_t s, size_t lds, u
 template <class Op>
 int launch_stream(const Op &op, ahead_hip_ws *ws, hipStream_t s, size_t lds = 0) {
     using namespace ahead_dev;
-    static const uint32_t cus = [] {
-        int dev = 0, c = 0;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || c <= 0)
-            c = 256;
-        return static_cast<uint32_t>(c);
-    }();
+    const uint32_t cus = device_cus();
     // Tiles of fewer rows for calls that leave CUs idle otherwise, or give them one tile each, whose loads,
     // lookups and places then follow one another (see kStreamMidG).
     if constexpr (Op::kG > kStreamSmallG) {

@@ -62,6 +62,7 @@ namespace lockstep {
 enum Op : int { kNone, kBarrier, kBallot, kShfl, kFirst, kRead, kDpp, kSync };
 void launch(const char *name, dim3 grid, dim3 block, const std::function<void()> &kernel);
 uint32_t thread_id();
+void count_cas();
 uint32_t block_id();
 uint32_t block_size();
 uint32_t grid_size();
@@ -174,6 +175,7 @@ inline T atomicMax(T *p, U v) {
 }
 template <class T>
 inline T atomicCAS(T *p, T c, T v) {
+    lockstep::count_cas();
     const T o = *p;
     if (o == c) *p = v;
     return o;

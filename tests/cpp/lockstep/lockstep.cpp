@@ -37,8 +37,10 @@ char *stacks;
 const std::function<void()> *body;
 uint32_t cur, bid, bdim, gdim;
 bool bar_any, bar_out;
+uint64_t swaps;  // compare-and-swaps of the launch
 uint64_t steps;  // wave-wide operations and barriers, summed over the waves, of the launch
-int descending, dry, cus = 4, device;
+int descending, dry, device;
+int cus[2] = {256, 4};  // device 0 is a large card, device 1 a small one
 std::string log_;
 std::vector<std::string> attrs;
 
@@ -115,6 +117,7 @@ void run_block() {
 }  // namespace
 
 uint32_t thread_id() { return cur; }
+void count_cas() { ++swaps; }
 uint32_t block_id() { return bid; }
 uint32_t block_size() { return bdim; }
 uint32_t grid_size() { return gdim; }
@@ -138,9 +141,9 @@ const uint64_t *wave_op(Op op, uint64_t v, uint64_t *on) {
 void launch(const char *name, dim3 grid, dim3 block, const std::function<void()> &kernel) {
     struct Log {
         std::string head;
-        ~Log() { log_ += head + std::to_string(steps) + "\n"; }
+        ~Log() { log_ += head + std::to_string(steps) + " " + std::to_string(swaps) + "\n"; }
     } log{std::string(name) + " " + std::to_string(grid.x) + " " + std::to_string(block.x) + " "};
-    steps = 0;
+    steps = swaps = 0;
     if (dry) return;
     if (block.x > kMost) bad("workgroup too large");
     if (stacks == nullptr) {
@@ -167,8 +170,8 @@ hipError_t hipMemset(void *p, int v, size_t bytes) {
     memset(p, v, bytes);
     return hipSuccess;
 }
-hipError_t hipDeviceGetAttribute(int *v, int, int) {
-    *v = lockstep::cus;
+hipError_t hipDeviceGetAttribute(int *v, int, int dev) {
+    *v = lockstep::cus[dev];
     return hipSuccess;
 }
 hipError_t hipGetDevice(int *dev) {
@@ -185,14 +188,14 @@ hipError_t hipFuncSetAttribute(const void *, int, int) {
 }
 
 extern "C" {
-// Waves in descending order; kernels recorded but not run; the CUs of the card.
-void lockstep_set(int descending, int dry, int cus) {
+// Waves in descending order; kernels recorded but not run; the current device.
+void lockstep_set(int descending, int dry, int device) {
     lockstep::descending = descending;
     lockstep::dry = dry;
-    lockstep::cus = cus;
+    lockstep::device = device;
 }
-void lockstep_device(int device) { lockstep::device = device; }
-// The launches since the last call, one line each: kernel, workgroups, threads, steps run.
+// The launches since the last call, one line each: kernel, workgroups, threads, steps run,
+// compare-and-swaps.
 const char *lockstep_launches(void) {
     static std::string out;
     out.swap(lockstep::log_);

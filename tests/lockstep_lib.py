@@ -7,6 +7,7 @@ import ctypes
 import os
 import subprocess
 from pathlib import Path
+from typing import NamedTuple
 
 import numpy as np
 
@@ -62,7 +63,6 @@ def lib() -> ctypes.CDLL:
                 fn = getattr(L, name)
                 fn.argtypes, fn.restype = args, res
         L.lockstep_set.argtypes = [ctypes.c_int] * 3
-        L.lockstep_device.argtypes = [ctypes.c_int]
         L.lockstep_launches.restype = ctypes.c_char_p
         _lib = L
     return _lib
@@ -85,16 +85,23 @@ class Workspace:
         lib().ahead_hip_ws_destroy(self.h)
 
 
-def launches() -> list[tuple[str, int, int, int]]:
-    """(kernel, workgroups, threads, steps) of every launch since the last call, the steps being the wave-wide
-    operations and barriers its waves went through; ("attribute", device, 0, 0) for each hipFuncSetAttribute."""
+class Launch(NamedTuple):
+    kernel: str
+    grid: int
+    block: int
+    steps: int  # wave-wide operations and barriers its waves went through
+    swaps: int  # compare-and-swaps its lanes made
+
+
+def launches() -> list[Launch]:
+    """Every launch since the last call; ("attribute", device, 0, 0, 0) for each hipFuncSetAttribute."""
     out = []
     for line in lib().lockstep_launches().decode().splitlines():
         if line.startswith("attribute"):
-            out.append(("attribute", int(line.split()[1]), 0, 0))
+            out.append(Launch("attribute", int(line.split()[1]), 0, 0, 0))
         else:
-            name, grid, block, steps = line.rsplit(" ", 3)
-            out.append((name.strip("()"), int(grid), int(block), int(steps)))
+            name, *v = line.rsplit(" ", 4)
+            out.append(Launch(name.strip("()"), *map(int, v)))
     return out
 
 

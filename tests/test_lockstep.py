@@ -12,15 +12,15 @@ from ahead_amd import an, capi, datagen
 pytestmark = pytest.mark.skipif(not L.available(), reason="no clang++ of ROCm to compile the kernels for the CPU")
 
 
-CUS = 256
+CUS = 256  # of device 0; device 1 has 4
 
 
 @pytest.fixture(params=[0, 1], ids=["ascending", "descending"])
 def waves(request):
     lib = L.lib()
-    lib.lockstep_set(request.param, 0, CUS)
+    lib.lockstep_set(request.param, 0, 0)
     yield request.param
-    lib.lockstep_set(0, 0, CUS)
+    lib.lockstep_set(0, 0, 0)
 
 
 @pytest.mark.parametrize("n,bad", [(5, 1), (16 * 1024 * 2 + 77, 3)])
@@ -44,12 +44,12 @@ def test_single_pass_engine_under_uneven_waves(waves, n, bad):
 
 @pytest.fixture
 def recorded():
-    """Launches are recorded, not run, on a card of 256 CUs."""
+    """Launches are recorded, not run."""
     lib = L.lib()
-    lib.lockstep_set(0, 1, CUS)
+    lib.lockstep_set(0, 1, 0)
     L.launches()
     yield lib
-    lib.lockstep_set(0, 0, CUS)
+    lib.lockstep_set(0, 0, 0)
 
 
 def _somewhere(n, meta, **kw):
@@ -89,7 +89,7 @@ def test_single_pass_engine_spreads_a_call_over_the_card(recorded, n):
     for name, call in _calls(n, ws):
         L.launches()
         L.check(call())
-        grids = [x[1] for x in L.launches() if x[0].startswith("k_stream")]
+        grids = [x.grid for x in L.launches() if x.kernel.startswith("k_stream")]
         assert grids, name
         for g in grids:
             assert min(-(-n // 4096), CUS * 3 // 8) <= g <= CUS, (name, n, g)
@@ -117,8 +117,8 @@ def _merge(t1, h2, ws):
 
 def test_merge_stops_when_list_1_fails_a_check():
     """The pass over list 1 ends soon after a row fails; the walk that writes the outputs is not its concern."""
-    n = 200_000
-    L.lib().lockstep_set(0, 0, CUS)
+    n = 60_000
+    L.lib().lockstep_set(0, 0, 0)
     ws, keys = L.Workspace(), np.arange(n, dtype=np.uint64) * np.uint64(3)
     lists = keys * np.uint64(an.A_OID), keys[::2] * np.uint64(an.A_OID)
     steps = []
@@ -126,7 +126,7 @@ def test_merge_stops_when_list_1_fails_a_check():
         t1 = lists[0].copy()
         if bad:
             t1[700] = t1[699] - np.uint64(an.A_OID)
-        steps.append(sum(x[3] for x in _merge(t1, lists[1], ws) if "k_stream" in x[0]))
+        steps.append(sum(x.steps for x in _merge(t1, lists[1], ws) if "k_stream" in x.kernel))
     assert steps[1] * 4 < steps[0]
 
 
@@ -155,7 +155,7 @@ def _sums(n, groups, ws, run=True):
 @pytest.mark.parametrize("n,groups", [(0, 7), (1, 1), (2047, 3), (2049, 5), (4097, 4096), (6000, 4097), (5000, 130)])
 def test_grouped_sum_partials(n, groups):
     """Workgroups without rows leave no partials, and none of another call's are summed."""
-    L.lib().lockstep_set(0, 0, CUS)
+    L.lib().lockstep_set(0, 0, 0)
     ws = L.Workspace()
     _sums(9000, min(groups, 4096), ws, run=False)
     _sums(n, groups, ws)
@@ -166,3 +166,17 @@ def test_grouped_sum_partials_follow_the_rows(recorded):
     ws = L.Workspace()
     _sums(n, groups, ws, run=False)
     assert ws.bytes() < 2 * 8 * groups * (n // 2048 + 1) + (4 << 20)
+
+
+def test_every_device_has_its_own_launch_geometry(recorded):
+    """The LDS attribute and the CUs are the current device's, not those of the first one used."""
+    n = 4_000_000
+    for device, cus, first in ((0, CUS, True), (1, 4, True), (0, CUS, False)):
+        recorded.lockstep_set(0, 1, device)
+        ws, oid, col = L.Workspace(device), _somewhere(n, RESOID), _somewhere(5000, an.an_meta(an.RESINT, 65117))
+        b = capi.Buf(4096, n)
+        L.launches()
+        L.check(recorded.ahead_hip_fetchjoin_an(ctypes.byref(oid), ctypes.byref(col), 0, 0, 1, b, b, b, 4096, ws.h, None))
+        log = L.launches()
+        assert [x.grid for x in log if x.kernel == "attribute"] == [device] * first
+        assert [x.grid for x in log if x.kernel.startswith("k_stream")] == [cus]
