@@ -1120,7 +1120,8 @@ __device__ __forceinline__ V mi_last_lane(V x) {
 }
 
 // List 1, on the single-pass engine: order and validity checks, and the pairs of the rows whose key is set.
-// A failed check sets the path's second flag; the sub-tile kernels then write all outputs (and counts) again.
+// A failed check sets the path's second flag; the sub-tile kernels then write all outputs (and counts) again,
+// and the tiles still to come are skipped.
 // V: keys are compared in 32 bits where every valid key fits (codes of up to 4 bytes, 8-byte codes whose
 // values fit and check by multiplying back, void ranges below 2^32).  VOID1: the keys are seqbase + row (a
 // whole dimension meets a selection of it).  GATHER: the right tails are read from t2 at the keys' rows.
@@ -1131,7 +1132,7 @@ __device__ __forceinline__ V mi_last_lane(V x) {
 // 21 us with 16 rows per lane, 9 with 8 and fixed widths).
 template <typename K, typename V, bool VOID1, bool GATHER, bool W8>
 struct IntersectOp {
-    static constexpr int kErr = 1;  // (no error on this path)
+    static constexpr int kErr = 1;  // rows that fail a check: the path does not apply (failed)
     static constexpr int kG = !W8 ? 4 : sizeof(V) == 8 || VOID1 || GATHER ? 8 : 10;
     static constexpr uint32_t kPack = 64u * kG;  // (8.2M of 30M rows kept: 151 -> 129 us)
     struct RawK {
@@ -1163,7 +1164,8 @@ struct IntersectOp {
         bool any;      // keys of type V reach the bitmap
     };
     __device__ bool skip() const { return mi.ok[0] == 0u || (choose && (mi.ok[2] != 0u) != (sizeof(V) == 8)); }
-    __device__ bool stop() const { return __hip_atomic_load(&mi.ok[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u; }
+    // (a flag of its own: every workgroup of this launch decides to run by ok[0])
+    __device__ void failed() const { mi.ok[1] = 1u; }
     __device__ void init(char *) const {}
     __device__ Uniform begin(const char *) const {
         const uint64_t lo = mi.range[0];
@@ -1238,9 +1240,7 @@ struct IntersectOp {
             if constexpr (GATHER) st[g].j = static_cast<uint32_t>(__popcll(mid.word[g] & ((1ull << b) - 1ull)));
         }
         keep &= live & mid.in;
-        err[0] = 0;
-        // (a flag of its own: every workgroup of this launch decides to run by ok[0])
-        if ((live & mid.bad) != 0u) __hip_atomic_store(&mi.ok[1], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        err[0] = live & mid.bad;
     }
     __device__ void report(uint64_t, State &, uint32_t &) const {}
     __device__ __forceinline__ void emit(const Uniform &u, const State &st, uint64_t first, uint64_t pos, uint32_t row,

@@ -50,8 +50,8 @@
 //   void init(char *lds) const;         // all threads, before the first tile; a barrier follows
 //   bool skip() const;                  // the whole launch stands down (from device state that no
 //                                       // workgroup of this launch changes)
-//   bool stop() const;                  // (optional) nothing this launch writes will be used: read by one thread
-//                                       // with every ticket; the tiles still to come are counted as empty
+//   void failed() const;                // (optional) one thread, for a tile that reports: nothing this launch writes
+//                                       // will be used, and the tiles still to come are counted as empty
 #pragma once
 
 #include "rowtile.hpp"
@@ -74,10 +74,13 @@ struct StreamArgs {
 
 __device__ __forceinline__ uint32_t uniform(uint32_t x) { return __builtin_amdgcn_readfirstlane(x); }
 
-// A ticket word's tile; the holder of the launch's last ticket starts the next epoch.
+// What a failed launch's ticket words carry above the ticket (at most 2^21 tiles and workgroups).
+constexpr uint32_t kStreamFailed = 1u << 31;
+
+// A ticket word's tile, and kStreamFailed; the holder of the launch's last ticket starts the next epoch.
 __device__ __forceinline__ uint32_t stream_tile(const StreamArgs &m, unsigned long long v) {
     const uint32_t t = static_cast<uint32_t>(v);
-    if (t == m.last)
+    if ((t & ~kStreamFailed) == m.last)
         __hip_atomic_store(m.te, ((v >> 32) + 1ull) << 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     return t;
 }
@@ -120,9 +123,20 @@ __device__ __forceinline__ void stream_load(const Op &op, uint64_t first, uint32
 }
 
 template <class Op, class = void>
-struct has_stop : std::false_type {};
+struct can_fail : std::false_type {};
 template <class Op>
-struct has_stop<Op, std::void_t<decltype(std::declval<const Op &>().stop())>> : std::true_type {};
+struct can_fail<Op, std::void_t<decltype(std::declval<const Op &>().failed())>> : std::true_type {};
+
+// The workgroup's tiles from `tile` on, published as empty, so that no other one waits for them (thread 0).
+template <int NS>
+__device__ __forceinline__ void stream_drain(const StreamArgs &m, uint32_t epoch, uint32_t tile) {
+    while (tile < m.tiles) {
+        lb_store(&m.agg[tile], stream_word(epoch, 0));
+#pragma unroll
+        for (int s = 0; s < NS; ++s) lb_store(&m.incl[static_cast<size_t>(s) * m.tiles + tile], stream_word(epoch, 0));
+        tile = stream_tile(m, atomicAdd(m.te, 1ull)) & ~kStreamFailed;
+    }
+}
 
 template <class Op, int G, class = void>
 struct pack_rows : std::integral_constant<uint32_t, 0> {};
@@ -148,7 +162,7 @@ __global__ __launch_bounds__(kStreamThreads) void k_stream(Op op, StreamArgs m) 
     __shared__ uint32_t s_cnt[NS][NW], s_sum[NS][NW];
     // (the first tile has a word of its own: thread 0 stores the second one before the next barrier, when
     // other waves may still have to read the first)
-    __shared__ uint32_t s_begin, s_tile, s_epoch, s_stop;
+    __shared__ uint32_t s_begin, s_tile, s_epoch;
     constexpr uint32_t kPack = pack_rows<Op, G>::value;
     __shared__ StreamPack<Op, G> s_pack[kPack ? NW : 1];
     if (op.skip()) return;
@@ -163,6 +177,12 @@ __global__ __launch_bounds__(kStreamThreads) void k_stream(Op op, StreamArgs m) 
     const uint32_t wave = uniform(threadIdx.x >> 6);
     const uint32_t epoch = uniform(s_epoch);
     uint32_t tile = uniform(s_begin);
+    if constexpr (can_fail<Op>::value) {
+        if ((tile & kStreamFailed) != 0u) {
+            if (threadIdx.x == 0) stream_drain<NS>(m, epoch, tile & ~kStreamFailed);
+            return;
+        }
+    }
     auto first_of = [&](uint32_t t) { return (static_cast<uint64_t>(t) * NW + wave) * kWaveRows; };
     auto left_of = [&](uint32_t t) {
         const uint64_t first = first_of(t);
@@ -177,11 +197,7 @@ __global__ __launch_bounds__(kStreamThreads) void k_stream(Op op, StreamArgs m) 
     }
     while (tile < m.tiles) {
         unsigned long long ticket;  // the next tile's, taken by thread 0 while the inputs arrive
-        bool stop = false;
-        if (threadIdx.x == 0) {
-            ticket = atomicAdd(m.te, 1ull);
-            if constexpr (has_stop<Op>::value) stop = op.stop();
-        }
+        if (threadIdx.x == 0) ticket = atomicAdd(m.te, 1ull);
         const uint64_t first = first_of(tile);
         const uint32_t left = left_of(tile);
         typename Op::State st0[H], st1[H];
@@ -225,10 +241,7 @@ __global__ __launch_bounds__(kStreamThreads) void k_stream(Op op, StreamArgs m) 
 #pragma unroll
             for (int e = 0; e < Op::kErr; ++e) s_cnt[1 + e][wave] = ecnt[e];
         }
-        if (threadIdx.x == 0) {
-            s_tile = stream_tile(m, ticket);
-            if constexpr (has_stop<Op>::value) s_stop = stop ? 1u : 0u;
-        }
+        if (threadIdx.x == 0) s_tile = stream_tile(m, ticket);
         __syncthreads();
         uint32_t agg[NS], before[NS], rep = 0;
 #pragma unroll
@@ -255,8 +268,14 @@ __global__ __launch_bounds__(kStreamThreads) void k_stream(Op op, StreamArgs m) 
             }
             lb_store(&m.agg[tile], stream_word(epoch, (rep != 0u ? 1ull << 33 : 0ull) | agg[0]));
         }
-        const uint32_t next = uniform(s_tile);
-        if constexpr (has_stop<Op>::value) stop = uniform(s_stop) != 0u;
+        const uint32_t drawn = uniform(s_tile), next = can_fail<Op>::value ? drawn & ~kStreamFailed : drawn;
+        if constexpr (can_fail<Op>::value) {
+            // (before the workgroup's last ticket, and so before the next launch's first one)
+            if (rep != 0u && threadIdx.x == 0) {
+                op.failed();
+                if (next < m.tiles) atomicOr(m.te, static_cast<unsigned long long>(kStreamFailed));
+            }
+        }
         if (next < m.tiles) {
             stream_load<Op, H>(op, first_of(next), lane, left_of(next), 0, raw0);
             stream_load<Op, H>(op, first_of(next), lane, left_of(next), 1, raw1);
@@ -370,14 +389,9 @@ __global__ __launch_bounds__(kStreamThreads) void k_stream(Op op, StreamArgs m) 
             op.finish(totals);
         }
         tile = next;
-        if constexpr (has_stop<Op>::value) {
-            if (stop) {  // the workgroup's further tiles: empty, so that no other one waits for them
-                while (threadIdx.x == 0 && tile < m.tiles) {
-                    lb_store(&m.agg[tile], stream_word(epoch, 0));
-#pragma unroll
-                    for (int s = 0; s < NS; ++s) lb_store(&m.incl[static_cast<size_t>(s) * m.tiles + tile], stream_word(epoch, 0));
-                    tile = stream_tile(m, atomicAdd(m.te, 1ull));
-                }
+        if constexpr (can_fail<Op>::value) {
+            if ((drawn & kStreamFailed) != 0u) {
+                if (threadIdx.x == 0) stream_drain<NS>(m, epoch, tile);
                 return;
             }
         }
