@@ -37,8 +37,13 @@ constexpr uint32_t kDictSlots = 1u << kDictBits;  // at most half full; slot kDi
 constexpr uint32_t kGsBits = 11;
 constexpr uint32_t kGsSlots = 1u << kGsBits;  // key set of a k_grp_first_set workgroup (key + 1, 0 = free)
 constexpr uint32_t kGsFill = kGsSlots / 4 * 3;  // keys it takes; rows of further keys go to the HBM table
-constexpr uint64_t kGsRows = 8192;            // rows of a workgroup, at least (its set costs 3 us)
-constexpr uint32_t kGsPerCu = 3;              // workgroups per CU (of 256): each publishes every key it met
+// Rows of a workgroup, at least, and workgroups per CU (of 256).  A workgroup publishes every key it met, so
+// few keys ask for few workgroups; many keys are inserted in the HBM table one by one, at its latency, and
+// ask for all that fit.  us for 8192 rows and 3 a CU / 2048 and 5: 12M binary keys, 35 groups 86 / 91;
+// 500,000 8-byte keys, 100,000 distinct 502 / 202, ascending 159 / 104; 4M keys, 1.3M distinct ascending
+// 631 / 396; 30M keys, 100,000 distinct 4300 / 3460.
+constexpr uint64_t kGsRows = 2048;
+constexpr uint32_t kGsPerCu = 5;
 constexpr uint32_t kGfDirectWords = 2048;     // bitmap set of unary keys below 2^16 (one bit a key)
 constexpr uint32_t kDirectKeys = 1024;        // AssignOp's LDS table indexed by the key: keys below 2^10
 // flags: [0] table overflow, [8] distinct keys claimed, [9] more than kGrpFastMax (compaction path)
@@ -304,7 +309,8 @@ __global__ __launch_bounds__(kBlock) void k_grp_first(GrpKey k, GrpTable t, uint
 // All other keys.  A workgroup's set holds key + 1 and the smallest row of every key it has met.  A row
 // reads its key's home slot and first row and is done when the key is there with an earlier row; the
 // few others (new keys, keys past their home slot, rows of a key's first batch) probe and insert with
-// LDS atomics, every lane for itself.  The set it replaced belonged to a wave, which listed its new
+// LDS atomics, every lane for itself; a key in several of a lane's rows once, which also spares columns in
+// key order an insert in HBM for every row once the set takes no more keys.  The set it replaced belonged to a wave, which listed its new
 // keys one after another: 35 keys in each of 8192 waves took longer than their rows.  12M binary keys,
 // 35 groups: 65 us before, 27 now (145 while the whole table was walked to publish it).
 template <class T, bool BIN>
@@ -368,6 +374,9 @@ __global__ __launch_bounds__(kBlock) void k_grp_first_set(GrpKey k, GrpTable t, 
             uint64_t kj = key[0];
 #pragma unroll
             for (int i = 1; i < R; ++i) kj = j == static_cast<uint32_t>(i) ? key[i] : kj;
+            // (the lane's later rows of the key have nothing to add)
+#pragma unroll
+            for (int i = 1; i < R; ++i) pend &= key[i] == kj ? ~(1u << i) : ~0u;
             const unsigned long long word = kj == ~0ull ? 1ull : kj + 1ull;
             uint32_t s = kj == ~0ull ? kGsSlots : gs_slot(kj);
             bool in = false;

@@ -180,3 +180,40 @@ def test_every_device_has_its_own_launch_geometry(recorded):
         log = L.launches()
         assert [x.grid for x in log if x.kernel == "attribute"] == [device] * first
         assert [x.grid for x in log if x.kernel.startswith("k_stream")] == [cus]
+
+
+def _group(codes, meta, ws, groups):
+    n = codes.size
+    out, first, cnt = np.zeros(n, np.uint64), np.zeros(groups, np.uint64), np.zeros(6, np.uint64)
+    errs = [np.zeros(4, np.uint64) for _ in range(2)]
+    void, col = L.column(None, an.plain_meta(an.VOID), n), L.column(codes, meta)
+    L.launches()
+    L.check(L.lib().ahead_hip_groupby_an(ctypes.byref(void), ctypes.byref(col), an.A_OID, 0, out.ctypes.data, L.buf(first),
+                                         *[L.buf(e) for e in errs], cnt.ctypes.data, ws.h, None))
+    ref = O.groupby_an(O.void(n), O.Col(codes, meta))
+    assert cnt.tolist() == [n, ref[1].size, 0, 0, 0, 0]
+    assert np.array_equal(out, ref[0]) and np.array_equal(first[:ref[1].size], ref[1])
+    return [x for x in L.launches() if x.kernel.startswith("k_grp_first_set")]
+
+
+def test_group_keys_in_order_are_inserted_once_per_lane():
+    """A workgroup whose set is full inserts a key of a lane's eight rows once, not for every row."""
+    meta = an.an_meta(an.RESINT, 65117)
+    L.lib().lockstep_set(0, 0, 1)  # few workgroups, so that each meets more keys than its set takes
+    ws = L.Workspace(1)
+    n = 16 * 8192
+    keys = (np.arange(n, dtype=np.uint64) // np.uint64(8)) * np.uint64(7) + np.uint64(1 << 20)
+    (run,) = _group(keys * np.uint64(meta.a), meta, ws, n)
+    assert n // run.grid > 8 * 1792  # more keys than the set's 1536
+    assert run.swaps < 3 * (n // 8), run
+    L.lib().lockstep_set(0, 0, 0)
+
+
+@pytest.mark.parametrize("n", [100_000, 500_000, 2_000_000])
+def test_first_sightings_spread_over_the_card(recorded, n):
+    ws, void = L.Workspace(), L.column(None, an.plain_meta(an.VOID), n)
+    col, b = _somewhere(n, an.an_meta(an.RESINT, 65117)), capi.Buf(4096, n)
+    L.launches()
+    L.check(recorded.ahead_hip_groupby_an(ctypes.byref(void), ctypes.byref(col), an.A_OID, 0, 4096, b, b, b, 4096, ws.h, None))
+    (run,) = [x for x in L.launches() if x.kernel.startswith("k_grp_first_set")]
+    assert run.grid >= min(2 * CUS, n // 2048) // 2
