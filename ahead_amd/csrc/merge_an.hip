@@ -841,10 +841,11 @@ __global__ __launch_bounds__(kMmThreads) void k_mm_move(MergeArgs a) {
 
 
 // ---- the intersection path -------------------------------------------------------------------
-// When both key lists are strictly ascending in decoded value and every code of h1, t1, h2 and t2
-// is valid, no check of the walk fails and each list-1 key meets at most one list-2 key: the
-// walk's output is the sorted intersection, (h1[i], t2[j]) for every t1[i] == h2[j] in ascending
-// i, with empty error vectors.  Such inputs take streaming passes instead of the sub-tile walk:
+// When list 2 is strictly ascending in decoded value, list 1 ascending, and every code of h1, t1, h2
+// and t2 is valid, no check of the walk fails and each list-2 key is met by the first list-1 row that
+// holds it (a match advances both cursors; further rows of the key are skipped): the walk's output is
+// the sorted intersection, (h1[i], t2[j]) for every such i with t1[i] == h2[j] in ascending i, with
+// empty error vectors.  Such inputs take streaming passes instead of the sub-tile walk:
 //  k_mi_clear  list 2's first and last keys give the key range [lo2, hi2] (the path applies when
 //              it spans at most kMiBitsPerRow bits per list-2 row), whose bitmap words it clears;
 //  k_mi_build  a bitmap of list 2's keys over the range (bit k - lo2) and, when the pairs' tails
@@ -853,7 +854,7 @@ __global__ __launch_bounds__(kMmThreads) void k_mm_move(MergeArgs a) {
 //  k_mi_tails  the words the build waves share, ORed in;
 //  IntersectOp on the single-pass engine (stream.hpp): the pairs of list 1's rows whose key is set.
 // Both passes check the conditions on every row they read (valid codes, each key above the one
-// before it); after a failure the sub-tile kernels, which otherwise return, write all outputs.
+// before it, in list 1 not below it); after a failure the sub-tile kernels, which otherwise return, write all outputs.
 constexpr uint64_t kMiBitsPerRow = 16;
 constexpr uint64_t kMiWordsMax = 1ull << 26;  // a key's bit number fits 32 bits: all 32-bit OIDs
 constexpr uint32_t kMiNone = 0xFFFFFFFFu;  // no bitmap word
@@ -1119,7 +1120,8 @@ __device__ __forceinline__ V mi_last_lane(V x) {
     else return static_cast<V>(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(x >> 32), 63))) << 32 | lo;
 }
 
-// List 1, on the single-pass engine: order and validity checks, and the pairs of the rows whose key is set.
+// List 1, on the single-pass engine: order and validity checks, and the pairs of the rows whose key is set
+// and not the row before's (30M x 15M OIDs with a repeated key: 503 us as a walk of sub-tiles, 190 so).
 // A failed check sets the path's second flag; the sub-tile kernels then write all outputs (and counts) again,
 // and the tiles still to come are skipped.
 // V: keys are compared in 32 bits where every valid key fits (codes of up to 4 bytes, 8-byte codes whose
@@ -1213,12 +1215,26 @@ struct IntersectOp {
         V edge = 0;
         const bool has = first > 0 && first - 1 < n;
         if (has) edge = static_cast<V>(a.t1.dec_of(a.t1.raw(first - 1)));
+        const V edge0 = edge;
+        uint32_t low = 0;  // keys not above the one before
 #pragma unroll
         for (int g = 0; g < G; ++g) {
             const V prev = mi_lane_below(mid.v[g], edge);
             const bool check = g > 0 || lane != 0u || has;
-            mid.bad |= (check && !(prev < mid.v[g]) ? 1u : 0u) << g;
+            low |= (check && !(prev < mid.v[g]) ? 1u : 0u) << g;
             edge = mi_last_lane(mid.v[g]);
+        }
+        // A key equal to the one before it has no partner: the walk advances both lists on a match, and list 2
+        // has the key once.  A key below the one before fails.
+        if (__ballot((low & live) != 0u) != 0ull) {
+            mid.in &= ~low;
+            edge = edge0;
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                const V prev = mi_lane_below(mid.v[g], edge);
+                mid.bad |= ((low >> g) & 1u) != 0u && prev > mid.v[g] ? 1u << g : 0u;
+                edge = mi_last_lane(mid.v[g]);
+            }
         }
         if (chk_h1) {
 #pragma unroll

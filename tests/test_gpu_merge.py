@@ -288,3 +288,55 @@ def test_merge_list1_tile_edges(n1, void1):
             for codes, meta in ((oid_list(k1, seed, 5), RESOID), (datagen.encode(k1, 32417, 8), m_int)):
                 both(capi.Column.from_numpy(h1, RESOID), capi.Column.from_numpy(codes, meta), right,
                      O.Col(h1, RESOID), O.Col(codes, meta))
+
+
+def _pairs_of_repeats(k1, k2):
+    """Rows of list 1 that pair: the first one of each key that list 2 holds."""
+    return np.isin(k1, k2) & np.concatenate([[True], k1[1:] != k1[:-1]]) if k1.size else np.zeros(0, bool)
+
+
+@pytest.mark.parametrize("n1,runs", [(2, 2), (130, 64), (1500, 70), (4097, 3), (8193, 900), (20_000, 1), (300_001, 2),
+                                     (1_000_003, 40)])
+def test_merge_repeated_keys_in_list1(n1, runs):
+    """List 1 ascending with runs of equal keys (across lanes, halves, waves and tiles), list 2 strictly so: the
+    first row of a key pairs.  One row out of order, or an invalid code, after them: the walk's result."""
+    rng = np.random.default_rng(n1 + runs)
+    k1 = np.repeat(np.arange(n1, dtype=np.uint64) * 2, rng.integers(1, runs + 1, n1))[:n1] + np.uint64(3)
+    k2 = np.unique(np.concatenate([rng.choice(np.unique(k1), max(1, np.unique(k1).size // 2)),
+                                   rng.integers(3, int(k1[-1]) + 9, n1 // 4 + 1).astype(np.uint64)]))
+    t1, h2 = oid_list(k1, 9, 1), oid_list(k2, 9, 2)
+    h1, t2 = oid_list(np.arange(n1, dtype=np.uint64), 9, 3), oid_list(np.arange(k2.size, dtype=np.uint64), 9, 4)
+    ref = run_both(h1, t1, h2, t2, RESOID, RESOID, RESOID, RESOID)
+    assert ref[0].size == _pairs_of_repeats(k1, k2).sum() and all(x.size == 0 for x in ref[2:])
+    run_both(t1, t1, h2, h2, RESOID, RESOID, RESOID, RESOID)
+    if n1 < 20_001:  # (a walk of its own from there on)
+        t1[n1 // 2] = t1[0]
+        h1[n1 - 1] ^= np.uint64(4)
+        run_both(h1, t1, h2, t2, RESOID, RESOID, RESOID, RESOID)
+
+
+@pytest.mark.parametrize("base", [0, (1 << 32) - 40_000, (1 << 32) - 1, 1 << 32, 1 << 45])
+@pytest.mark.parametrize("kind", ["resoid", "resbigint", "bigint"])
+def test_merge_keys_past_32_bits(base, kind):
+    """Ascending keys below, across and above 2^32, in codes whose A does and does not fit 32 bits, plain ones
+    too; repeated and corrupt ones among them."""
+    rng = np.random.default_rng(base % 1000 + len(kind))
+    a = {"resoid": an.A_OID, "resbigint": 32417, "bigint": 1}[kind]
+    t = {"resoid": an.RESOID, "resbigint": an.RESBIGINT, "bigint": an.BIGINT}[kind]
+    meta = an.an_meta(t, a) if t.encoded else an.plain_meta(t)
+    k1 = np.uint64(base) + np.unique(rng.integers(0, 90_000, 30_000)).astype(np.uint64)
+    k2 = np.uint64(base) + np.unique(rng.integers(0, 90_000, 20_000)).astype(np.uint64)
+
+    def codes(k):
+        with np.errstate(over="ignore"):
+            return k * np.uint64(a)
+    h1, t2 = oid_list(np.arange(k1.size, dtype=np.uint64), 3, 1), oid_list(np.arange(k2.size, dtype=np.uint64), 3, 2)
+    ref = run_both(h1, codes(k1), codes(k2), t2, RESOID, meta, meta, RESOID)
+    assert ref[0].size == np.intersect1d(k1, k2).size
+    run_both(codes(k1), codes(k1), codes(k2), codes(k2), meta, meta, meta, meta)
+    k1[5000:5003] = k1[5000]
+    run_both(h1, codes(k1), codes(k2), t2, RESOID, meta, meta, RESOID)
+    if t.encoded:
+        c1 = codes(k1)
+        c1[7000] ^= np.uint64(1 << 50)
+        run_both(h1, c1, codes(k2), t2, RESOID, meta, meta, RESOID)
