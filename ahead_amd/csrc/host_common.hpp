@@ -72,9 +72,13 @@ int ws_ensure(ahead_hip_ws *ws, size_t bytes);
 int ws_ensure_status(ahead_hip_ws *ws, size_t bytes);
 
 // The single-pass engine's ticket word and `bytes` of status words.  The allocation is cleared when
-// it grows, and by a fill kernel on the stream before its 30-bit epoch could repeat.
+// it grows, and by a fill kernel on the stream before its 30-bit epoch could repeat, counting the launches
+// that come through here: replays of a captured one advance the epoch uncounted (2^29 of them, at 8 us each
+// more than an hour of nothing else, are the caller's to count).
 int stream_state(ahead_hip_ws *ws, size_t bytes, hipStream_t s, unsigned long long **te, uint64_t **status);
 constexpr size_t kStreamHeader = 256;
+// Its status words at most: 2^32 rows in tiles of 8192 rows with three error streams, or of 4096 with one.
+constexpr size_t kStreamMost = 32u << 20;
 
 // Next look-back epoch (1 .. 2^30-1).  On wrap-around the status allocation is cleared.
 int ws_next_epoch(ahead_hip_ws *ws, uint32_t *epoch);

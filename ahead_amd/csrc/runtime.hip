@@ -221,7 +221,7 @@ int ahead_hip_ws_destroy(ahead_hip_ws *ws) {
 int ahead_hip_ws_reserve(ahead_hip_ws *ws, size_t bytes) {
     int st = ws_ensure(ws, bytes);
     if (st == AHEAD_OK) st = ws_ensure_status(ws, bytes);
-    if (st == AHEAD_OK) st = ws_ensure_stream(ws, bytes);
+    if (st == AHEAD_OK) st = ws_ensure_stream(ws, bytes < kStreamMost ? bytes : kStreamMost);
     return st;
 }
 

@@ -513,6 +513,8 @@ int launch_stream_g(const Op &op, ahead_hip_ws *ws, hipStream_t s, size_t lds, u
 template <class Op>
 int launch_stream(const Op &op, ahead_hip_ws *ws, hipStream_t s, size_t lds = 0) {
     using namespace ahead_dev;
+    static_assert(((1ull << 32) / (kStreamThreads * Op::kG)) * (2 + 2 * Op::kErr) * 8 <= kStreamMost,
+                  "the status words of the largest call");
     const uint32_t cus = device_cus();
     // Tiles of fewer rows for calls that leave CUs idle otherwise, or give them one tile each, whose loads,
     // lookups and places then follow one another (see kStreamMidG).

@@ -75,10 +75,12 @@ const char *ahead_hip_version(void);
 int ahead_hip_ws_create(int device, ahead_hip_ws **ws);
 int ahead_hip_ws_destroy(ahead_hip_ws *ws);
 /* Grows the workspace now (so later calls do not allocate, e.g. under stream capture): its
- * scratch to at least `bytes` and its scan-state area to at least `bytes` too.  A reservation
- * covers every call whose scratch plus scan state fits in `bytes`. */
+ * scratch to at least `bytes`, its look-back state to at least `bytes` and its ticketed scan state
+ * (the operators that write each output entry once, at most 32 MiB for any call) to at least
+ * min(`bytes`, 32 MiB).  A reservation covers every call whose scratch and scan states each fit
+ * in `bytes`. */
 int ahead_hip_ws_reserve(ahead_hip_ws *ws, size_t bytes);
-/* Device bytes the workspace holds (scratch + scan state). */
+/* Device bytes the workspace holds (scratch + both scan states). */
 size_t ahead_hip_ws_bytes(const ahead_hip_ws *ws);
 
 /* Tiling of the streaming operators: a look-back tile covers up to `max_subtiles` sub-tiles of
@@ -251,7 +253,9 @@ int ahead_hip_groupby2_an(const ahead_col *head, const ahead_col *tail, const ah
 /* aggregate_sum_groupedAN (OperatorsAN.hpp:125-134; aggregateAN.tcc:41-119): sums[g] =
  * sum of tail codes * (a_result * inv(A_tail)) mod 2^64 over rows with a valid group id
  * (corrupt tails are added and reported).  A decoded group id above maxU or >= num_groups is
- * reported in e_group and skipped.  d_counts[0..3] = num_groups, #e_head, #e_tail, #e_group. */
+ * reported in e_group and skipped.  d_counts[0..3] = num_groups, #e_head, #e_tail, #e_group.
+ * Workspace for up to 4096 groups: 8 bytes per group and workgroup (one per 2048 rows, at most as
+ * many as the device holds at once: 42 MB for 4096 groups on an MI355X).                       */
 int ahead_hip_aggregate_sum_grouped_an(const ahead_col *head, const ahead_col *tail,
                                        const ahead_col *grouping, uint64_t num_groups,
                                        uint64_t a_result, uint64_t a_oid, uint64_t *sums,

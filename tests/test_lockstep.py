@@ -217,3 +217,14 @@ def test_first_sightings_spread_over_the_card(recorded, n):
     L.check(recorded.ahead_hip_groupby_an(ctypes.byref(void), ctypes.byref(col), an.A_OID, 0, 4096, b, b, b, 4096, ws.h, None))
     (run,) = [x for x in L.launches() if x.kernel.startswith("k_grp_first_set")]
     assert run.grid >= min(2 * CUS, n // 2048) // 2
+
+
+def test_reserve_sets_the_ticketed_state_apart_once():
+    """A reservation sizes the scratch and the look-back state; the ticketed state is never needed beyond 32 MiB."""
+    L.lib().lockstep_set(0, 0, 0)
+    ws, size = L.Workspace(), 160 << 20
+    L.check(L.lib().ahead_hip_ws_reserve(ws.h, size))
+    assert 2 * size + (32 << 20) <= ws.bytes() < 2 * size + (33 << 20)
+    small = L.Workspace()
+    L.check(L.lib().ahead_hip_ws_reserve(small.h, 5 << 20))
+    assert small.bytes() >= 3 * (5 << 20)
