@@ -1135,7 +1135,7 @@ __device__ __forceinline__ V mi_last_lane(V x) {
 template <typename K, typename V, bool VOID1, bool GATHER, bool W8>
 struct IntersectOp {
     static constexpr int kErr = 1;  // rows that fail a check: the path does not apply (failed)
-    static constexpr int kG = !W8 ? 4 : sizeof(V) == 8 || VOID1 || GATHER ? 8 : 10;
+    static constexpr int kG = !W8 || sizeof(V) == 8 || VOID1 || GATHER ? 8 : 10;
     static constexpr uint32_t kPack = 64u * kG;  // (8.2M of 30M rows kept: 151 -> 129 us)
     struct RawK {
         K c;
