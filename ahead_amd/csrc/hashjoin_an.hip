@@ -472,10 +472,74 @@ __device__ __forceinline__ uint64_t reencode(uint64_t v, uint64_t f) {
 }
 
 // The probe on the single-pass engine: when no build key has several rows, a probe row emits at most one
-// pair.
+// pair, and the build payload is gathered with the other lookups.
+struct ProbeOneState {
+    uint64_t pay, bpay;
+};
 struct ProbeOneOp : ProbeOp {
     static constexpr bool kMulti = false;
+    using State = ProbeOneState;
     __device__ bool skip() const { return t.flags[0] != 0u; }
+    __device__ const DCol &first_col() const { return phead; }
+    __device__ const DCol &second_col() const { return ptail; }
+    template <int G>
+    __device__ __forceinline__ void eval_codes(const bool (&live)[G], const uint64_t (&h)[G], const uint64_t (&tl)[G], State (&st)[G],
+                                               uint32_t (&errs)[G], bool (&keep)[G]) const {
+        uint64_t k[G], b[G];
+        uint64_t brow[G];
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            errs[g] = (phead.bad_of(h[g]) ? 1u : 0u) | (ptail.bad_of(tl[g]) ? 2u : 0u);
+            const uint64_t kv = key.dec_of(build_right ? tl[g] : h[g]);
+            st[g].pay = build_right ? h[g] : tl[g];
+            keep[g] = live[g] && (kv & guard_mask) <= build_max;
+            k[g] = kv & key_mask;
+        }
+        if (t.flags[4] != 0u) {  // direct map (one row per key: no flag bit)
+            const uint64_t lo = t.flags[3], span = t.flags[5] - t.flags[3];
+            uint32_t e[G];
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                const uint64_t rel = k[g] - lo;
+                keep[g] = keep[g] && rel <= span;
+                e[g] = t.dmap[keep[g] ? rel : 0ull];
+            }
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                keep[g] = keep[g] && e[g] != 0u;
+                brow[g] = e[g] - 1u;
+            }
+        } else {
+            uint32_t sl[G], f[G];
+            t.ht.find_n<G>(k, keep, sl);
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                keep[g] = keep[g] && sl[g] != UINT32_MAX;
+                f[g] = t.first[keep[g] ? sl[g] : 0u];
+            }
+#pragma unroll
+            for (int g = 0; g < G; ++g) brow[g] = f[g];
+        }
+        bpay.raw_n<G>(brow, keep, b);
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            st[g].pay = reenc_p ? (st[g].pay * f_p) & m_p : st[g].pay;
+            st[g].bpay = reenc_b ? (b[g] * f_b) & m_b : b[g];
+        }
+    }
+    // (the error streams of a row)
+    __device__ uint32_t eval(uint64_t row, State &, uint32_t &errs, uint64_t &) const {
+        if (phead.bad_of(phead.raw(row))) errs |= 1u;
+        if (ptail.bad_of(ptail.raw(row))) errs |= 2u;
+        return 0;
+    }
+    __device__ void emit_main(uint64_t, const State &st, uint64_t pos, uint32_t) const {
+        store_w(build_right ? out_h : out_t, pos, w_p, st.pay);
+        store_w(build_right ? out_t : out_h, pos, w_b, st.bpay);
+    }
+    __device__ void emit_err(int e, uint64_t row, const State &, uint64_t pos) const {
+        if (pos < cap[e]) err[e][pos] = row * a_oid;
+    }
 };
 
 // The probe for its common shapes, on the single-pass engine: every build key has one row, the probe

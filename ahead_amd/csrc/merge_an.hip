@@ -1130,8 +1130,8 @@ __device__ __forceinline__ V mi_last_lane(V x) {
 // Two ascending lists of 30.0M and 16.4M 8-byte OIDs, 8.2M matches: a count, a scan and a write pass over
 // list 1 took 184 us together, this pass 129.
 // W8: both outputs are 8 bytes wide; a run-time width makes eight stores of each row's two, so much code
-// that a small call waits for its instructions, and takes fewer rows per lane (one tile of 2,556 void rows:
-// 21 us with 16 rows per lane, 9 with 8 and fixed widths).
+// that a small call waits for its instructions (one tile of 2,556 void rows: 21 us with 16 rows per lane, 9
+// with 8 and fixed widths).
 template <typename K, typename V, bool VOID1, bool GATHER, bool W8>
 struct IntersectOp {
     static constexpr int kErr = 1;  // rows that fail a check: the path does not apply (failed)

@@ -387,14 +387,13 @@ struct MatchPosOp {
     uint64_t cap[3];
     uint64_t *d_counts;
 
-    static constexpr bool kBatched = true;
+    __device__ const DCol &first_col() const { return h1; }
+    __device__ const DCol &second_col() const { return t1; }
     template <int G>
-    __device__ void eval_n(const uint64_t (&row)[G], const bool (&live)[G], State (&st)[G], uint32_t (&errs)[G],
-                           uint32_t (&cnt)[G], uint64_t &) const {
-        uint64_t h[G], o[G], p2[G], v[G];
+    __device__ __forceinline__ void eval_codes(const bool (&live)[G], const uint64_t (&h)[G], const uint64_t (&o)[G], State (&st)[G],
+                                               uint32_t (&errs)[G], bool (&keep)[G]) const {
+        uint64_t p2[G], v[G];
         bool in[G];
-        h1.raw_n<G>(row, live, h);
-        t1.raw_n<G>(row, live, o);
 #pragma unroll
         for (int g = 0; g < G; ++g) {
             p2[g] = o[g] * t1.a_inv;
@@ -403,22 +402,11 @@ struct MatchPosOp {
         t2.raw_n<G>(p2, in, v);
 #pragma unroll
         for (int g = 0; g < G; ++g) {
-            errs[g] = 0;
-            cnt[g] = 0;
-            if (!live[g]) continue;
-            if (h1.bad_of(h[g])) errs[g] |= 1u;
+            const bool bad = t2.bad_of(v[g]);
+            errs[g] = (h1.bad_of(h[g]) ? 1u : 0u) | (!in[g] ? 2u : bad ? 4u : 0u);
+            keep[g] = in[g] && !bad;
             st[g].h = reenc_h ? (h[g] * f_h1) & mh : h[g];
-            if (!in[g]) {
-                errs[g] |= 2u;
-                continue;
-            }
-            if (t2.bad_of(v[g])) {
-                errs[g] |= 4u;
-                st[g].v = p2[g];
-                continue;
-            }
             st[g].v = reenc_t ? (v[g] * f_t2) & mt : v[g];
-            cnt[g] = 1;
         }
     }
 

@@ -34,7 +34,8 @@
 //   struct Raw; using State;            // a row's streamed inputs; what its entry needs
 //   uint64_t out_cap;                   // entries the outputs hold
 //   struct Uniform; Uniform begin(const char *lds) const;      // read once per workgroup, after init
-//   void load(uint64_t first, uint32_t k, Raw &) const;        // row first + k
+//   void load(uint64_t first, uint32_t k, Raw &) const;        // row first + k; or, with kLoadN, H rows at once:
+//   template <int H> void load_n(uint64_t first, const uint32_t (&k)[H], Raw (&)[H]) const;
 //   template <int G> void open_tile(const char *lds, const Uniform &, uint64_t first, uint32_t lane,
 //            uint32_t live, const Raw (&)[G], Mid<G> &) const;
 //       // rows first + 64 g + lane: decodes them and issues their lookups (bit g of live: the row
@@ -108,6 +109,11 @@ __device__ __forceinline__ uint32_t wave_rank(uint64_t ballot) {
                                      __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(ballot), 0u));
 }
 
+template <class Op, class = void>
+struct loads_halves : std::false_type {};
+template <class Op>
+struct loads_halves<Op, std::void_t<decltype(Op::kLoadN)>> : std::true_type {};
+
 // The streamed inputs of a lane's G rows first + 64 g + lane, of which the wave has `left`; rows past
 // the end repeat the last one (a wave past the end: row 0).
 template <class Op, int H>
@@ -115,10 +121,17 @@ __device__ __forceinline__ void stream_load(const Op &op, uint64_t first, uint32
                                             typename Op::Raw (&raw)[H]) {
     const uint64_t base = left != 0u ? first : 0ull;
     const uint32_t top = left != 0u ? left - 1u : 0u;
+    uint32_t k[H];
 #pragma unroll
     for (int g = 0; g < H; ++g) {
-        const uint32_t k = static_cast<uint32_t>((half * H + g) * 64) + lane;
-        op.load(base, k < top ? k : top, raw[g]);
+        k[g] = static_cast<uint32_t>((half * H + g) * 64) + lane;
+        k[g] = k[g] < top ? k[g] : top;
+    }
+    if constexpr (loads_halves<Op>::value) {
+        op.template load_n<H>(base, k, raw);
+    } else {
+#pragma unroll
+        for (int g = 0; g < H; ++g) op.load(base, k[g], raw[g]);
     }
 }
 
@@ -398,12 +411,18 @@ __global__ __launch_bounds__(kStreamThreads) void k_stream(Op op, StreamArgs m) 
     }
 }
 
-// An operator of the row-tile interface (at most one entry per row, eval_n) on this engine: the rows
-// are loaded when they are evaluated, not a tile ahead.
+// An operator over columns of any width (at most one entry per row) on this engine.  Beside the row-tile
+// interface it has two streamed columns and the evaluation of rows whose codes are there:
+//   DCol first_col() const, second_col() const;
+//   template <int G> void eval_codes(const bool (&live)[G], const uint64_t (&c1)[G], const uint64_t (&c2)[G], State (&)[G],
+//                                    uint32_t (&errs)[G], bool (&keep)[G]) const;
 template <class Op>
 struct StreamRows : Op {
     static constexpr int kErr = Op::kErr, kG = 8;
-    struct Raw {};
+    static constexpr bool kLoadN = true;
+    struct Raw {
+        uint64_t c1, c2;
+    };
     using State = typename Op::State;
     StreamRows() = default;
     explicit StreamRows(const Op &op) : Op(op) {}
@@ -414,30 +433,44 @@ struct StreamRows : Op {
     struct Uniform {};
     __device__ void init(char *) const {}
     __device__ Uniform begin(const char *) const { return Uniform{}; }
-    __device__ __forceinline__ void load(uint64_t, uint32_t, Raw &) const {}
+    template <int H>
+    __device__ __forceinline__ void load_n(uint64_t first, const uint32_t (&k)[H], Raw (&raw)[H]) const {
+        uint64_t rows[H], c1[H], c2[H];
+        bool on[H];
+#pragma unroll
+        for (int g = 0; g < H; ++g) {
+            rows[g] = first + k[g];
+            on[g] = true;
+        }
+        Op::first_col().template raw_n<H>(rows, on, c1);
+        Op::second_col().template raw_n<H>(rows, on, c2);
+#pragma unroll
+        for (int g = 0; g < H; ++g) raw[g] = Raw{c1[g], c2[g]};
+    }
     template <int G>
     struct Mid {
         State st[G];
         uint32_t keep, err[kErr];
     };
     template <int G>
-    __device__ __forceinline__ void open_tile(const char *, const Uniform &, uint64_t first, uint32_t lane, uint32_t live,
-                                              const Raw (&)[G], Mid<G> &mid) const {
-        uint64_t rows[G], acc = 0;
-        bool on[G];
-        uint32_t errs[G], cnt[G];
+    __device__ __forceinline__ void open_tile(const char *, const Uniform &, uint64_t, uint32_t, uint32_t live, const Raw (&raw)[G],
+                                              Mid<G> &mid) const {
+        uint64_t c1[G], c2[G];
+        bool on[G], keep[G];
+        uint32_t errs[G];
 #pragma unroll
         for (int g = 0; g < G; ++g) {
-            rows[g] = first + static_cast<uint32_t>(g * 64) + lane;
+            c1[g] = raw[g].c1;
+            c2[g] = raw[g].c2;
             on[g] = (live >> g) & 1u;
         }
-        Op::template eval_n<G>(rows, on, mid.st, errs, cnt, acc);
+        Op::template eval_codes<G>(on, c1, c2, mid.st, errs, keep);
         mid.keep = 0;
 #pragma unroll
         for (int e = 0; e < kErr; ++e) mid.err[e] = 0;
 #pragma unroll
         for (int g = 0; g < G; ++g) {
-            mid.keep |= (cnt[g] != 0u ? 1u : 0u) << g;
+            mid.keep |= (keep[g] ? 1u : 0u) << g;
 #pragma unroll
             for (int e = 0; e < kErr; ++e) mid.err[e] |= ((errs[g] >> e) & 1u) << g;
         }
