@@ -167,17 +167,6 @@ __device__ __forceinline__ uint32_t dict_slot(uint64_t key) {
     return (x * 0x9E3779B1u) >> (32 - kDictBits);
 }
 
-template <class K>
-__device__ __forceinline__ K readlane_k(K v, uint32_t l) {
-    const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(static_cast<uint32_t>(v)), l));
-    if constexpr (sizeof(K) == 4) {
-        return lo;
-    } else {
-        const uint32_t hi = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v >> 32), l));
-        return (static_cast<uint64_t>(hi) << 32) | lo;
-    }
-}
-
 // A key with a first row into the HBM table.  Reads before the atomic: waves run roughly in row
 // order, so most find an earlier first row and make no atomic at all.
 __device__ __forceinline__ void grp_publish(const GrpTable &t, uint32_t *flags, uint32_t *list, uint64_t key,
@@ -310,9 +299,9 @@ __global__ __launch_bounds__(kBlock) void k_grp_first(GrpKey k, GrpTable t, uint
 // reads its key's home slot and first row and is done when the key is there with an earlier row; the
 // few others (new keys, keys past their home slot, rows of a key's first batch) probe and insert with
 // LDS atomics, every lane for itself; a key in several of a lane's rows once, which also spares columns in
-// key order an insert in HBM for every row once the set takes no more keys.  The set it replaced belonged to a wave, which listed its new
-// keys one after another: 35 keys in each of 8192 waves took longer than their rows.  12M binary keys,
-// 35 groups: 65 us before, 27 now (145 while the whole table was walked to publish it).
+// key order an insert in HBM for every row once the set takes no more keys.  The set it replaced belonged to
+// a wave, which listed its new keys one after another: 35 keys in each of 8192 waves took longer than their
+// rows.  12M binary keys, 35 groups: 65 us before, 31 now (145 while the whole table was walked to publish it).
 template <class T, bool BIN>
 __global__ __launch_bounds__(kBlock) void k_grp_first_set(GrpKey k, GrpTable t, uint32_t *flags, uint32_t *list,
                                                           uint64_t n, uint64_t per_block, uint32_t vec) {

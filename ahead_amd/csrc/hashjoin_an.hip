@@ -15,11 +15,11 @@
 //             first-row arrays.
 //  * checks : the build side's head/tail checks are an ordered two-stream pass on the row-tile
 //             engine (positions in build-scan order).
-//  * probe  : row-tile engine over the probe side: per row the head/tail checks, the key
-//             (decoded, guarded by `(larger_t)key <= max(build unencoded type)` and truncated to the
-//             build key width, :156-157 and :199-200 -- even for a corrupt probe key), and the
-//             matching rows' count; phase 2 writes the (probe payload, build payload) pairs of
-//             every probe row in probe order, build rows in insertion order.
+//  * probe  : per row the head/tail checks, the key (decoded, guarded by `(larger_t)key <= max(build
+//             unencoded type)` and truncated to the build key width, :156-157 and :199-200 -- even for a
+//             corrupt probe key) and the matching rows; (probe payload, build payload) pairs of every probe
+//             row in probe order, build rows in insertion order.  On the single-pass engine while every
+//             build key has one row (ProbeLeanOp, ProbeOneOp), else on the row-tile engine (ProbeOp).
 // Both hash sides (hash_side_t::right / ::left) and the re-encoding variants are supported.
 #include "htable.hpp"
 #include "stream.hpp"

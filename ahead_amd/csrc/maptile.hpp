@@ -30,16 +30,11 @@ constexpr int kMapG = 4;              // rows per lane per iteration (unless the
 struct MapArgs {
     uint64_t rows_per_wave;
     uint32_t waves;
-    uint32_t *wcnt;    // [NS][waves]: (unused), error streams
+    uint32_t *wcnt;    // [kErr][waves] errors per stream
     uint32_t *wpre;    // same shape: exclusive prefixes over the waves
     uint32_t *werows;  // [waves] rows with any error
     uint64_t *elist;   // [waves][kMapErrList] error bits << 32 | row
-    uint64_t *totals;  // [NS] per stream (k_map_scan)
-};
-
-template <class Op>
-struct MapTraits {
-    static constexpr int NS = 1 + Op::kErr;
+    uint64_t *totals;  // [1 + kErr] per error stream from 1 on (k_map_scan; [0], a main stream's, is not written)
 };
 
 __device__ __forceinline__ uint32_t map_below(uint64_t ballot) {
@@ -109,7 +104,7 @@ struct SharedWords<Op, true> {
 // Rows of one wave's range; lane l handles rows seg + g * 64 + l (one coalesced run per g).
 template <class Op>
 __global__ __launch_bounds__(kBlock) void k_map(Op op, MapArgs m) {
-    static_assert(!Op::kMulti && !Op::kMain, "the map engine takes operators without an ordered main output");
+    static_assert(!Op::kMulti && !Op::kMain && Op::kErr > 0, "the map engine takes operators whose ordered outputs are errors");
     constexpr int G = MapG<Op>::value;
     __shared__ unsigned long long s_acc[SharedWords<Op>::value];
     __shared__ uint64_t s_filt[FilterWords<Op>::value];
@@ -129,7 +124,7 @@ __global__ __launch_bounds__(kBlock) void k_map(Op op, MapArgs m) {
     const uint64_t begin = static_cast<uint64_t>(gw) * m.rows_per_wave;
     const uint64_t end = begin + m.rows_per_wave < op.n ? begin + m.rows_per_wave : op.n;
     uint32_t err_rows = 0;  // wave-uniform
-    uint32_t ecnt[Op::kErr > 0 ? Op::kErr : 1] = {};
+    uint32_t ecnt[Op::kErr] = {};
     uint64_t acc = 0;
     for (uint64_t seg = begin; seg < end; seg += 64u * G) {
         uint64_t rows[G];
@@ -173,14 +168,13 @@ __global__ __launch_bounds__(kBlock) void k_map(Op op, MapArgs m) {
         if (lane == 0) op.tile_done(gw, t);
     }
     if (lane == 0) {
-        m.wcnt[gw] = 0u;
 #pragma unroll
-        for (int e = 0; e < Op::kErr; ++e) m.wcnt[static_cast<size_t>(1 + e) * m.waves + gw] = ecnt[e];
+        for (int e = 0; e < Op::kErr; ++e) m.wcnt[static_cast<size_t>(e) * m.waves + gw] = ecnt[e];
         m.werows[gw] = err_rows;
     }
 }
 
-// One workgroup of 1024 threads per count stream: exclusive prefixes over the
+// One workgroup of 1024 threads per error stream: exclusive prefixes over the
 // waves and the stream total.
 template <class Op>
 __global__ __launch_bounds__(1024) void k_map_scan(Op op, MapArgs m) {
@@ -218,7 +212,7 @@ __global__ __launch_bounds__(1024) void k_map_scan(Op op, MapArgs m) {
         }
         carry += tot;
     }
-    if (threadIdx.x == 0) m.totals[s] = carry;
+    if (threadIdx.x == 0) m.totals[1 + s] = carry;
 }
 
 // Error positions.
@@ -236,10 +230,10 @@ __global__ __launch_bounds__(kBlock) void k_map_fix(Op op, MapArgs m) {
 
     // error positions
     const uint32_t nrows = m.werows[gw];
-    if (nrows != 0u && Op::kErr > 0) {
-        uint64_t idx[Op::kErr > 0 ? Op::kErr : 1];
+    if (nrows != 0u) {
+        uint64_t idx[Op::kErr];
 #pragma unroll
-        for (int e = 0; e < Op::kErr; ++e) idx[e] = m.wpre[static_cast<size_t>(1 + e) * m.waves + gw];
+        for (int e = 0; e < Op::kErr; ++e) idx[e] = m.wpre[static_cast<size_t>(e) * m.waves + gw];
         const bool listed = nrows <= kMapErrList;
         const uint64_t span = listed ? nrows : end - begin;
         for (uint64_t j0 = 0; j0 < span; j0 += 64u) {
@@ -297,7 +291,7 @@ uint32_t map_grid(uint64_t n) {
 template <class Op>
 size_t map_scratch_bytes(uint64_t n) {
     using namespace ahead_dev;
-    constexpr int NS = MapTraits<Op>::NS;
+    constexpr int NS = Op::kErr;
     const size_t waves = static_cast<size_t>(map_grid<Op>(n)) * kWaves;
     return 2 * align_up(NS * waves * 4, 256) + align_up(waves * 4, 256) + align_up(waves * kMapErrList * 8, 256) + 256;
 }
@@ -324,7 +318,7 @@ uint32_t map_parts(uint64_t n) {
 template <class Op>
 int launch_map(const Op &op, ahead_hip_ws *ws, size_t offset, hipStream_t s) {
     using namespace ahead_dev;
-    constexpr int NS = MapTraits<Op>::NS;
+    constexpr int NS = Op::kErr;
     const uint32_t grid = map_grid<Op>(op.n);
     const uint32_t waves = grid * kWaves;
     const size_t o_cnt = offset, o_pre = o_cnt + align_up(static_cast<size_t>(NS) * waves * 4, 256),
@@ -344,7 +338,7 @@ int launch_map(const Op &op, ahead_hip_ws *ws, size_t offset, hipStream_t s) {
     m.werows = reinterpret_cast<uint32_t *>(ws_region(ws, o_erows));
     m.elist = reinterpret_cast<uint64_t *>(ws_region(ws, o_elist));
     m.totals = reinterpret_cast<uint64_t *>(ws_region(ws, o_totals));
-    static_assert(8 * NS <= 256, "totals fit their block");
+    static_assert(8 * (1 + NS) <= 256, "totals fit their block");
     hipLaunchKernelGGL(k_map<Op>, dim3(grid), dim3(kBlock), 0, s, op, m);
     hipLaunchKernelGGL(k_map_scan<Op>, dim3(NS), dim3(1024), 0, s, op, m);
     hipLaunchKernelGGL(k_map_fix<Op>, dim3(grid), dim3(kBlock), 0, s, op, m);

@@ -904,12 +904,6 @@ __device__ __forceinline__ uint64_t mi_rows_end(uint64_t begin, uint64_t per, ui
     return begin + per < n ? begin + per : n;
 }
 
-// Lanes below the calling one whose ballot bit is set.
-__device__ __forceinline__ uint32_t mi_below(uint64_t ballot) {
-    return __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(ballot >> 32),
-                                     __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(ballot), 0u));
-}
-
 // Codes of N rows of a column of K codes, loaded as K (widened where they are used, so a load's
 // wait sits at its first use).  Rows that are not ok read row 0.
 template <typename K, int N>

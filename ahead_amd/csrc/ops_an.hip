@@ -1,6 +1,7 @@
-// ops_an.hip -- per-operator gfx950 kernels on the row-tile engine (rowtile.hpp):
+// ops_an.hip -- per-operator gfx950 kernels.  On the single-pass engine (stream.hpp):
 //   fetchjoinAN                 (lib/column_operators/AN/matchjoinAN.tcc:312-353)
 //   matchjoinAN, positional     (matchjoinAN.tcc:240-301)
+// and on the map engine (maptile.hpp):
 //   aggregate_sum_groupedAN     (aggregateAN.tcc:41-119)
 //   aggregate_mul_sumAN         (aggregateAN_scalar.tcc:58-131)
 //   arithmeticAN                (arithmeticAN_scalar.tcc:60-112)
@@ -14,8 +15,6 @@ using namespace ahead_dev;
 
 namespace {
 
-constexpr int kG = 8;  // row groups of 256 per tile (2048 rows)
-
 // ---------------------------------------------------------------------------------------------------
 // fetchjoinAN on the single-pass engine.  The gathers bound it: a random 2-byte gather costs a 128-byte
 // line between L1 and L2, so 60M of them take 270 us where the rest of the operator takes 100.  A column
@@ -23,8 +22,9 @@ constexpr int kG = 8;  // row groups of 256 per tile (2048 rows)
 //   kRaw     its codes, when they fit;
 //   kPacked  its decoded values less the smallest, in the fewest bits that hold them, several to a word;
 //            the all-ones field sends the row to the column (corrupt codes; the largest value, where the
-//            bits leave no other field), whose code is checked; the other rows' values are valid.  Rows past the words' capacity read the column too, so a column
-//            of 200,000 8-bit values serves three quarters of its rows from LDS.
+//            bits leave no other field), whose code is checked; the other rows' values are valid.  Rows past
+//            the words' capacity read the column too, so a column of 200,000 8-bit values serves three
+//            quarters of its rows from LDS.
 // 60M OIDs into 2-byte columns, the lookups alone with the streaming around them: 40,000 rows 220 us from
 // L2, 104 from LDS; 200,000 rows 264 and 150; without any lookup 97.  The whole operator into 200,000 8-bit
 // values: 408 us before (gathers 340, moving the entries behind a dropped row 67), 205 now.
@@ -337,11 +337,14 @@ int launch_fetch(const ahead_col *oids, const ahead_col *col, int reenc, uint64_
     op.e2 = static_cast<uint64_t *>(err2.data);
     op.e2_cap = err2.data ? err2.cap : 0;
     op.d_counts = d_counts;
-    // A workgroup fills its table from L2 at about 100 KB per microsecond, the packed one after two small
-    // launches; a gather it saves is worth 3 ps over the whole card.  The codes of the column pay from 4
-    // OIDs a byte on, packed values from 16; packing serves columns up to 2 MB (below a quarter of the rows in
-    // LDS the kernel leaves it).  A corrupt value re-encodes differently from its decoded form, so the
-    // packed table needs A^-1 to be A's inverse.
+    // Every workgroup fills a table of its own, the packed one after two small launches, which the gathers it
+    // saves have to earn.  us a call, from the column / from the table.  Codes: 40 KB, 500,000 OIDs 11 / 11,
+    // 1M 16 / 14, 8M 45 / 31; 140 KB, 250,000 10 / 12, 500,000 11 / 13, 1M 17 / 16, 8M 57 / 33.  So they pay
+    // from about 4 OIDs a byte on.  Packed values: 200,000 8-bit ones (400 KB of codes) 4M 40 / 38, 8M
+    // 62 / 48, 60M 317 / 179; 60,000 16-bit ones (240 KB) 2M 26 / 28, 4M 40 / 35; 1M 8-bit ones 16M
+    // 105 / 112, 60M 335 / 339 (below a quarter of the rows in LDS the kernel leaves it).  So from 16 OIDs
+    // a byte on, and up to 2 MB.  A corrupt value re-encodes differently from its decoded form, so the packed
+    // table needs A^-1 to be A's inverse.
     const uint64_t bytes = col->n * sizeof(T);
     size_t lds = 0;
     if (col->n && bytes <= kFetchTableBytes && op.n / 4 >= bytes) {
@@ -952,12 +955,6 @@ DCol dcol(const ahead_col &c) {
     d.max_u = c.max_u & d.mask;
     d.seqbase = c.seqbase;
     return d;
-}
-
-uint32_t encoded_width(const ahead_col &c) {
-    if (c.encoded) return c.width;
-    const uint32_t w = c.data ? c.width : 4;
-    return w >= 4 ? 8 : 2 * w;
 }
 
 }  // namespace ahead_host

@@ -1,5 +1,7 @@
-// rowtile.hpp -- the generic tile engine of the per-operator kernels (fetch, positional match,
-// hash-join probe, group-id assignment, grouped sum, product sum, arithmetic).
+// rowtile.hpp -- the generic tile engine: ordered outputs of rows that may emit several entries (hash-join
+// probes of repeated keys, list offsets), of pairs checked together, and of few rows (build-side checks).
+// Operators whose rows emit at most one entry run on stream.hpp, those without an ordered main output on
+// maptile.hpp; both use this file's operator interface and columns.
 //
 // A tile is G groups of 256 consecutive rows; row = base + g*256 + threadIdx.x, so every global
 // load and store of a row group is one coalesced run.  Per row the operator's eval() returns the
@@ -230,8 +232,6 @@ struct DCol {
 namespace ahead_host {
 
 ahead_dev::DCol dcol(const ahead_col &c);
-// width of TypeMap<T>::v2_encoded_t::type_t for a column of the given kind
-uint32_t encoded_width(const ahead_col &c);
 
 // Launches one row-tile operator over n rows with `streams` look-back streams (1 + Op::kErr).
 // It uses no scratch region of the workspace: an operator's own regions stay intact.
