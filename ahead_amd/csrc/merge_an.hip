@@ -841,11 +841,12 @@ __global__ __launch_bounds__(kMmThreads) void k_mm_move(MergeArgs a) {
 
 
 // ---- the intersection path -------------------------------------------------------------------
-// When list 2 is strictly ascending in decoded value, list 1 ascending, and every code of h1, t1, h2
-// and t2 is valid, no check of the walk fails and each list-2 key is met by the first list-1 row that
-// holds it (a match advances both cursors; further rows of the key are skipped): the walk's output is
-// the sorted intersection, (h1[i], t2[j]) for every such i with t1[i] == h2[j] in ascending i, with
-// empty error vectors.  Such inputs take streaming passes instead of the sub-tile walk:
+// When list 2 is strictly ascending in decoded value, list 1 ascending, and every code of t1, h2 and
+// t2 is valid, each list-2 key is met by the first list-1 row that holds it (a match advances both
+// cursors; further rows of the key are skipped): the walk's output is the sorted intersection, (h1[i],
+// t2[j]) for every such i with t1[i] == h2[j] in ascending i.  Of the checks only those of h1 can
+// fail: e1 holds the corrupt heads of the rows the walk skips while list 2 lasts, that is, of those
+// without a partner whose key is below list 2's last; e2 to e4 are empty.  Such inputs take streaming passes instead of the sub-tile walk:
 //  k_mi_clear  list 2's first and last keys give the key range [lo2, hi2] (the path applies when
 //              it spans at most kMiBitsPerRow bits per list-2 row), whose bitmap words it clears;
 //  k_mi_build  a bitmap of list 2's keys over the range (bit k - lo2) and, when the pairs' tails
@@ -862,7 +863,7 @@ constexpr int kMiG = 4;  // rows per lane per step
 
 struct MiArgs {
     uint32_t *ok;       // [0] nonzero while the path applies, [1] list 1 failed a check, [2] its keys need 64 bits
-    uint64_t *range;    // [0] lo2, [1] bitmap words in use
+    uint64_t *range;    // [0] lo2, [1] bitmap words in use, [2] hi2
     uint64_t *bits;     // [words_cap]
     uint32_t *first;    // [words_cap] list-2 row of the first key in each word that holds one
     uint64_t words_cap;
@@ -876,11 +877,11 @@ struct MiArgs {
 // thread 0 publishes it), and the bitmap words in use cleared.
 __global__ __launch_bounds__(kBlock) void k_mi_clear(MergeArgs a, MiArgs mi, uint32_t eligible) {
     uint32_t ok = eligible && a.n1 > 0 && a.n2 > 0 ? 1u : 0u;
-    uint64_t lo = 0, words = 0;
+    uint64_t lo = 0, hi = 0, words = 0;
     if (ok) {
         const uint64_t c0 = a.h2.raw(0), c1 = a.h2.raw(a.n2 - 1);
         lo = a.h2.dec_of(c0);
-        const uint64_t hi = a.h2.dec_of(c1);
+        hi = a.h2.dec_of(c1);
         if (a.h2.bad_of(c0) || a.h2.bad_of(c1) || hi < lo) {
             ok = 0;
         } else {
@@ -892,6 +893,7 @@ __global__ __launch_bounds__(kBlock) void k_mi_clear(MergeArgs a, MiArgs mi, uin
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         mi.range[0] = lo;
         mi.range[1] = words;
+        mi.range[2] = hi;
         mi.ok[0] = ok;
         mi.ok[1] = 0u;
         mi.ok[2] = ok && a.t1.dec_of(a.t1.raw(a.n1 - 1)) > 0xFFFFFFFFull ? 1u : 0u;
@@ -1126,9 +1128,12 @@ __device__ __forceinline__ V mi_last_lane(V x) {
 // W8: both outputs are 8 bytes wide; a run-time width makes eight stores of each row's two, so much code
 // that a small call waits for its instructions (one tile of 2,556 void rows: 21 us with 16 rows per lane, 9
 // with 8 and fixed widths).
-template <typename K, typename V, bool VOID1, bool GATHER, bool W8>
+// CHK: h1 may have codes of its own to check (chk_h1); its error rows are evaluated again, and with ten rows a
+// lane eight registers spill (the lists above in such a form 193 -> 199 us; 30M heads of their own 282, with
+// eight rows a lane and no spill 303).
+template <typename K, typename V, bool VOID1, bool GATHER, bool W8, bool CHK>
 struct IntersectOp {
-    static constexpr int kErr = 1;  // rows that fail a check: the path does not apply (failed)
+    static constexpr int kErr = 1;  // e1, and the rows that fail a check: the path does not apply (failed)
     static constexpr int kG = !W8 || sizeof(V) == 8 || VOID1 || GATHER ? 8 : 10;
     static constexpr uint32_t kPack = 64u * kG;  // (8.2M of 30M rows kept: 151 -> 129 us)
     struct RawK {
@@ -1160,9 +1165,17 @@ struct IntersectOp {
         bool any;      // keys of type V reach the bitmap
     };
     __device__ bool skip() const { return mi.ok[0] == 0u || (choose && (mi.ok[2] != 0u) != (sizeof(V) == 8)); }
-    // (a flag of its own: every workgroup of this launch decides to run by ok[0])
-    __device__ void failed() const { mi.ok[1] = 1u; }
-    __device__ void init(char *) const {}
+    // A row that fails a check says so in LDS; the tile reports it.  (A flag of its own in HBM: every workgroup of
+    // this launch decides to run by ok[0].)
+    static constexpr size_t kLds = 16;
+    __device__ void init(char *lds) const {
+        if (threadIdx.x == 0) *reinterpret_cast<uint32_t *>(lds) = 0u;
+    }
+    __device__ bool failed(const char *lds) const {
+        if (*reinterpret_cast<const uint32_t *>(lds) == 0u) return false;
+        mi.ok[1] = 1u;
+        return true;
+    }
     __device__ Uniform begin(const char *) const {
         const uint64_t lo = mi.range[0];
         return Uniform{lo, static_cast<V>(lo), static_cast<uint32_t>(mi.range[1] * 64ull - 1ull), lo <= static_cast<V>(~static_cast<V>(0))};
@@ -1174,13 +1187,13 @@ struct IntersectOp {
     struct Mid {
         V v[G];
         uint64_t word[G];
-        uint32_t in, bad;
+        uint32_t in, rep;
     };
     template <int G>
-    __device__ __forceinline__ void open_tile(const char *, const Uniform &u, uint64_t first, uint32_t lane, uint32_t live,
+    __device__ __forceinline__ void open_tile(char *lds, const Uniform &u, uint64_t first, uint32_t lane, uint32_t live,
                                               const Raw (&raw)[G], Mid<G> &mid) const {
         mid.in = 0;
-        mid.bad = 0;
+        uint32_t fails = 0;
 #pragma unroll
         for (int g = 0; g < G; ++g) {
             V v;
@@ -1196,7 +1209,7 @@ struct IntersectOp {
                     v = static_cast<V>(a.t1.dec_of(c));
                     bad = a.t1.bad_of(c);
                 }
-                mid.bad |= (bad ? 1u : 0u) << g;
+                fails |= (bad ? 1u : 0u) << g;
             }
             mid.v[g] = v;
             const V off = v - u.lo_v;
@@ -1226,15 +1239,29 @@ struct IntersectOp {
 #pragma unroll
             for (int g = 0; g < G; ++g) {
                 const V prev = mi_lane_below(mid.v[g], edge);
-                mid.bad |= ((low >> g) & 1u) != 0u && prev > mid.v[g] ? 1u << g : 0u;
+                fails |= ((low >> g) & 1u) != 0u && prev > mid.v[g] ? 1u << g : 0u;
                 edge = mi_last_lane(mid.v[g]);
             }
         }
-        if (chk_h1) {
+        fails &= live;
+        if (fails != 0u) *reinterpret_cast<uint32_t *>(lds) = 1u;
+        mid.rep = fails;
+        if (CHK && chk_h1) {
+            uint32_t e1 = 0;
 #pragma unroll
             for (int g = 0; g < G; ++g) {
-                if (((live >> g) & 1u) && a.h1.bad_of(a.h1.raw(first + static_cast<uint32_t>(g * 64) + lane)))
-                    mid.bad |= 1u << g;
+                if (((live >> g) & 1u) && a.h1.bad_of(a.h1.raw(first + static_cast<uint32_t>(g * 64) + lane))) e1 |= 1u << g;
+            }
+            // the walk checks the head of a row that it skips: one without a partner, below list 2's last key
+            if (__ballot(e1 != 0u) != 0ull) {
+                const uint64_t hi = mi.range[2];
+#pragma unroll
+                for (int g = 0; g < G; ++g) {
+                    const bool pairs = ((mid.in >> g) & 1u) != 0u &&
+                                       ((mid.word[g] >> (static_cast<uint32_t>(mid.v[g] - u.lo_v) & 63u)) & 1ull) != 0ull;
+                    if (pairs || static_cast<uint64_t>(mid.v[g]) >= hi) e1 &= ~(1u << g);
+                }
+                mid.rep |= e1;
             }
         }
     }
@@ -1250,9 +1277,16 @@ struct IntersectOp {
             if constexpr (GATHER) st[g].j = static_cast<uint32_t>(__popcll(mid.word[g] & ((1ull << b) - 1ull)));
         }
         keep &= live & mid.in;
-        err[0] = live & mid.bad;
+        err[0] = mid.rep;
     }
-    __device__ void report(uint64_t, State &, uint32_t &) const {}
+    __device__ void report(uint64_t row, State &, uint32_t &errs) const {
+        if (!CHK || !chk_h1 || !a.h1.bad_of(a.h1.raw(row))) return;
+        const uint64_t v = dec_at(a.t1, row), lo = mi.range[0];
+        if (v >= mi.range[2]) return;
+        const bool pairs = v >= lo && ((v - lo) >> 6) < mi.range[1] && ((mi.bits[(v - lo) >> 6] >> ((v - lo) & 63u)) & 1ull) != 0ull &&
+                           !(row > 0 && dec_at(a.t1, row - 1) == v);
+        errs = pairs ? 0u : 1u;
+    }
     __device__ __forceinline__ void emit(const Uniform &u, const State &st, uint64_t first, uint64_t pos, uint32_t row,
                                          uint32_t k) const {
         const uint64_t v = u.lo + st.off;
@@ -1269,16 +1303,21 @@ struct IntersectOp {
             store_w(a.out_t, pos + k, a.wout_t, ot);
         }
     }
-    __device__ void emit_err(int, uint64_t, const State &, uint64_t) const {}
+    __device__ void emit_err(int, uint64_t row, const State &, uint64_t pos) const {
+        if (CHK && pos < a.err_cap[0]) a.err[0][pos] = row * a.a_oid;
+    }
     __device__ void finish(const uint64_t *t) const {
         a.d_counts[0] = t[0];
+        a.d_counts[1] = t[1];
 #pragma unroll
-        for (int s = 1; s < kMmStreams; ++s) a.d_counts[s] = 0ull;
+        for (int s = 2; s < kMmStreams; ++s) a.d_counts[s] = 0ull;
     }
 };
 
 template <typename K, typename V, bool VOID1>
 int launch_intersect(const MergeArgs &a, const MiArgs &mi, uint32_t back, bool choose, ahead_hip_ws *ws, hipStream_t s) {
+    const bool chk_h1 = a.h1.encoded && (VOID1 || !(a.h1.data == a.t1.data && a.h1.width == a.t1.width && a.t1.encoded &&
+                                                    a.h1.a_inv == a.t1.a_inv && a.h1.max_u == a.t1.max_u));
     auto run = [&](auto op) {
         op.n = a.n1;
         op.a = a;
@@ -1287,14 +1326,16 @@ int launch_intersect(const MergeArgs &a, const MiArgs &mi, uint32_t back, bool c
         op.back = back;
         op.choose = choose ? 1u : 0u;
         op.same = a.h1_from_t1 && a.t1.encoded == a.h2.encoded && (!a.t1.encoded || (a.a_t1 == a.a_h2 && a.t1.mask == a.h2.mask));
-        op.chk_h1 = a.h1.encoded && (VOID1 || !(a.h1.data == a.t1.data && a.h1.width == a.t1.width && a.t1.encoded &&
-                                                a.h1.a_inv == a.t1.a_inv && a.h1.max_u == a.t1.max_u));
+        op.chk_h1 = chk_h1 ? 1u : 0u;
         op.out_cap = a.out_cap;
-        return ahead_host::launch_stream(op, ws, s);
+        return ahead_host::launch_stream(op, ws, s, op.kLds);
     };
-    if (a.wout_h == 8 && a.wout_t == 8)
-        return a.t2_from_h2 ? run(IntersectOp<K, V, VOID1, false, true>{}) : run(IntersectOp<K, V, VOID1, true, true>{});
-    return a.t2_from_h2 ? run(IntersectOp<K, V, VOID1, false, false>{}) : run(IntersectOp<K, V, VOID1, true, false>{});
+    auto shape = [&](auto w8, auto chk) {
+        constexpr bool W = decltype(w8)::value, C = decltype(chk)::value;
+        return a.t2_from_h2 ? run(IntersectOp<K, V, VOID1, false, W, C>{}) : run(IntersectOp<K, V, VOID1, true, W, C>{});
+    };
+    if (a.wout_h != 8 || a.wout_t != 8) return shape(std::false_type{}, std::true_type{});
+    return chk_h1 ? shape(std::true_type{}, std::true_type{}) : shape(std::true_type{}, std::false_type{});
 }
 
 }  // namespace

@@ -51,8 +51,8 @@
 //   void init(char *lds) const;         // all threads, before the first tile; a barrier follows
 //   bool skip() const;                  // the whole launch stands down (from device state that no
 //                                       // workgroup of this launch changes)
-//   void failed() const;                // (optional) one thread, for a tile that reports: nothing this launch writes
-//                                       // will be used, and the tiles still to come are counted as empty
+//   bool failed(const char *lds) const; // (optional) one thread, for a tile that reports: true if nothing that this
+//                                       // launch writes will be used; the tiles still to come are then counted as empty
 #pragma once
 
 #include "rowtile.hpp"
@@ -138,7 +138,7 @@ __device__ __forceinline__ void stream_load(const Op &op, uint64_t first, uint32
 template <class Op, class = void>
 struct can_fail : std::false_type {};
 template <class Op>
-struct can_fail<Op, std::void_t<decltype(std::declval<const Op &>().failed())>> : std::true_type {};
+struct can_fail<Op, std::void_t<decltype(std::declval<const Op &>().failed(nullptr))>> : std::true_type {};
 
 // The workgroup's tiles from `tile` on, published as empty, so that no other one waits for them (thread 0).
 template <int NS>
@@ -284,10 +284,8 @@ __global__ __launch_bounds__(kStreamThreads) void k_stream(Op op, StreamArgs m) 
         const uint32_t drawn = uniform(s_tile), next = can_fail<Op>::value ? drawn & ~kStreamFailed : drawn;
         if constexpr (can_fail<Op>::value) {
             // (before the workgroup's last ticket, and so before the next launch's first one)
-            if (rep != 0u && threadIdx.x == 0) {
-                op.failed();
-                if (next < m.tiles) atomicOr(m.te, static_cast<unsigned long long>(kStreamFailed));
-            }
+            if (rep != 0u && threadIdx.x == 0 && op.failed(s_op) && next < m.tiles)
+                atomicOr(m.te, static_cast<unsigned long long>(kStreamFailed));
         }
         if (next < m.tiles) {
             stream_load<Op, H>(op, first_of(next), lane, left_of(next), 0, raw0);

@@ -340,3 +340,31 @@ def test_merge_keys_past_32_bits(base, kind):
         c1 = codes(k1)
         c1[7000] ^= np.uint64(1 << 50)
         run_both(h1, c1, codes(k2), t2, RESOID, meta, meta, RESOID)
+
+
+@pytest.mark.parametrize("n1,n2,hi2,rate", [(1, 1, 5, 1.0), (70, 40, 60, 0.3), (5000, 3000, 5200, 0.02), (9001, 4000, 4000, 0.5),
+                                            (300_001, 100_000, 400_000, 1e-3), (300_001, 100_000, 150_000, 0.05),
+                                            (1_000_003, 700_000, 1_100_000, 1e-5)])
+@pytest.mark.parametrize("void1", [False, True])
+def test_merge_corrupt_heads_of_list1(n1, n2, hi2, rate, void1):
+    """Heads of list 1 in a column of their own, some corrupt: reported where the walk skips the row (no partner, a
+    repeated key among them, while list 2 lasts), joined unseen where it pairs."""
+    rng = np.random.default_rng(n1 + n2 + void1)
+    k1 = (np.arange(n1, dtype=np.uint64) + np.uint64(2) if void1 else
+          np.sort(rng.integers(0, max(2, int(1.2 * n1)), n1)).astype(np.uint64))
+    k2 = np.unique(rng.integers(0, hi2, n2)).astype(np.uint64)
+    h1 = oid_list(np.arange(n1, dtype=np.uint64), 7, 1)
+    bad = rng.random(n1) < rate
+    bad[[0, n1 // 2, n1 - 1]] = True
+    h1[bad] ^= np.uint64(1) << rng.integers(0, 64, int(bad.sum())).astype(np.uint64)
+    t1, h2, t2 = oid_list(k1, 7, 2), oid_list(k2, 7, 3), oid_list(np.arange(k2.size, dtype=np.uint64), 7, 4)
+    pairs = _pairs_of_repeats(k1, k2)
+    want = np.nonzero(bad & ~pairs & (k1 < k2[-1]))[0].astype(np.uint64) * np.uint64(an.A_OID_ERR)
+    for right in (h2, t2):
+        if void1:
+            ref = O.matchjoin_merge_an(O.Col(h1, RESOID), O.void(n1, 2), O.Col(h2, RESOID), O.Col(right, RESOID))
+            same(capi.matchjoin_merge_an(capi.Column.from_numpy(h1, RESOID), capi.Column.void(n1, 2),
+                                         *[capi.Column.from_numpy(x, RESOID) for x in (h2, right)], err_cap=2), ref)
+        else:
+            ref = run_both(h1, t1, h2, right, RESOID, RESOID, RESOID, RESOID)
+        assert ref[0].size == pairs.sum() and np.array_equal(ref[2], want) and all(x.size == 0 for x in ref[3:])
