@@ -1,7 +1,6 @@
-"""The streaming engine (maptile.hpp) on fetchjoinAN, where a corrupt fetched code or an OID past
-the column drops the row: no drops, few drops (entries moved into place), many drops (every wave
-writes again), an output smaller than the input (the tile engine runs instead), all bit-exact
-against the oracle, error positions included."""
+"""fetchjoinAN where a corrupt fetched code or an OID past the column drops the row: no drops, few and many
+drops, and an output smaller than the input, all on the single-pass engine (stream.hpp) and bit-exact against
+the oracle, error positions included."""
 import ctypes
 
 import numpy as np

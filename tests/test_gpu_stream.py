@@ -1,5 +1,5 @@
-"""The single-pass engine (stream.hpp) at the edges of its tiles (1024 threads x 16 rows; 32 for 2-byte
-codes) and of its 512-tile window, against the oracle: outputs, counts and error positions."""
+"""The single-pass engine (stream.hpp) at the edges of its tiles (1024 threads x 4, 8, 16 or 32 rows, by the size
+of the call) and of its 512-tile window, against the oracle: outputs, counts and error positions."""
 import ctypes
 
 import numpy as np
